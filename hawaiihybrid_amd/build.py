@@ -91,7 +91,7 @@ def build_oracle(verbose=True):
     r = subprocess.run(["make", "-C", os.path.join(REPO, "oracle"), "-s"], capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("oracle build failed:\n" + r.stdout + r.stderr)
-    if os.path.isdir("/root/reference"):
+    if os.path.exists("/root/reference/thirdparty/mtwist.c"):   # the checkers' sources
         r = subprocess.run(["make", "-C", os.path.join(REPO, "oracle"), "-s", "ref"], capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError("reference checker build failed:\n" + r.stdout + r.stderr)
