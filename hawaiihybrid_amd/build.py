@@ -28,6 +28,8 @@ SOURCES = [
     # becomes one FMA, nothing across statements), so kernels of different shape (one item per
     # thread, the lane pool, stage vectors in LDS or in the buffer arena) compute the same bits
     ("hh_kernels.hip", DEVICE + ["-ffp-contract=on"]),
+    # constants hoisted out of the row kernel's loops would take all its registers
+    ("hh_rows.hip", DEVICE + ["-ffp-contract=on", "-mllvm", "-disable-machine-licm"]),
     ("hh_aux.hip", DEVICE),
     ("hh_pipnn.hip", DEVICE),
     ("hh_zimm.hip", DEVICE),

@@ -58,6 +58,7 @@ struct JobDesc {
     long long item_begin;    // first global item index of this job
     long long n_items;       // ntraj * halves
     int* done;               // finished-item counter of the job (nullptr: not counted)
+    unsigned long long* pool_done;   // finished-item counter of the job's pool (nullptr: not counted)
     const int* order;        // admission group's order: the item run at queue position g is
     long long order_base;    //   order_base + order[g - order_base] (nullptr: the item g itself)
     int halves;              // 1: forward only, 2: forward + momentum-inverted backward
@@ -110,6 +111,10 @@ struct PoolCtl {
     long long ticks;
     int ring;
     int pad;
+    // The lane kernel ends its slice early once *finished (the pool's finished items) has reached
+    // finish_target: what is left is few enough for the row kernel.
+    const unsigned long long* finished;
+    unsigned long long finish_target;
 };
 
 // Rejection-sampler M0 (calculate_M0, src/hawaii.c:1423-1491)

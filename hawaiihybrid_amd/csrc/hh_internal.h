@@ -24,6 +24,10 @@ hipError_t run_plain(int sys, const SysConst& sc, const JobDesc* jobs_dev, int n
                      hipStream_t st);
 hipError_t run_pool(int sys, bool mixed, int block, int waves, const SysConst& sc, const JobDesc* ring,
                     const PoolCtl& ctl, const LaneSlots& sl, double* ws, hipStream_t st);
+// one slice of a pool with one trajectory per 16-lane row (hh_rows.hip): wgs workgroups of 16 rows,
+// rows_used rows of each wavefront refill from the queue; the live slots are ranks below 16 wgs
+hipError_t run_rows(int sys, bool mixed, const SysConst& sc, const JobDesc* ring, const PoolCtl& ctl, const LaneSlots& sl,
+                    int wgs, int rows_used, hipStream_t st);
 hipError_t run_slots_clear(const LaneSlots& sl, hipStream_t st);
 hipError_t run_clamp_next(unsigned long long* next, unsigned long long total, hipStream_t st);
 // right-hand sides spent on the job in ring slot `ring_slot` (added to *out)
@@ -124,6 +128,7 @@ struct PoolJob {
     size_t bytes = 0;           // device bytes held by `buf`
     std::shared_ptr<DevBuf> group_order;   // order of the admission group this job belongs to
     bool items_done = false;    // every item of the job has finished (seen after a slice)
+    long long items_finished = 0;   // items finished (seen after a slice)
     // mixed precision: items handed over to FP64 (jd.orbit_items / jd.orbit_count) run as orbit
     // jobs in the FP64 pool `orbit_pool` at rtol = atol = orbit_rtol; the job is reduced once its
     // own items and all its orbit jobs have finished
@@ -149,6 +154,7 @@ struct LanePool {
     int ring_cap = 8192;
     DevBuf slots[2];            // double-buffered for repacking
     int cur = 0;
+    // next: the queue head, then the number of items finished since the pool exists
     DevBuf arena, ring, ring_done, ring_orbit, ring_orbit_nrhs, next, scratch, sort_tmp;
     // every pool's slices run on its own stream (default priority), so the slices of different
     // pools (an FP64 orbit pool beside its mixed pool, classes of a serving mix) overlap
@@ -160,6 +166,7 @@ struct LanePool {
     long long next_seq = 0;
     unsigned long long total = 0;   // items admitted
     bool drained_repacked = false;
+    bool live_slots = false;        // a slice has left items in the lane slots
     long long unordered_seq = 0;    // first job not yet ordered (pool_order_group)
     LaneSlots view(int which) const { return slots_view(sys, slots[which].p, S); }
     // one slice as a captured graph: [repack (when the queue has drained), clamp of the queue

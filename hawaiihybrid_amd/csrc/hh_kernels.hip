@@ -23,14 +23,10 @@
 // vectors in registers needs ~440 registers per lane for CO2-Ar (one wave per SIMD).
 #include <hip/hip_runtime.h>
 
-#include "dop853_coeffs.h"
-#include "hh_engine.h"
-#include "hh_systems.h"
+#include "hh_integrate.h"
 
 namespace hh {
 
-constexpr double kEPS = 2.220446049250313e-16;
-constexpr int kMaxTotalSteps = 400000;   // attempts per item; the longest CO2-Ar items take ~6e3
 constexpr int kSlots = 16;               // K0..K15
 #ifndef HH_MIN_WAVES
 #define HH_MIN_WAVES 2   // occupancy target (waves per SIMD) of the trajectory kernels
@@ -160,6 +156,7 @@ __device__ __forceinline__ void finish_item(const JobDesc& jb, Lane<N>& ln, int 
         jb.nrhs[ln.local] = ln.nrhs;
     jb.e_drift[ln.local] = drift;
     if (jb.done) atomicAdd(jb.done, 1);
+    if (jb.pool_done) atomicAdd(jb.pool_done, 1ull);
     ln.active = 0;
 }
 
@@ -334,65 +331,12 @@ __device__ __forceinline__ void stages(const SysConst& sc, const Arena<N>& ar, c
     }
 }
 
-// Dense output of coordinate c (state index 2c) at x = (t_k - t) / h of an accepted step:
-// DOP853's 7th-order continuous extension (Hairer's contd8) in Horner form.
-__device__ __forceinline__ double dense_value(const double (&F)[7], double y0, double x)
-{
-    const double omx = 1.0 - x;
-    double v = F[5] + x * F[6];
-    v = F[4] + omx * v;
-    v = F[3] + x * v;
-    v = F[2] + omx * v;
-    v = F[1] + x * v;
-    v = F[0] + omx * v;
-    return y0 + x * v;
-}
-
 template <int NQ>
 __device__ __forceinline__ double dense_coord(const double (&Fc)[7][NQ], int c, double y0, double x)
 {
     const double F[7] = {Fc[0][c], Fc[1][c], Fc[2][c], Fc[3][c], Fc[4][c], Fc[5][c], Fc[6][c]};
     return dense_value(F, y0, x);
 }
-
-// CF value mu(0) . mu(t_k) of a sample
-template <typename P>
-__device__ __forceinline__ double cf_value(const double* mu0, const P (&m)[3])
-{
-    return mu0[0] * (double)m[0] + mu0[1] * (double)m[1] + mu0[2] * (double)m[2];
-}
-
-// Checks of one sample in the reference's order (src/hawaii.c:2181-2236): a NaN dipole, a
-// huge CF value, a jump by more than 1e10 from the previous sample (from sample 2 on).  A
-// PR/mu series (record 2) has no check that ends it: the reference skips a sample whose dipole
-// is NaN and integrates on (src/hawaii.c:3664-3677), leaving that sample of its zeroed series at
-// 0 (store_sample).
-template <typename P>
-__device__ __forceinline__ int sample_status(const P (&m)[3], double curr, double prev, int k, int record)
-{
-    if (record == 2) return ITEM_OK;
-    if (isnan((double)m[0]) || isnan((double)m[1]) || isnan((double)m[2])) return ITEM_FAIL_DIPOLE_NAN;
-    if (fabs(curr) > 1e100) return ITEM_FAIL_CF_HUGE;
-    if (k > 1 && fabs(curr / prev) > 1e10) return ITEM_FAIL_CF_JUMP;
-    return ITEM_OK;
-}
-
-// sample k of an item whose row starts at `row`: mu(0) . mu(t_k), or the three dipole
-// components (rows [3][L]) when the job records the series
-template <typename P>
-__device__ __forceinline__ void store_sample(double* row, int L, int record, int k, const P (&m)[3], double curr)
-{
-    if (record) {
-        const bool skip = record == 2 && (isnan((double)m[0]) || isnan((double)m[1]) || isnan((double)m[2]));
-        row[k] = skip ? 0.0 : (double)m[0];
-        row[L + k] = skip ? 0.0 : (double)m[1];
-        row[2 * (long long)L + k] = skip ? 0.0 : (double)m[2];
-    } else {
-        row[k] = curr;
-    }
-}
-
-enum StepOutcome : int { STEP_ENDED = 0, STEP_REJECTED = 1, STEP_ACCEPTED = 2 };
 
 // One attempted DOP853 step [t, t + h] of a lane: stages, error estimate, step-size control.
 // STEP_ACCEPTED: yn holds the new state, h the step taken and fac11 the error factor; when a
@@ -603,33 +547,12 @@ struct WaveShare {
     double last[64];  // CF value of the lane's last sample
 };
 
-// Fields of a lane's step record (field f at arena slot 1 + f / N, component f % N), in pairs
-// that one 16-byte access moves: the sample-time scalars [0, CF0), the CF scalars [CF0, YN),
-// the coordinates at the step's end (used only for a sample at exactly t + h), then per
-// coordinate c its value at the step's start followed by its seven dense-output coefficients
-// (Y + 8c .. Y + 8c + 7).
-template <int NQ>
-struct StepRecord {
-    static constexpr int T = 0, H = 1, TNEW = 2, DT = 3, K0 = 4, CF0 = 6, MU0 = 6, CURR = 9, ROW = 10, L = 11,
-                         RECORD = 12, YN = 14, Y = YN + (NQ + 1) / 2 * 2, SIZE = Y + 8 * NQ;
-};
-
 // fields [f0, f0 + n) of the record of lane `owner` (f0 and n even)
 template <int N, int NREC>
 __device__ __forceinline__ void rec_load_block(const Arena<N>& ar, int owner, int f0, int n, double (&r)[NREC])
 {
 #pragma unroll
     for (int f = f0; f < f0 + n; f += 2) ar.ld2_lane(owner, 1 + f / N, f % N, r[f], r[f + 1]);
-}
-
-// Memory written by one lane (LDS, the wavefront's arena block) is visible to the others
-// after this; every lane of the wavefront executes it.  A wavefront's own memory operations
-// are performed in order and its lanes share one vector L1, so the wavefront-scope fence only
-// keeps the compiler from moving accesses across it (it emits no wait).
-__device__ __forceinline__ void wave_share_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 
 // Evaluate, check and store the n pending samples of every lane (n = 0: none).  Called by all
@@ -837,22 +760,6 @@ __device__ __forceinline__ void dop853_step_shared(const SysConst& sc, const Job
 }
 
 // ------------------------------------------------------------------ kernels
-// CO2-Ar surface tables are staged into LDS once per workgroup: every right-hand side reads
-// 6 Legendre slots x 8 coefficients at a lane-dependent radial branch.
-template <int SYS, typename P>
-__device__ __forceinline__ SysConst stage_tables(const SysConst& sc, Co2ArTables<P>* s_tab)
-{
-    SysConst out = sc;
-    if constexpr (SYS == SYS_CO2AR) {
-        const double* src = (const double*)sc.tables;
-        double* dst = (double*)s_tab;
-        for (unsigned i = threadIdx.x; i < sizeof(Co2ArTables<P>) / sizeof(double); i += blockDim.x) dst[i] = src[i];
-        __syncthreads();
-        out.tables = s_tab;
-    }
-    return out;
-}
-
 // plain: lane g owns item g; ws holds one arena block per wavefront of the grid
 template <int SYS>
 __global__ void __launch_bounds__(256, HH_MIN_WAVES) plain_cf_kernel(SysConst sc, const JobDesc* __restrict__ jobs, int njobs,
@@ -932,21 +839,6 @@ __device__ __forceinline__ void save_lane(const LaneSlots& sl, long long s, cons
     sl.local[s] = ln.local;
 }
 
-// ring slot of the job holding global item g: jobs [first_seq, last_seq] are in flight, their
-// item ranges are consecutive and increasing with the sequence number
-__device__ __forceinline__ int ring_job(const JobDesc* __restrict__ ring, const PoolCtl& c, unsigned long long g)
-{
-    long long lo = c.first_seq, hi = c.last_seq;
-    while (lo < hi) {
-        const long long mid = (lo + hi + 1) >> 1;
-        if ((long long)g >= ring[mid % c.ring].item_begin)
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    return (int)(lo % c.ring);
-}
-
 // One slice of the batched engine.  Every lane slot restores its item (if any), integrates
 // and refills from the queue until the slice's time is up or no work is left, and saves its
 // state at a step boundary, so slices can be separated by admission of new jobs, reductions
@@ -969,8 +861,13 @@ __global__ void __launch_bounds__(BS, W) pool_cf_kernel(SysConst sc, const JobDe
     Lane<N> ln;
     restore_lane<N>(sl, slot, ar, ln);
     bool queue_open = true;   // the queue only grows between slices
-    for (;;) {
+    for (unsigned step = 0;; ++step) {
         if (wall_clock64() >= t_end) break;
+        // few enough items are left for the row kernel (looked at every eighth step: the load
+        // takes as long as a stage's)
+        if ((step & 7) == 7 &&
+            __hip_atomic_load(ctl.finished, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= ctl.finish_target)
+            break;
         if (!ln.active && queue_open) {
             bool got = false;
             while (!got) {

@@ -50,15 +50,15 @@ int pool_get(hh_engine* e, PoolSet& set, const hh_system& sys, bool mixed, LaneP
         pl->ring_done.ensure(pl->ring_cap * sizeof(int)) != hipSuccess ||
         pl->ring_orbit.ensure(pl->ring_cap * sizeof(int)) != hipSuccess ||
         pl->ring_orbit_nrhs.ensure(pl->ring_cap * sizeof(unsigned long long)) != hipSuccess ||
-        pl->next.ensure(sizeof(unsigned long long)) != hipSuccess ||
+        pl->next.ensure(2 * sizeof(unsigned long long)) != hipSuccess ||
         pl->scratch.ensure((size_t)(pl->S / 256 + 1) * sizeof(int)) != hipSuccess)
         return fail(HH_E_NOMEM, "cannot allocate a lane pool (%.1f MiB of slots and arena)",
                     (2.0 * sb + arena) / 1048576.0);
     HH_CHECK(hipStreamCreateWithFlags(&pl->stream, hipStreamNonBlocking));
     HH_CHECK(hipEventCreate(&pl->slice_end));
     HH_CHECK(run_slots_clear(pl->view(0), e->stream));
-    const unsigned long long z = 0;
-    HH_CHECK(hipMemcpyAsync(pl->next.p, &z, sizeof z, hipMemcpyHostToDevice, e->stream));
+    const unsigned long long z[2] = {0, 0};
+    HH_CHECK(hipMemcpyAsync(pl->next.p, z, sizeof z, hipMemcpyHostToDevice, e->stream));
     HH_CHECK(hipStreamSynchronize(e->stream));
     *out = pl.get();
     set.push_back(std::move(pl));
@@ -118,6 +118,7 @@ int pool_admit(hh_engine* e, LanePool& pl, const hh_cf_params& p, const double* 
     jd.item_begin = (long long)pl.total;
     jd.n_items = n_items;
     jd.done = pl.ring_done.as<int>() + slot;
+    jd.pool_done = pl.next.as<unsigned long long>() + 1;
     jd.halves = halves;
     jd.L = p.L;
     jd.max_steps = p.max_steps > 0 ? p.max_steps : 50000;
@@ -292,6 +293,30 @@ namespace {
 
 SysConst pool_sysconst(const hh_engine* e, const LanePool& pl) { return sysconst(e, pl.system, pl.mixed); }
 
+// Items left (in slots or queued) up to which a pool's slice runs on the row kernel.  Its rate grows
+// with the wavefronts in flight and levels off at two per SIMD (2048 wavefronts of four rows), where
+// the lane kernel still gains from every lane that is filled: measured on whole calls with limits of
+// 0, 1024, 2048, 4096 and 8192 items, 1153 CO2-Ar trajectories in FP64 take 45.3, 24.1, 23.3, 22.9 and
+// 21.7 ms, 65536 mixed ones (their tail) 282, 185, 182, 184 and 170 ms, 12289 CH4-CO2 ones 356, 266,
+// 238, 225 and 208 ms, 4096 He-Ar ones 7.7, 6.0, 5.5, 4.2 and 4.3 ms.
+constexpr long long kRowLimit = 8192;
+
+long long row_limit(const LanePool& pl) { return std::min(kRowLimit, pl.S / 8); }
+
+// The grid for `left` items: one row per wavefront while they fit one wavefront, then two, per SIMD (a
+// lone row has no neighbours to diverge from), then two wavefronts per SIMD of two to four rows.
+struct RowPlan {
+    int wgs, rows_used;
+};
+
+RowPlan row_plan(const hh_engine* e, long long left)
+{
+    const long long cus = e->prop.multiProcessorCount;   // a workgroup: one wavefront per SIMD
+    if (left <= 4 * cus) return {(int)cus, 1};
+    const long long waves = 8 * cus;
+    return {(int)(2 * cus), (int)std::min<long long>(4, (left + waves - 1) / waves)};
+}
+
 // The items that `parent` handed over since its last orbit job, [parent.orbit_admitted, count)
 // of its list, as one orbit job of the FP64 pool of the same class: the job shares the parent's
 // buffers and maps its item k to the parent's item orbit_items[orbit_admitted + k].
@@ -314,6 +339,7 @@ int admit_orbit_job(hh_engine* e, PoolSet& set, LanePool& parent_pool, PoolJob& 
     jd.item_begin = (long long)op->total;
     jd.n_items = n;
     jd.done = op->ring_done.as<int>() + slot;
+    jd.pool_done = op->next.as<unsigned long long>() + 1;
     jd.order = nullptr;
     jd.order_base = 0;
     jd.map = parent.jd.orbit_items + parent.orbit_admitted;
@@ -358,14 +384,30 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
             ctl.last_seq = pl->inflight.back()->seq;
             ctl.ticks = (long long)(slice_ms * e->wall_khz);
             ctl.ring = pl->ring_cap;
+            const long long limit = e->use_graphs ? 0 : row_limit(*pl);
+            ctl.finished = pl->next.as<unsigned long long>() + 1;
+            ctl.finish_target = limit > 0 && pl->total > (unsigned long long)limit ? pl->total - limit : ~0ull;
             HH_CHECK(hipStreamWaitEvent(pl->stream, e->ev[0], 0));
-            if (e->use_graphs) {
+            long long left = 0;
+            for (auto& j : pl->inflight)
+                if (j->state == 0 && !j->items_done) left += j->jd.n_items - j->items_finished;
+            if (left <= limit) {
+                if (pl->live_slots) {
+                    HH_CHECK(run_repack(pl->sys, pl->view(pl->cur), pl->view(1 - pl->cur), pl->scratch.as<int>(),
+                                        pl->stream));
+                    pl->cur = 1 - pl->cur;
+                }
+                const RowPlan rp = row_plan(e, left);
+                HH_CHECK(run_rows(pl->sys, pl->mixed, pool_sysconst(e, *pl), pl->ring.as<JobDesc>(), ctl,
+                                  pl->view(pl->cur), rp.wgs, rp.rows_used, pl->stream));
+            } else if (e->use_graphs) {
                 const int rc = launch_slice_graph(e, *pl, ctl, pool_sysconst(e, *pl));
                 if (rc != HH_OK) return rc;
             } else {
                 HH_CHECK(run_pool(pl->sys, pl->mixed, pl->block, pl->waves, pool_sysconst(e, *pl),
                                   pl->ring.as<JobDesc>(), ctl, pl->view(pl->cur), pl->arena.as<double>(), pl->stream));
             }
+            pl->live_slots = true;
             HH_CHECK(hipEventRecord(pl->slice_end, pl->stream));
             HH_CHECK(hipStreamWaitEvent(e->stream, pl->slice_end, 0));
             if (launches) ++*launches;
@@ -415,8 +457,12 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
                 const int rc = admit_orbit_job(e, set, *pl, j, orbit[slot]);
                 if (rc != HH_OK) return rc;
             }
+            j.items_finished = done[slot];
             if (done[slot] >= j.jd.n_items) j.items_done = true;
         }
+        bool integrating = false;
+        for (auto& j : pl->inflight) integrating |= j->state == 0 && !j->items_done;
+        pl->live_slots = integrating;
     }
     // a finished orbit job leaves its pool at once (its slot frees for the next hand-overs)
     for (auto& pp : set) {

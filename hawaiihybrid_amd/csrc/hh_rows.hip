@@ -1,0 +1,853 @@
+// Row kernel of the batched engine: one trajectory per DPP row (16 lanes) of a wavefront.
+//
+// The lane kernel (pool_cf_kernel, one trajectory per lane) needs 64 trajectories per wavefront
+// and thousands of wavefronts to pay for its stage arena: a stage reads its tableau row's columns
+// from memory, so one right-hand side takes 2.3 us however few lanes hold a trajectory.  Small
+// requests, and the last few thousand trajectories of large ones, are then a chain of memory round
+// trips.  Here lane i of a row holds component i of the state: the 16 stage vectors are 16
+// registers of every lane, a tableau row is one FMA per non-zero column for all components at
+// once, and the independent parts of a right-hand side run side by side in the row's lanes (the
+// angles' sines and cosines, the reciprocals, the radial slots of CO2-Ar, the site pairs of
+// CH4-CO2), exchanged with DPP row broadcasts.  What is serial (the Legendre recurrence, Hamilton's
+// equations, the sums in their order) runs in every lane of the row.
+//
+// Every expression is the lane kernel's, in its order, so a trajectory's row is the same bits
+// whichever kernel integrates it, and the two share the slot format: a slice of a pool can run on
+// either.  The rows of a grid hold the slots of ranks 0, 1, ... of a repacked pool.
+//
+// Bound: a lone wavefront's instruction issue (about 520 instructions per FP64 CO2-Ar right-hand
+// side).  One trajectory's right-hand side: 2.3 -> 1.0 us; 1153 CO2-Ar trajectories in FP64 (L = 1024)
+// 45.3 -> 21.7 ms, 4096 He-Ar ones (L = 2048) 7.7 -> 4.3 ms.
+#include <hip/hip_runtime.h>
+
+#include <utility>
+
+#include "hh_integrate.h"
+
+namespace hh {
+
+typedef unsigned int rw_v2u __attribute__((ext_vector_type(2)));
+
+constexpr int kRowBlock = 256;   // four wavefronts share the CO2-Ar tables in LDS
+
+// the value of lane L of the caller's row (row_newbcast); every lane of the row takes part
+template <int L>
+__device__ __forceinline__ int bcast(int v)
+{
+    return __builtin_amdgcn_mov_dpp(v, 0x150 + L, 0xf, 0xf, true);
+}
+template <int L>
+__device__ __forceinline__ float bcast(float v)
+{
+    return __builtin_bit_cast(float, bcast<L>(__builtin_bit_cast(int, v)));
+}
+template <int L>
+__device__ __forceinline__ double bcast(double v)
+{
+    const rw_v2u u = __builtin_bit_cast(rw_v2u, v);
+    return __builtin_bit_cast(double, rw_v2u{(unsigned)bcast<L>((int)u.x), (unsigned)bcast<L>((int)u.y)});
+}
+template <int L>
+__device__ __forceinline__ long long bcast(long long v)
+{
+    return __builtin_bit_cast(long long, bcast<L>(__builtin_bit_cast(double, v)));
+}
+
+// out[i] = lane i's value, i < N
+template <typename T, int N, int... I>
+__device__ __forceinline__ void gather_impl(T v, T (&out)[N], std::integer_sequence<int, I...>)
+{
+    ((out[I] = bcast<I>(v)), ...);
+}
+template <typename T, int N>
+__device__ __forceinline__ void gather(T v, T (&out)[N])
+{
+    gather_impl<T, N>(v, out, std::make_integer_sequence<int, N>{});
+}
+
+// v[comp] by selects; the empty asm keeps the values in registers (the compiler would turn the
+// selects into an indexed load of an array in scratch)
+template <int N>
+__device__ __forceinline__ double pick(const double (&v)[N], int comp)
+{
+    double r = v[0];
+#pragma unroll
+    for (int i = 1; i < N; ++i) {
+        double x = v[i];
+        __asm__("" : "+v"(x));
+        r = comp == i ? x : r;
+    }
+    return r;
+}
+
+// What a lane keeps for the whole kernel: its component and the reciprocals of the constants
+// (uniform), and for CH4-CO2 its site pair (lane l < 15: CO2 site l / 5, CH4 site l % 5).
+template <int SYS, typename P>
+struct RowCtx {
+    int lane, comp;      // lane of the row; component (the last one again past QP)
+    double imu, iI, i0, i1;
+    P sgn, s2, e4, h0, h1, h2;
+    P* scratch;          // CH4-CO2: the row's LDS scratch [5][16]
+};
+
+template <int SYS, typename P>
+__device__ __forceinline__ RowCtx<SYS, P> row_ctx(const SysConst& sc, P* scratch)
+{
+    RowCtx<SYS, P> cx{};
+    cx.lane = (int)(threadIdx.x & 15);
+    cx.comp = min(cx.lane, SysTraits<SYS>::QP - 1);
+    cx.imu = 1.0 / sc.mu;
+    cx.iI = SYS == SYS_HEAR ? 0.0 : 1.0 / sc.I;
+    cx.scratch = scratch;
+    if constexpr (SYS == SYS_CH4CO2) {
+        using namespace ch4co2;
+        cx.i0 = 1.0 / sc.IR[0];
+        cx.i1 = 1.0 / sc.IR[1];
+        const int l = min(cx.lane, 14), j = l / 5, i = l % 5;
+        const P hs = P(kRCH / 1.7320508075688772);
+#pragma unroll
+        for (int q = 0; q < 15; ++q) {
+            // the lane kernel's compile-time constants, picked by lane
+            const int jj = q / 5, ii = q % 5, tj = jj == 0 ? 2 : 3, ti = ii == 0 ? 0 : 1;
+            const double sig = 0.5 * (kSigma[ti] + kSigma[tj]) * kAng;
+            const P s2 = P(sig * sig);
+            const P e4 = P(4.0 * kWellScale * kKelvinHartree) * (P)__builtin_sqrt(kEpsilon[ti] * kEpsilon[tj]);
+            const P h0 = ii == 0 ? P(0) : hs * P(kH[ii == 0 ? 0 : ii - 1][0]);
+            const P h1 = ii == 0 ? P(0) : hs * P(kH[ii == 0 ? 0 : ii - 1][1]);
+            const P h2 = ii == 0 ? P(0) : hs * P(kH[ii == 0 ? 0 : ii - 1][2]);
+            if (q == 5 * j + i) {
+                cx.sgn = jj == 0 ? P(0) : (jj == 1 ? P(1) : P(-1));
+                cx.s2 = s2;
+                cx.e4 = e4;
+                cx.h0 = h0;
+                cx.h1 = h1;
+                cx.h2 = h2;
+            }
+        }
+    }
+    return cx;
+}
+
+// ------------------------------------------------------------------ right-hand sides
+// The component of Hamilton's equations of the calling lane; y: the lane's component of the
+// state.  noise as in rhs().  Each branch follows rhs<SYS, P> expression by expression.
+template <int SYS, typename P>
+__device__ __forceinline__ double row_rhs(const SysConst& sc, const RowCtx<SYS, P>& cx, double y, double& noise)
+{
+    constexpr int N = SysTraits<SYS>::QP;
+    noise = 0.0;
+    double yd[N];
+    double s, c;                      // every lane's own sine and cosine; the angles' lanes are read
+    sincos_p<double>(y, &s, &c);
+    P sP, cP;                         // and in the surfaces' precision
+    if constexpr (sizeof(P) == 8) {
+        sP = s;
+        cP = c;
+    } else {
+        sincos_p<P>(y, &sP, &cP);
+    }
+    const double R = bcast<4>(y);
+    if constexpr (SYS == SYS_HEAR) {
+        const double x = kHearB * R;
+        const double arg = cx.lane == 0 ? -x : -kHearA1 * R - kHearA2 * R * R;
+        const double ex = exp(arg);
+        double dV[3];
+        dV[0] = 0.0;
+        dV[1] = 0.0;
+        dV[2] = hear_dV_exps(R, bcast<0>(ex), bcast<1>(ex));
+        const double r = recip<P>(cx.lane == 4 ? y : s);
+        pair_eom(bcast<1>(y), bcast<3>(y), bcast<5>(y), bcast<2>(c), cx.imu, bcast<4>(r), bcast<2>(r), dV, yd);
+    } else if constexpr (SYS == SYS_CO2AR) {
+        const Co2ArTables<P>* tb = (const Co2ArTables<P>*)sc.tables;
+        // the lane's radial slot: value and derivative
+        const int b = co2ar_branch(R);
+        const int slot = min(cx.lane, 5);
+        const double rc = recip<P>(cx.lane == 4 ? y : s);
+        const double iR = bcast<4>(rc);
+        P v, dv;
+        if (b == 0) {
+            const P r = (P)R;
+            const P e = tb->pes_exp[slot][0] * exp(tb->pes_exp[slot][1] * r);
+            v = e;
+            dv = tb->pes_exp[slot][1] * e;
+        } else {
+            const P x = (P)(R - tb->center[b]);
+            const P sinv = (P)iR;
+            slot_eval<P>(tb->pes[b][slot], x, sinv, v, dv);
+        }
+        const double sT = bcast<2>(s), cT = bcast<2>(c), st = bcast<8>(s), ct = bcast<8>(c);
+        const Co2ArAngles<P> g = co2ar_angles<P>(bcast<0>(sP), bcast<0>(cP), (P)sT, (P)cT, bcast<6>(sP), bcast<6>(cP),
+                                                 (P)st, (P)ct);
+        P Pl[11], dPl[11];
+        legendre10<P>(g.c, Pl, dPl);
+        P vs[6], dvs[6];
+        gather<P, 6>(v, vs);
+        gather<P, 6>(dv, dvs);
+        P dVdR = P(0), dVdc = P(0), mag = P(0);
+#pragma unroll
+        for (int q = 0; q < 6; ++q) {
+            const P tR = dvs[q] * Pl[2 * q], tc = vs[q] * dPl[2 * q];
+            dVdR += tR;
+            dVdc += tc;
+            if constexpr (sizeof(P) == 4) mag += fabs(tR) + fabs(tc);
+        }
+        noise = sizeof(P) == 4 ? kF32NoiseUnits * (double)mag : 0.0;
+        double dV[5];
+        co2ar_gradient<P>(g, dVdR, dVdc, dV);
+        pair_eom(bcast<1>(y), bcast<3>(y), bcast<5>(y), cT, cx.imu, iR, bcast<2>(rc), dV, yd);
+        linear_rotor_eom(bcast<7>(y), bcast<9>(y), ct, cx.iI, bcast<8>(rc), dV[3], dV[4], yd + 6);
+    } else {
+        Ch4Co2Frame<P> f;
+        const double sT = bcast<2>(s), cT = bcast<2>(c), s1 = bcast<8>(s), c1 = bcast<8>(c);
+        const double sp = bcast<10>(s), cp = bcast<10>(c), s2 = bcast<14>(s), c2 = bcast<14>(c);
+        f.sP = bcast<0>(sP), f.cP = bcast<0>(cP), f.sf = bcast<6>(sP), f.cf = bcast<6>(cP);
+        f.sP2 = bcast<12>(sP), f.cP2 = bcast<12>(cP);
+        f.sT = (P)sT, f.cT = (P)cT, f.s1 = (P)s1, f.c1 = (P)c1, f.sp = (P)sp, f.cp = (P)cp, f.s2 = (P)s2, f.c2 = (P)c2;
+        ch4co2_axes<P>(f);
+        const P Rp = (P)R;
+        P gs[3], gd[3], mag = P(0);
+        {
+            // the lane's site pair
+            using namespace ch4co2;
+            const P sgn = cx.sgn;
+            const P X[3] = {Rp * f.a[0] + sgn * P(kRCO) * f.b[0], Rp * f.a[1] + sgn * P(kRCO) * f.b[1],
+                            Rp * f.a[2] + sgn * P(kRCO) * f.b[2]};
+            const P d0 = X[0] - cx.h0, d1 = X[1] - cx.h1, d2 = X[2] - cx.h2;
+            const P r2 = d0 * d0 + d1 * d1 + d2 * d2;
+            const P ir2 = P(1) / r2;
+            const P sr2 = cx.s2 * ir2, sr6 = sr2 * sr2 * sr2, sr12 = sr6 * sr6;
+            const P w = cx.e4 * (P(-12) * sr12 + P(6) * sr6) * ir2;   // (dV/dr) / r
+            P* sm = cx.scratch;
+            sm[cx.lane] = w;
+            sm[16 + cx.lane] = d0;
+            sm[32 + cx.lane] = d1;
+            sm[48 + cx.lane] = d2;
+            if constexpr (sizeof(P) == 4) sm[64 + cx.lane] = fabs(d0) + fabs(d1) + fabs(d2);
+            wave_share_sync();
+            // lane 3 j + k sums component k of CO2 site j over the five CH4 sites, in site order
+            const int jk = min(cx.lane, 8), j = jk / 3, k = jk - 3 * j;
+            P g = P(0);
+#pragma unroll
+            for (int i = 0; i < 5; ++i) g += sm[5 * j + i] * sm[16 + 16 * k + 5 * j + i];
+            if constexpr (sizeof(P) == 4) {
+#pragma unroll
+                for (int q = 0; q < 15; ++q) mag += fabs(sm[q]) * sm[64 + q];
+            }
+            wave_share_sync();
+            P gj[9];
+            gather<P, 9>(g, gj);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                gs[q] = P(0);
+                gd[q] = P(0);
+                gs[q] += gj[q];
+                gd[q] += P(0);
+                gs[q] += gj[3 + q];
+                gd[q] += gj[3 + q];
+                gs[q] += gj[6 + q];
+                gd[q] += -gj[6 + q];
+            }
+        }
+        double dV[8];
+        ch4co2_gradient<P>(f, Rp, gs, gd, dV);
+        noise = ch4co2_noise<P>(Rp, mag);
+        const double rc = recip<P>(cx.lane == 4 ? y : s);
+        // the rotor's 1/sin(theta1) is a division in both precisions
+        const double is1 = sizeof(P) == 8 ? bcast<8>(rc) : 1.0 / s1;
+        pair_eom(bcast<1>(y), bcast<3>(y), bcast<5>(y), cT, cx.imu, bcast<4>(rc), bcast<2>(rc), dV, yd);
+        const double m[6] = {0.0, bcast<7>(y), 0.0, bcast<9>(y), 0.0, bcast<11>(y)};
+        rotor_rhs(sc.IR, m, dV + 3, s1, c1, sp, cp, is1, cx.i0, cx.i1, yd + 6);
+        linear_rotor_eom(bcast<13>(y), bcast<15>(y), c2, cx.iI, bcast<14>(rc), dV[6], dV[7], yd + 12);
+    }
+    return pick<N>(yd, cx.comp);
+}
+
+// ------------------------------------------------------------------ a row's trajectory
+// y and K are the lane's component; everything else is the same in the 16 lanes of the row
+struct RowItem {
+    double y;
+    double t, h, E0;
+    double mx, my, mz;               // mu(0)
+    double prev, curr;
+    double dt, rtol, atol, Rcut;   // of the job, kept in registers
+    double* row;
+    long long local;
+    int L, max_steps, record;
+    int job, k, steps, total_steps, nrhs, reject, active;
+};
+
+__device__ __forceinline__ void row_job(const JobDesc& jb, RowItem& it)
+{
+    it.dt = jb.dt;
+    it.rtol = jb.rtol;
+    it.atol = jb.atol;
+    it.Rcut = jb.Rcut;
+    it.L = jb.L;
+    it.max_steps = jb.max_steps;
+    it.record = jb.record;
+    it.row = jb.rows + it.local * (long long)jb.L * row_width(jb.record);
+}
+
+// finish_item of the lane kernel, by the row's first lane
+__device__ __forceinline__ void row_finish(const JobDesc& jb, int lane, RowItem& it, int status, int last, float drift)
+{
+    if (lane == 0) {
+        jb.len[it.local] = last + 1;
+        jb.status[it.local] = status;
+        if (jb.map) {
+            jb.nrhs[it.local] += it.nrhs;
+            atomicAdd(jb.orbit_nrhs, (unsigned long long)it.nrhs);
+        } else
+            jb.nrhs[it.local] = it.nrhs;
+        jb.e_drift[it.local] = drift;
+        if (jb.done) atomicAdd(jb.done, 1);
+        if (jb.pool_done) atomicAdd(jb.pool_done, 1ull);
+    }
+    it.active = 0;
+}
+
+// sum over the components, in their order, of the squares of the lanes' values
+template <int N>
+__device__ __forceinline__ double sum_squares(double q)
+{
+    double v[N], acc = 0.0;
+    gather<double, N>(q, v);
+#pragma unroll
+    for (int i = 0; i < N; ++i) acc += v[i] * v[i];
+    return acc;
+}
+
+// The lane's stage values K0..K15, each a variable of its own: as an array they become one 32-register
+// vector, which this compiler (ROCm 7.2) updates wrongly across the divergent branches of a step.
+struct Stages {
+    double k0, k1, k2, k3, k4, k5, k6, k7, k8, k9, k10, k11, k12, k13, k14, k15;
+    template <int I>
+    __device__ __forceinline__ double& at()
+    {
+        if constexpr (I == 0) return k0;
+        else if constexpr (I == 1) return k1;
+        else if constexpr (I == 2) return k2;
+        else if constexpr (I == 3) return k3;
+        else if constexpr (I == 4) return k4;
+        else if constexpr (I == 5) return k5;
+        else if constexpr (I == 6) return k6;
+        else if constexpr (I == 7) return k7;
+        else if constexpr (I == 8) return k8;
+        else if constexpr (I == 9) return k9;
+        else if constexpr (I == 10) return k10;
+        else if constexpr (I == 11) return k11;
+        else if constexpr (I == 12) return k12;
+        else if constexpr (I == 13) return k13;
+        else if constexpr (I == 14) return k14;
+        else return k15;
+    }
+};
+
+// tableau row R (its columns those of row C) applied to the lane's stage values, from column q on
+template <int C, int R, int Q = 0>
+__device__ __forceinline__ double stage_sum(Stages& K, double acc = 0.0)
+{
+    if constexpr (Q == DOP853_SP_NNZ[C]) {
+        return acc;
+    } else {
+        acc += DOP853_SP_VAL[R][Q] * K.at<DOP853_SP_COL[C][Q]>();
+        return stage_sum<C, R, Q + 1>(K, acc);
+    }
+}
+
+__device__ __forceinline__ double stage_dot(Stages& K, int s)
+{
+    switch (s) {
+    case 1: return stage_sum<1, 1>(K);
+    case 2: return stage_sum<2, 2>(K);
+    case 3: return stage_sum<3, 3>(K);
+    case 4: return stage_sum<4, 4>(K);
+    case 5: return stage_sum<5, 5>(K);
+    case 6: return stage_sum<6, 6>(K);
+    case 7: return stage_sum<7, 7>(K);
+    case 8: return stage_sum<8, 8>(K);
+    case 9: return stage_sum<9, 9>(K);
+    case 10: return stage_sum<10, 10>(K);
+    case 11: return stage_sum<11, 11>(K);
+    case 12: return stage_sum<12, 12>(K);
+    case 13: return stage_sum<13, 13>(K);
+    case 14: return stage_sum<14, 14>(K);
+    default: return stage_sum<15, 15>(K);
+    }
+}
+
+template <int S0, int S1>
+__device__ __forceinline__ void stage_store(Stages& K, int s, double k)
+{
+    K.at<S0>() = s == S0 ? k : K.at<S0>();
+    if constexpr (S0 < S1) stage_store<S0 + 1, S1>(K, s, k);
+}
+
+template <int SYS, typename P, int S0, int S1>
+__device__ __forceinline__ void row_stages(const SysConst& sc, const RowCtx<SYS, P>& cx, double y, double h, Stages& K,
+                                           double& noise)
+{
+    noise = 0.0;
+#pragma unroll 1
+    for (int s = S0; s <= S1; ++s) {
+        double yt = stage_dot(K, s);
+        yt = y + h * yt;
+        double nz;
+        const double k = row_rhs<SYS, P>(sc, cx, yt, nz);
+        noise = fmax(noise, nz);
+        stage_store<S0, S1>(K, s, k);
+    }
+}
+
+// init_item of the lane kernel: the initial condition, mu(0), sample 0, H(0), f(y0), Hairer's HINIT
+template <int SYS, typename P>
+__device__ __forceinline__ bool row_init(const SysConst& sc, const RowCtx<SYS, P>& cx, const JobDesc& jb, int j,
+                                         long long local, RowItem& it, Stages& K)
+{
+    constexpr int N = SysTraits<SYS>::QP;
+    it.job = j;
+    it.local = jb.map ? (long long)jb.map[local] : local;
+    row_job(jb, it);
+    const long long traj = it.local / jb.halves;
+    const bool back = (it.local % jb.halves) == 1;
+    const double v = jb.ic[(long long)cx.comp * jb.ntraj + traj];
+    it.y = (back && (cx.comp & 1)) ? -v : v;
+    double yv[N];
+    gather<double, N>(it.y, yv);
+    if constexpr (SYS == SYS_CH4CO2) {
+        if (cx.lane < N && !(cx.lane & 1)) it.row[cx.lane >> 1] = it.y;
+        it.mx = it.my = it.mz = 0.0;
+    } else {
+        P m[3];
+        dipole<SYS, P>(sc, yv, m);
+        it.mx = m[0];
+        it.my = m[1];
+        it.mz = m[2];
+        if (cx.lane == 0) {
+            if (it.record) {
+                it.row[0] = it.mx;
+                it.row[it.L] = it.my;
+                it.row[2 * (long long)it.L] = it.mz;
+            } else {
+                it.row[0] = it.mx * it.mx + it.my * it.my + it.mz * it.mz;
+            }
+        }
+    }
+    it.E0 = hamiltonian<SYS, P>(sc, yv);
+    it.t = 0.0;
+    it.k = 1;
+    it.steps = 0;
+    it.total_steps = 0;
+    it.reject = 0;
+    it.nrhs = 0;
+    it.prev = 0.0;
+    it.curr = 0.0;
+    it.active = 1;
+    if (it.L <= 1) {
+        row_finish(jb, cx.lane, it, ITEM_OK, 0, 0.0f);
+        return false;
+    }
+    // Hairer's HINIT (initial_step)
+    const double hmax = (it.L - 1) * it.dt;
+    const double sk = it.atol + it.rtol * fabs(it.y);
+    double y1 = it.y, h = 0.0, dnf = 0.0, nz;
+#pragma unroll 1
+    for (int pass = 0; pass < 2; ++pass) {
+        const double f = row_rhs<SYS, P>(sc, cx, y1, nz);
+        if (pass == 0) {
+            K.k0 = f;
+            dnf = sum_squares<N>(f / sk);
+            const double dny = sum_squares<N>(it.y / sk);
+            h = (dnf <= 1e-10 || dny <= 1e-10) ? 1e-6 : sqrt(dny / dnf) * 0.01;
+            h = fmin(h, hmax);
+            y1 = it.y + h * f;
+        } else {
+            double der2 = sum_squares<N>((f - K.k0) / sk);
+            der2 = sqrt(der2) / h;
+            const double der12 = fmax(fabs(der2), sqrt(dnf));
+            const double h1 = (der12 <= 1e-15) ? fmax(1e-6, fabs(h) * 1e-3) : sqrt(sqrt(sqrt(0.01 / der12)));
+            h = fmin(fmin(100.0 * fabs(h), h1), hmax);
+        }
+    }
+    it.nrhs = 2;
+    it.h = h;
+    return true;
+}
+
+// ------------------------------------------------------------------ samples
+// The wavefront evaluates the pending samples of its four rows 64 at a time, as shared_samples of
+// the lane kernel; the rows' step records lie in LDS.
+template <int NQ>
+struct RowShare {
+    double rec[4][StepRecord<NQ>::SIZE];
+    double last[4];
+    int fail[4];
+};
+
+template <int SYS, typename P>
+__device__ __forceinline__ void row_samples(const SysConst& sc, RowShare<SysTraits<SYS>::QP / 2>& ws, int n)
+{
+    constexpr int N = SysTraits<SYS>::QP, NQ = N / 2;
+    using R = StepRecord<NQ>;
+    const int lane = (int)__lane_id();
+    const int n0 = __builtin_amdgcn_readlane(n, 0), n1 = __builtin_amdgcn_readlane(n, 16);
+    const int n2 = __builtin_amdgcn_readlane(n, 32), n3 = __builtin_amdgcn_readlane(n, 48);
+    const int p1 = n0, p2 = n0 + n1, p3 = p2 + n2, total = p3 + n3;
+    if (total == 0) return;
+    if (lane < 4) ws.fail[lane] = 0x7fffffff;
+    wave_share_sync();
+    double carry = 0.0;
+#pragma unroll 1
+    for (int base = 0; base < total; base += 64) {
+        const int g = base + lane;
+        const bool valid = g < total;
+        int owner = 0, q = 0, k = 0, cnt = 0, record = 0;
+        double curr = 0.0, prev_start = 0.0;
+        double* row = nullptr;
+        int rowL = 0;
+        P m[3] = {P(0), P(0), P(0)};
+        if (valid) {
+            owner = g < p1 ? 0 : (g < p2 ? 1 : (g < p3 ? 2 : 3));
+            const int first = owner == 0 ? 0 : (owner == 1 ? p1 : (owner == 2 ? p2 : p3));
+            cnt = owner == 0 ? n0 : (owner == 1 ? n1 : (owner == 2 ? n2 : n3));
+            q = g - first;
+            const double* r = ws.rec[owner];
+            k = (int)r[R::K0] + q;
+            const double tk = k * r[R::DT];
+            double ys[N];
+#pragma unroll
+            for (int i = 1; i < N; i += 2) ys[i] = 0.0;
+            if (tk == r[R::TNEW]) {
+#pragma unroll
+                for (int c = 0; c < NQ; ++c) ys[2 * c] = r[R::YN + c];
+            } else {
+                const double x = sizeof(P) == 4 ? (tk - r[R::T]) * rcp_nr(r[R::H]) : (tk - r[R::T]) / r[R::H];
+#pragma unroll
+                for (int c = 0; c < NQ; ++c) {
+                    const double* f = r + R::Y + 8 * c;
+                    const double F[7] = {f[1], f[2], f[3], f[4], f[5], f[6], f[7]};
+                    ys[2 * c] = dense_value(F, f[0], x);
+                }
+            }
+            row = __builtin_bit_cast(double*, r[R::ROW]);
+            rowL = (int)r[R::L];
+            record = (int)r[R::RECORD];
+            if constexpr (SYS == SYS_CH4CO2) {
+#pragma unroll
+                for (int c = 0; c < NQ; ++c) row[(long long)k * NQ + c] = ys[2 * c];
+            } else {
+                dipole<SYS, P>(sc, ys, m);
+                const double mu0[3] = {r[R::MU0], r[R::MU0 + 1], r[R::MU0 + 2]};
+                curr = cf_value<P>(mu0, m);
+            }
+            prev_start = r[R::CURR];
+        }
+        const double up = __shfl_up(curr, 1, 64);
+        const double prev = q == 0 ? prev_start : (lane > 0 ? up : carry);
+        carry = __shfl(curr, 63, 64);
+        if (valid && SYS != SYS_CH4CO2) {
+            const int st = sample_status<P>(m, curr, prev, k, record);
+            if (st != ITEM_OK) atomicMin(&ws.fail[owner], (q << 3) | st);
+        }
+        wave_share_sync();
+        if (valid) {
+            if (SYS != SYS_CH4CO2 && q < (ws.fail[owner] >> 3)) store_sample<P>(row, rowL, record, k, m, curr);
+            if (q == cnt - 1) ws.last[owner] = curr;
+        }
+    }
+    wave_share_sync();
+}
+
+// One attempted DOP853 step of every row of the wavefront (dop853_attempt, dop853_step_shared and
+// advance of the lane kernel)
+template <int SYS, typename P>
+__device__ __forceinline__ void row_step(const SysConst& sc, const RowCtx<SYS, P>& cx, const JobDesc* __restrict__ ring,
+                                         RowItem& it, Stages& K, RowShare<SysTraits<SYS>::QP / 2>& ws)
+{
+    constexpr int N = SysTraits<SYS>::QP, NQ = N / 2;
+    using R = StepRecord<NQ>;
+    const int row = (int)(__lane_id() >> 4);
+    double yn = 0.0, h = 0.0, fac11 = 0.0;
+    int outcome = STEP_ENDED, n = 0;
+    bool end = false;
+    if (it.active) {
+        const double tend = (it.L - 1) * it.dt;
+        if (it.steps >= it.max_steps || ++it.total_steps > kMaxTotalSteps) {
+            row_finish(ring[it.job], cx.lane, it, ITEM_FAIL_STEPS, it.k - 1, 0.0f);
+        } else if (0.1 * fabs(it.h) <= fabs(it.t) * kEPS) {
+            row_finish(ring[it.job], cx.lane, it, ITEM_FAIL_STEPSIZE, it.k - 1, 0.0f);
+        } else {
+            h = it.h;
+            if (it.t + 1.01 * h - tend > 0.0) h = tend - it.t;
+            double noise;
+            row_stages<SYS, P, 1, 12>(sc, cx, it.y, h, K, noise);
+            it.nrhs += 12;
+            const double be0 = stage_sum<DOP853_ROW_B, DOP853_ROW_B>(K), be1 = stage_sum<DOP853_ROW_B, DOP853_ROW_E5>(K);
+            const double be2 = stage_sum<DOP853_ROW_B, DOP853_ROW_E3>(K);
+            const double floor_p = fabs(h) * noise;
+            yn = it.y + h * be0;
+            const double sk = it.atol + it.rtol * fmax(fabs(it.y), fabs(yn)) + ((cx.comp & 1) ? floor_p : 0.0);
+            double e5, e3;
+            if constexpr (sizeof(P) == 4) {
+                const double isk = rcp_nr(sk);
+                e5 = be1 * isk, e3 = be2 * isk;
+            } else {
+                e5 = be1 / sk, e3 = be2 / sk;
+            }
+            double err = sum_squares<N>(e5);
+            const double err2 = sum_squares<N>(e3);
+            double deno = err + 0.01 * err2;
+            if (deno <= 0.0) deno = 1.0;
+            err = fabs(h) * err * sqrt(1.0 / (N * deno));
+            fac11 = sqrt(sqrt(sqrt(err)));
+            if (!(err == err) || !(h == h)) {
+                row_finish(ring[it.job], cx.lane, it, ITEM_FAIL_STEPSIZE, it.k - 1, 0.0f);
+            } else if (err > 1.0) {
+                it.h = h / fmin(1.0 / 0.333, fac11 / 0.9);
+                it.reject = 1;
+                outcome = STEP_REJECTED;
+            } else {
+                ++it.steps;
+                outcome = STEP_ACCEPTED;
+                const double tnew = it.t + h;
+                if (it.k < it.L && it.k * it.dt <= tnew) {
+                    double nz_dense;
+                    row_stages<SYS, P, 13, 15>(sc, cx, it.y, h, K, nz_dense);
+                    it.nrhs += 3;
+                    double F[7];
+                    const double dy = yn - it.y;
+                    F[0] = dy;
+                    F[1] = h * K.k0 - dy;
+                    F[2] = 2.0 * dy - h * (K.k12 + K.k0);
+                    F[3] = h * stage_sum<DOP853_ROW_D, DOP853_ROW_D>(K);
+                    F[4] = h * stage_sum<DOP853_ROW_D, DOP853_ROW_D + 1>(K);
+                    F[5] = h * stage_sum<DOP853_ROW_D, DOP853_ROW_D + 2>(K);
+                    F[6] = h * stage_sum<DOP853_ROW_D, DOP853_ROW_D + 3>(K);
+                    // the samples of the step, up to the one that ends the item
+                    double FR[7];
+#pragma unroll
+                    for (int d = 0; d < 7; ++d) FR[d] = bcast<4>(F[d]);
+                    const double R0 = bcast<4>(it.y), R1 = bcast<4>(yn);
+                    double span = 0.0;
+#pragma unroll
+                    for (int d = 0; d < 7; ++d) span += fabs(FR[d]);
+                    const double rmax = R0 + span * (1.0 + 1e-12) + 1e-12 * fabs(R0);
+                    if (rmax < it.Rcut && R1 < it.Rcut) {
+                        int kf = (int)fmin(floor(tnew / it.dt), (double)(it.L - 1));
+                        while (kf + 1 <= it.L - 1 && (kf + 1) * it.dt <= tnew) ++kf;
+                        while (kf > it.k && kf * it.dt > tnew) --kf;
+                        n = kf - it.k + 1;
+                        end = kf + 1 >= it.L;
+                    } else {
+                        for (int k = it.k; k < it.L && k * it.dt <= tnew; ++k) {
+                            ++n;
+                            const double tk = k * it.dt;
+                            const double Rk = tk == tnew ? R1 : dense_value(FR, R0, (tk - it.t) / h);
+                            if (Rk > it.Rcut || k + 1 >= it.L) {
+                                end = true;
+                                break;
+                            }
+                        }
+                    }
+                    double* r = ws.rec[row];
+                    if (cx.lane < N && !(cx.lane & 1)) {
+                        const int c = cx.lane >> 1;
+                        r[R::YN + c] = yn;
+                        r[R::Y + 8 * c] = it.y;
+#pragma unroll
+                        for (int d = 0; d < 7; ++d) r[R::Y + 8 * c + 1 + d] = F[d];
+                    }
+                    if (cx.lane == 1) {
+                        r[R::T] = it.t;
+                        r[R::H] = h;
+                        r[R::TNEW] = tnew;
+                        r[R::DT] = it.dt;
+                        r[R::K0] = (double)it.k;
+                    } else if (cx.lane == 3) {
+                        r[R::MU0] = it.mx;
+                        r[R::MU0 + 1] = it.my;
+                        r[R::MU0 + 2] = it.mz;
+                        r[R::CURR] = it.curr;
+                        r[R::ROW] = __builtin_bit_cast(double, it.row);
+                        r[R::L] = (double)it.L;
+                        r[R::RECORD] = (double)it.record;
+                    }
+                }
+            }
+        }
+    }
+    row_samples<SYS, P>(sc, ws, n);
+    if (outcome != STEP_ACCEPTED) return;
+    if (n > 0) {
+        const int f = ws.fail[row];
+        if (f != 0x7fffffff) {
+            row_finish(ring[it.job], cx.lane, it, f & 7, it.k + (f >> 3) - 1, 0.0f);
+            return;
+        }
+        it.steps = 0;
+        if (end) {
+            double yv[N];
+            gather<double, N>(yn, yv);
+            const float drift = (float)fabs(hamiltonian<SYS, P>(sc, yv) - it.E0);
+            row_finish(ring[it.job], cx.lane, it, ITEM_OK, it.k + n - 1, drift);
+            return;
+        }
+        it.k += n;
+        it.prev = it.curr;
+        it.curr = ws.last[row];
+    }
+    if constexpr (sizeof(P) == 4) {
+        if (bcast<5>(it.y) > 0.0 && bcast<5>(yn) <= 0.0) {
+            const JobDesc& jb = ring[it.job];
+            if (jb.orbit_items) {
+                if (cx.lane == 0) {
+                    const int at = atomicAdd(jb.orbit_count, 1);
+                    jb.orbit_items[at] = (int)it.local;
+                }
+                row_finish(jb, cx.lane, it, ITEM_ORBIT, it.k - 1, 0.0f);
+                return;
+            }
+        }
+    }
+    // advance: y <- y_new, f(y) <- K12 (first-same-as-last), the next step size
+    const double tend = (it.L - 1) * it.dt;
+    it.y = yn;
+    K.k0 = K.k12;
+    it.t = it.t + h;
+    const double fac = fmax(1.0 / 6.0, fmin(1.0 / 0.333, fac11 / 0.9));
+    double hnew = h / fac;
+    if (fabs(hnew) > tend) hnew = tend;
+    if (it.reject) {
+        hnew = fmin(fabs(hnew), fabs(h));
+        it.reject = 0;
+    }
+    it.h = hnew;
+}
+
+// ------------------------------------------------------------------ the kernel
+// Row r of wavefront w of the grid holds the pool slot of rank r * (wavefronts) + w, so few
+// trajectories spread one per wavefront; rank q is slot (q % W) * 64 + q / W of the pool's W
+// wavefronts (repack_move_kernel).  Rows r < rows_used refill from the queue.
+template <int SYS, typename P, int W>
+__global__ void __launch_bounds__(kRowBlock, W) row_cf_kernel(SysConst sc, const JobDesc* __restrict__ ring, PoolCtl ctl,
+                                                              LaneSlots sl, int rows_used)
+{
+    constexpr int N = SysTraits<SYS>::QP, NQ = N / 2;
+    __shared__ Co2ArTables<P> s_tab;
+    __shared__ RowShare<NQ> s_share[kRowBlock / 64];
+    __shared__ P s_scratch[SYS == SYS_CH4CO2 ? kRowBlock / 16 : 1][5 * 16];
+    const SysConst scl = stage_tables<SYS, P>(sc, &s_tab);
+    const int wave = (int)(threadIdx.x >> 6);
+    RowShare<NQ>& share = s_share[wave];
+    const RowCtx<SYS, P> cx = row_ctx<SYS, P>(scl, s_scratch[SYS == SYS_CH4CO2 ? threadIdx.x >> 4 : 0]);
+    const int row = (int)((threadIdx.x & 63) >> 4);
+    const long long waves = (long long)gridDim.x * (kRowBlock / 64);
+    const long long rank = row * waves + (long long)blockIdx.x * (kRowBlock / 64) + wave;
+    const long long S = sl.S, W64 = S / 64;
+    const long long slot = (rank % W64) * 64 + rank / W64;
+    const bool mine = rank < S;
+    const long long t_end = wall_clock64() + ctl.ticks;
+    RowItem it{};
+    Stages K{};
+    it.job = mine ? sl.i[slot] : -1;
+    it.active = it.job >= 0;
+    if (it.active) {
+        it.y = sl.d[cx.comp * S + slot];
+        K.k0 = sl.d[(N + cx.comp) * S + slot];
+        const double* d = sl.d + 2 * N * S + slot;
+        it.t = d[0];
+        it.h = d[S];
+        it.E0 = d[2 * S];
+        it.mx = d[3 * S];
+        it.my = d[4 * S];
+        it.mz = d[5 * S];
+        it.prev = d[6 * S];
+        it.curr = d[7 * S];
+        it.k = sl.i[S + slot];
+        it.steps = sl.i[2 * S + slot];
+        it.total_steps = sl.i[3 * S + slot];
+        it.nrhs = sl.i[4 * S + slot];
+        it.reject = sl.i[5 * S + slot];
+        it.local = sl.local[slot];
+        row_job(ring[it.job], it);
+    }
+    bool queue_open = mine && row < rows_used;
+    for (;;) {
+        if (wall_clock64() >= t_end) break;
+        if (!it.active && queue_open) {
+            bool got = false;
+            while (!got) {
+                long long g = -1;
+                if (cx.lane == 0 &&
+                    __hip_atomic_load(ctl.next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < ctl.total)
+                    g = (long long)atomicAdd(ctl.next, 1ull);
+                g = bcast<0>(g);
+                if (g < 0 || (unsigned long long)g >= ctl.total) break;
+                int j = ring_job(ring, ctl, (unsigned long long)g);
+                unsigned long long item = (unsigned long long)g;
+                if (ring[j].order) {
+                    item = (unsigned long long)(ring[j].order_base + ring[j].order[g - ring[j].order_base]);
+                    j = ring_job(ring, ctl, item);
+                }
+                got = row_init<SYS, P>(scl, cx, ring[j], j, (long long)item - ring[j].item_begin, it, K);
+            }
+            queue_open = got;
+        }
+        if (__ballot(it.active) == 0) break;
+        row_step<SYS, P>(scl, cx, ring, it, K, share);
+    }
+    if (!mine) return;
+    if (!it.active) {
+        if (cx.lane == 0) sl.i[slot] = -1;
+        return;
+    }
+    if (cx.lane < N) {
+        sl.d[cx.comp * S + slot] = it.y;
+        sl.d[(N + cx.comp) * S + slot] = K.k0;
+    }
+    if (cx.lane == 0) {
+        double* d = sl.d + 2 * N * S + slot;
+        d[0] = it.t;
+        d[S] = it.h;
+        d[2 * S] = it.E0;
+        d[3 * S] = it.mx;
+        d[4 * S] = it.my;
+        d[5 * S] = it.mz;
+        d[6 * S] = it.prev;
+        d[7 * S] = it.curr;
+        sl.i[slot] = it.job;
+        sl.i[S + slot] = it.k;
+        sl.i[2 * S + slot] = it.steps;
+        sl.i[3 * S + slot] = it.total_steps;
+        sl.i[4 * S + slot] = it.nrhs;
+        sl.i[5 * S + slot] = it.reject;
+        sl.local[slot] = it.local;
+    }
+}
+
+template <int SYS, typename P, int W>
+static hipError_t launch_rows(const SysConst& sc, const JobDesc* ring, const PoolCtl& ctl, const LaneSlots& sl, int wgs,
+                              int rows_used, hipStream_t st)
+{
+    hipLaunchKernelGGL((row_cf_kernel<SYS, P, W>), dim3((unsigned)wgs), dim3(kRowBlock), 0, st, sc, ring, ctl, sl,
+                       rows_used);
+    return hipGetLastError();
+}
+
+// one slice of a pool on the row kernel: wgs workgroups of 16 rows, rows_used rows of a wavefront
+// take new items; the pool's live slots are ranks below 16 wgs
+hipError_t run_rows(int sys, bool mixed, const SysConst& sc, const JobDesc* ring, const PoolCtl& ctl, const LaneSlots& sl,
+                    int wgs, int rows_used, hipStream_t st)
+{
+    if (wgs < 1 || rows_used < 1 || rows_used > 4) return hipErrorInvalidValue;
+    if (sys == SYS_CH4CO2)
+        return mixed ? launch_rows<SYS_CH4CO2, float, 2>(sc, ring, ctl, sl, wgs, rows_used, st)
+                     : launch_rows<SYS_CH4CO2, double, 2>(sc, ring, ctl, sl, wgs, rows_used, st);
+    if (sys == SYS_HEAR)
+        return mixed ? launch_rows<SYS_HEAR, float, 2>(sc, ring, ctl, sl, wgs, rows_used, st)
+                     : launch_rows<SYS_HEAR, double, 2>(sc, ring, ctl, sl, wgs, rows_used, st);
+    return mixed ? launch_rows<SYS_CO2AR, float, 2>(sc, ring, ctl, sl, wgs, rows_used, st)
+                 : launch_rows<SYS_CO2AR, double, 2>(sc, ring, ctl, sl, wgs, rows_used, st);
+}
+
+}  // namespace hh

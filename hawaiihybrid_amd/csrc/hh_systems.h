@@ -51,14 +51,17 @@ struct SysConst {
 // Tang-Toennies form V = A exp(-a1 R - a2 R^2) - sum_{n=3}^{8} C_2n f_2n(R)/R^2n with
 // f_2n = 1 - exp(-bR) sum_{k<=2n} (bR)^k/k!; derivative analytic.  Kept in FP64 in every
 // engine mode: f_2n cancels to 1e-5 below R ~ 5 bohr, beyond what FP32 can carry.
-__device__ __forceinline__ double hear_dV(double R)
+constexpr double kHearA = 0.2303058634e2, kHearA1 = 0.163051044e1, kHearA2 = 0.4680016e-1, kHearB = 0.16274792500000e1;
+
+// e = exp(-b R), ea = exp(-a1 R - a2 R^2)
+__device__ __forceinline__ double hear_dV_exps(double R, double e, double ea)
 {
-    const double A = 0.2303058634e2, a1 = 0.163051044e1, a2 = 0.4680016e-1, b = 0.16274792500000e1;
+    const double A = kHearA, a1 = kHearA1, a2 = kHearA2, b = kHearB;
     const double C[6] = {0.940835513e1, 0.165523018e3, 0.379715796e4, 0.1165179999e6, 0.466258000e7,
                          0.236861000e9};
-    const double x = b * R, e = exp(-x), inv = 1.0 / R, inv2 = inv * inv;
+    const double x = b * R, inv = 1.0 / R, inv2 = inv * inv;
     double term = 1.0, sum = 1.0;
-    double dV = A * exp(-a1 * R - a2 * R * R) * (-a1 - 2.0 * a2 * R);
+    double dV = A * ea * (-a1 - 2.0 * a2 * R);
     double ip = inv2 * inv2;  // R^-4
     int k = 0;
 #pragma unroll
@@ -73,6 +76,12 @@ __device__ __forceinline__ double hear_dV(double R)
         dV -= C[n - 3] * (b * e * term * ip - 2.0 * n * (1.0 - e * sum) * ip * inv);
     }
     return dV;
+}
+
+__device__ __forceinline__ double hear_dV(double R)
+{
+    const double x = kHearB * R;
+    return hear_dV_exps(R, exp(-x), exp(-kHearA1 * R - kHearA2 * R * R));
 }
 
 __device__ __forceinline__ double hear_V(double R)
@@ -221,6 +230,38 @@ struct Trig {
 // FP32 gradient noisy, 1e-6 relative and more where the terms nearly cancel).
 constexpr double kF32NoiseUnits = 8.0 / 16777216.0;
 
+// cos(theta_m) and its derivatives in the four angles
+template <typename P>
+struct Co2ArAngles {
+    P c, dPhi, dTheta, dphi, dtheta;
+};
+
+template <typename P>
+__device__ __forceinline__ Co2ArAngles<P> co2ar_angles(P sP, P cP, P sT, P cT, P sp, P cp, P st, P ct)
+{
+    Co2ArAngles<P> g;
+    const P Rx = sT * cP, Ry = sT * sP, Rz = cT;
+    const P ux = st * cp, uy = st * sp, uz = ct;
+    P c = Rx * ux + Ry * uy + Rz * uz;
+    c = c > P(1) ? P(1) : (c < P(-1) ? P(-1) : c);
+    g.c = c;
+    g.dPhi = -Ry * ux + Rx * uy;                       // dRhat/dPhi . u
+    g.dTheta = cT * cP * ux + cT * sP * uy - sT * uz;  // dRhat/dTheta . u
+    g.dphi = -Rx * uy + Ry * ux;                       // Rhat . du/dphi
+    g.dtheta = ct * cp * Rx + ct * sp * Ry - st * Rz;  // Rhat . du/dtheta
+    return g;
+}
+
+template <typename P>
+__device__ __forceinline__ void co2ar_gradient(const Co2ArAngles<P>& g, P dVdR, P dVdc, double* dV)
+{
+    dV[0] = (double)(dVdc * g.dPhi);
+    dV[1] = (double)(dVdc * g.dTheta);
+    dV[2] = (double)dVdR;
+    dV[3] = (double)(dVdc * g.dphi);
+    dV[4] = (double)(dVdc * g.dtheta);
+}
+
 // CO2-Ar lab-frame gradient dV/dq, q = [Phi, Theta, R, phi1, theta1] (Hartree / bohr, rad).
 // noise: for P = float an absolute bound on the rounding noise of every component (0 for FP64).
 template <typename P>
@@ -245,15 +286,8 @@ __device__ __forceinline__ void co2ar_dpes(const Co2ArTables<P>* __restrict__ tb
     P sP, cP, sp, cp;
     sincos_p<P>(y[0], &sP, &cP);
     sincos_p<P>(y[6], &sp, &cp);
-    const P sT = (P)tr.sT, cT = (P)tr.cT, st = (P)tr.st, ct = (P)tr.ct;
-    const P Rx = sT * cP, Ry = sT * sP, Rz = cT;
-    const P ux = st * cp, uy = st * sp, uz = ct;
-    P c = Rx * ux + Ry * uy + Rz * uz;
-    c = c > P(1) ? P(1) : (c < P(-1) ? P(-1) : c);
-    const P dc_dPhi = -Ry * ux + Rx * uy;                       // dRhat/dPhi . u
-    const P dc_dTheta = cT * cP * ux + cT * sP * uy - sT * uz;  // dRhat/dTheta . u
-    const P dc_dphi = -Rx * uy + Ry * ux;                       // Rhat . du/dphi
-    const P dc_dtheta = ct * cp * Rx + ct * sp * Ry - st * Rz;  // Rhat . du/dtheta
+    const Co2ArAngles<P> g = co2ar_angles<P>(sP, cP, (P)tr.sT, (P)tr.cT, sp, cp, (P)tr.st, (P)tr.ct);
+    const P c = g.c;
 
     P Pl[11], dPl[11];
     legendre10<P>(c, Pl, dPl);
@@ -284,11 +318,7 @@ __device__ __forceinline__ void co2ar_dpes(const Co2ArTables<P>* __restrict__ tb
         }
     }
     noise = sizeof(P) == 4 ? kF32NoiseUnits * (double)mag : 0.0;
-    dV[0] = (double)(dVdc * dc_dPhi);
-    dV[1] = (double)(dVdc * dc_dTheta);
-    dV[2] = (double)dVdR;
-    dV[3] = (double)(dVdc * dc_dphi);
-    dV[4] = (double)(dVdc * dc_dtheta);
+    co2ar_gradient<P>(g, dVdR, dVdc, dV);
 }
 
 template <typename P>
@@ -393,14 +423,10 @@ struct Ch4Co2Frame {
     P s1, c1, sp, cp, sT, cT, s2, c2;
 };
 
+// the unit vectors from the sines and cosines
 template <typename P>
-__device__ __forceinline__ void ch4co2_frame(const double* y, const Ch4Co2Trig& tr, Ch4Co2Frame<P>& f)
+__device__ __forceinline__ void ch4co2_axes(Ch4Co2Frame<P>& f)
 {
-    sincos_p<P>(y[0], &f.sP, &f.cP);
-    sincos_p<P>(y[6], &f.sf, &f.cf);
-    sincos_p<P>(y[12], &f.sP2, &f.cP2);
-    f.sT = (P)tr.sT, f.cT = (P)tr.cT, f.s1 = (P)tr.s1, f.c1 = (P)tr.c1;
-    f.sp = (P)tr.sp, f.cp = (P)tr.cp, f.s2 = (P)tr.s2, f.c2 = (P)tr.c2;
     f.Rh[0] = -f.sT * f.cP;
     f.Rh[1] = -f.sT * f.sP;
     f.Rh[2] = f.cT;
@@ -418,6 +444,17 @@ __device__ __forceinline__ void ch4co2_frame(const double* y, const Ch4Co2Trig& 
         o[k][1] = -f.sp * w0 + f.cp * x1;
         o[k][2] = x2;
     }
+}
+
+template <typename P>
+__device__ __forceinline__ void ch4co2_frame(const double* y, const Ch4Co2Trig& tr, Ch4Co2Frame<P>& f)
+{
+    sincos_p<P>(y[0], &f.sP, &f.cP);
+    sincos_p<P>(y[6], &f.sf, &f.cf);
+    sincos_p<P>(y[12], &f.sP2, &f.cP2);
+    f.sT = (P)tr.sT, f.cT = (P)tr.cT, f.s1 = (P)tr.s1, f.c1 = (P)tr.c1;
+    f.sp = (P)tr.sp, f.cp = (P)tr.cp, f.s2 = (P)tr.s2, f.c2 = (P)tr.c2;
+    ch4co2_axes<P>(f);
 }
 
 // Stand-in site sum at R, a, b: the energy (Hartree, scaled) and gs = dV/d(R a) summed over the
@@ -464,15 +501,10 @@ __device__ __forceinline__ P ch4co2_sites(P R, const P* a, const P* b, P* gs, P*
     return V;
 }
 
-// lab gradient dV/dq[8] of the stand-in; noise: FP32 rounding bound of the components (0 in FP64)
+// lab gradient dV/dq[8] from the site sums gs = dV/d(R a), gd = dV/d(r_CO b) (CH4 frame)
 template <typename P>
-__device__ __forceinline__ void ch4co2_dpes(const double* y, const Ch4Co2Trig& tr, double* dV, double& noise)
+__device__ __forceinline__ void ch4co2_gradient(const Ch4Co2Frame<P>& f, P R, const P* gs, const P* gd, double* dV)
 {
-    Ch4Co2Frame<P> f;
-    ch4co2_frame<P>(y, tr, f);
-    const P R = (P)y[4];
-    P gs[3], gd[3], mag;
-    (void)ch4co2_sites<P>(R, f.a, f.b, gs, gd, mag);
     P ga[3], gb[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -520,8 +552,27 @@ __device__ __forceinline__ void ch4co2_dpes(const double* y, const Ch4Co2Trig& t
     dV[5] = (double)dpsi1;
     dV[6] = (double)dphi2;
     dV[7] = (double)dtheta2;
-    // each component is a sum of pair forces times a lever arm of at most R + r_CO
-    noise = sizeof(P) == 4 ? kF32NoiseUnits * (double)mag * ((double)R + ch4co2::kRCO) : 0.0;
+}
+
+// FP32 rounding bound of the gradient (0 in FP64): each component is a sum of pair forces times a
+// lever arm of at most R + r_CO
+template <typename P>
+__device__ __forceinline__ double ch4co2_noise(P R, P mag)
+{
+    return sizeof(P) == 4 ? kF32NoiseUnits * (double)mag * ((double)R + ch4co2::kRCO) : 0.0;
+}
+
+// lab gradient dV/dq[8] of the stand-in; noise: FP32 rounding bound of the components (0 in FP64)
+template <typename P>
+__device__ __forceinline__ void ch4co2_dpes(const double* y, const Ch4Co2Trig& tr, double* dV, double& noise)
+{
+    Ch4Co2Frame<P> f;
+    ch4co2_frame<P>(y, tr, f);
+    const P R = (P)y[4];
+    P gs[3], gd[3], mag;
+    (void)ch4co2_sites<P>(R, f.a, f.b, gs, gd, mag);
+    ch4co2_gradient<P>(f, R, gs, gd, dV);
+    noise = ch4co2_noise<P>(R, mag);
 }
 
 template <typename P>
@@ -555,16 +606,44 @@ struct SysTraits<SYS_CH4CO2> {
     static constexpr int QP = 16;
 };
 
+// intermolecular part of Hamilton's equations (src/hawaii.c:586-591): iR = 1/R, is = 1/sin(Theta),
+// dV = dV/d(Phi, Theta, R)
+__device__ __forceinline__ void pair_eom(double pPhi, double pTheta, double pR, double cT, double imu, double iR,
+                                         double is, const double* dV, double* yd)
+{
+    const double iR2 = iR * iR;
+    const double is2 = is * is;
+    const double a = imu * iR2;               // 1/(mu R^2)
+    yd[4] = pR * imu;
+    yd[5] = (pTheta * pTheta + pPhi * pPhi * is2) * a * iR - dV[2];
+    yd[0] = pPhi * a * is2;
+    yd[1] = -dV[0];
+    yd[2] = pTheta * a;
+    yd[3] = pPhi * pPhi * cT * a * is2 * is - dV[1];
+}
+
+// linear rotor (src/hawaii.c:494-497): ist = 1/sin(theta), dVp = dV/dphi, dVt = dV/dtheta
+__device__ __forceinline__ void linear_rotor_eom(double pphi, double ptheta, double ct, double iI, double ist,
+                                                 double dVp, double dVt, double* yd)
+{
+    const double ist2 = ist * ist;
+    yd[0] = pphi * iI * ist2;
+    yd[1] = -dVp;
+    yd[2] = ptheta * iI;
+    yd[3] = pphi * pphi * ct * iI * ist2 * ist - dVt;
+}
+
 // rhsMonomer ROTOR (src/hawaii.c:505-531): monomer state m = (phi, pphi, theta, ptheta, psi, ppsi),
-// dV = dV/d(phi, theta, psi), sin/cos of theta and psi given
+// dV = dV/d(phi, theta, psi), sin/cos of theta and psi given; is = 1/sin(theta), i0 = 1/II[0],
+// i1 = 1/II[1]
 __device__ __forceinline__ void rotor_rhs(const double* II, const double* m, const double* dV, double st, double ct,
-                                          double sp, double cp, double* d)
+                                          double sp, double cp, double is, double i0, double i1, double* d)
 {
     const double pPhi = m[1], pTheta = m[3], pPsi = m[5];
     const double t1 = (pPhi - pPsi * ct) * sp + pTheta * st * cp;
     const double t2 = (pPhi - pPsi * ct) * cp - pTheta * st * sp;
     const double t3 = pPhi * ct - pPsi, t4 = pPsi * ct - pPhi;
-    const double is = 1.0 / st, is2 = is * is, i0 = 1.0 / II[0], i1 = 1.0 / II[1];
+    const double is2 = is * is;
     d[0] = (t1 * sp * i0 + t2 * cp * i1) * is2;
     d[1] = -dV[0];
     d[2] = (t1 * cp * i0 - t2 * sp * i1) * is;
@@ -591,21 +670,9 @@ __device__ __forceinline__ void rhs(const SysConst& sc, const double* __restrict
         sincos_p<double>(y[14], &ct.s2, &ct.c2);
         double dV[8];
         ch4co2_dpes<P>(y, ct, dV, noise);
-        const double iR = recip<P>(R), iR2 = iR * iR, imu = 1.0 / mu;
-        const double is = recip<P>(ct.sT), is2 = is * is;
-        const double a = imu * iR2;
-        yd[4] = pR * imu;
-        yd[5] = (pTheta * pTheta + pPhi * pPhi * is2) * a * iR - dV[2];
-        yd[0] = pPhi * a * is2;
-        yd[1] = -dV[0];
-        yd[2] = pTheta * a;
-        yd[3] = pPhi * pPhi * ct.cT * a * is2 * is - dV[1];
-        rotor_rhs(sc.IR, y + 6, dV + 3, ct.s1, ct.c1, ct.sp, ct.cp, yd + 6);
-        const double iI = 1.0 / sc.I, ist = recip<P>(ct.s2), ist2 = ist * ist;
-        yd[12] = y[13] * iI * ist2;
-        yd[13] = -dV[6];
-        yd[14] = y[15] * iI;
-        yd[15] = y[13] * y[13] * ct.c2 * iI * ist2 * ist - dV[7];
+        pair_eom(pPhi, pTheta, pR, ct.cT, 1.0 / mu, recip<P>(R), recip<P>(ct.sT), dV, yd);
+        rotor_rhs(sc.IR, y + 6, dV + 3, ct.s1, ct.c1, ct.sp, ct.cp, 1.0 / ct.s1, 1.0 / sc.IR[0], 1.0 / sc.IR[1], yd + 6);
+        linear_rotor_eom(y[13], y[15], ct.c2, 1.0 / sc.I, recip<P>(ct.s2), dV[6], dV[7], yd + 12);
         return;
     }
     Trig tr;
@@ -619,23 +686,9 @@ __device__ __forceinline__ void rhs(const SysConst& sc, const double* __restrict
         sincos_p<double>(y[8], &tr.st, &tr.ct);
         co2ar_dpes<P>((const Co2ArTables<P>*)sc.tables, y, tr, dV, noise);
     }
-    const double iR = recip<P>(R), iR2 = iR * iR, imu = 1.0 / mu;
-    const double is = recip<P>(tr.sT), is2 = is * is;
-    const double a = imu * iR2;               // 1/(mu R^2)
-    yd[4] = pR * imu;
-    yd[5] = (pTheta * pTheta + pPhi * pPhi * is2) * a * iR - dV[2];
-    yd[0] = pPhi * a * is2;
-    yd[1] = -dV[0];
-    yd[2] = pTheta * a;
-    yd[3] = pPhi * pPhi * tr.cT * a * is2 * is - dV[1];
-    if constexpr (SYS == SYS_CO2AR) {
-        const double iI = 1.0 / sc.I, ist = recip<P>(tr.st), ist2 = ist * ist;
-        const double pphi = y[7], ptheta = y[9];
-        yd[6] = pphi * iI * ist2;
-        yd[7] = -dV[3];
-        yd[8] = ptheta * iI;
-        yd[9] = pphi * pphi * tr.ct * iI * ist2 * ist - dV[4];
-    }
+    pair_eom(pPhi, pTheta, pR, tr.cT, 1.0 / mu, recip<P>(R), recip<P>(tr.sT), dV, yd);
+    if constexpr (SYS == SYS_CO2AR)
+        linear_rotor_eom(y[7], y[9], tr.ct, 1.0 / sc.I, recip<P>(tr.st), dV[3], dV[4], yd + 6);
 }
 
 template <int SYS, typename P>

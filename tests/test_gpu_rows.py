@@ -1,0 +1,46 @@
+"""The row kernel (one trajectory per 16-lane row: small requests and the tail of large ones) against
+the lane kernel (one trajectory per lane): the same bits.
+
+A job alone runs on the row kernel from its first step; beside a filler of 9000 trajectories in
+the same call it starts on the lane kernel and, depending on its items, ends on either.  Every
+item's row, length, status, right-hand-side count and energy drift, and the job's CF, must be equal
+bit for bit: both kernels run the same expressions in the same order.  Sizes: one row, less and more
+than a wavefront's four rows, more rows than wavefronts."""
+import numpy as np
+import pytest
+
+import hawaiihybrid_amd as H
+
+pytestmark = pytest.mark.gpu
+
+SYSTEMS = {"hear": (H.he_ar, 300.0, H.PESMIN_HEAR, 4.0), "co2ar": (H.co2_ar, 200.0, H.PESMIN_CO2AR, 4.0),
+           "ch4co2": (H.ch4_co2, 300.0, H.PESMIN_CH4CO2, 4.75)}
+
+
+@pytest.fixture(scope="module")
+def eng():
+    e = H.Engine(0)
+    yield e
+    e.close()
+
+
+@pytest.mark.parametrize("which", ["hear", "co2ar", "ch4co2"])
+@pytest.mark.parametrize("prec", [H.PREC_FP64, H.PREC_MIXED])
+@pytest.mark.parametrize("n", [1, 3, 17, 1500])
+def test_row_kernel_gives_the_lane_kernel_bits(eng, which, prec, n):
+    make, T, pesmin, rmin = SYSTEMS[which]
+    L = 1024 if n < 100 else 600
+    # injected close in, so that the trajectories collide within the series
+    smp = H.Sampler(H.IC_R0_INJECT, H.PAIR_FREE, T, rmin, 40.0, pesmin, 15.0)
+    ic = H.sample_ics(make(), smp, 5, n + 9000)[0]
+    x, filler = eng.to_device_soa(ic[:n]), eng.to_device_soa(ic[n:])
+    p = H.cf_params(L, rtol=1e-10 if prec == H.PREC_MIXED else 1e-12, Rcut=20.0, precision=prec)
+    alone, _ = eng.cf_run(make(), p, [x])
+    a = eng.items(0, n, L, rows=True)
+    beside, _ = eng.cf_run(make(), p, [x, filler])
+    b = eng.items(0, n, L, rows=True)
+    print(f"rows {which} prec {prec} n {n}: {int(a['nrhs'].sum())} right-hand sides", flush=True)
+    assert a["nrhs"].sum() > 0
+    for key in ("len", "status", "nrhs", "e_drift", "rows"):
+        assert np.array_equal(a[key], b[key]), key
+    assert np.array_equal(alone[0].cpu().numpy(), beside[0].cpu().numpy())
