@@ -10,17 +10,22 @@
 // trajectory kernel records the lab coordinates of every sample (record mode 3) and two kernels
 // here finish a job:
 //   ch4co2_dipole_kernel  one sample per lane, 64 consecutive samples of one trajectory per
-//                         workgroup of kDipWaves wavefronts: the frame of CH4 in every wavefront,
+//                         workgroup of kDipWaves<P> wavefronts: the frame of CH4 in every wavefront,
 //                         X and Y into LDS (a column per sample; the wavefronts share the orders
-//                         m), then each wavefront runs its share of the basis functions (split
-//                         by term count) over the term list, read by the whole wavefront at once
-//                         (uniform indices: scalar loads), with the radial functions of the
-//                         lane's interval (vector loads; the lanes share few intervals, so they
-//                         hit the same lines); the shares' partial dipoles are summed in
-//                         wavefront order and mu_lab = S1^T mu overwrites the sample's first
-//                         three coordinates.  The 287 harmonics of 64 samples take 73 KB (FP32)
-//                         or 147 KB (FP64) of LDS, so one wavefront per workgroup would leave
-//                         two or three of a CU's four SIMDs idle.
+//                         m), then each wavefront runs its share of the blocks below; the shares'
+//                         partial dipoles are summed in wavefront order and mu_lab = S1^T mu
+//                         overwrites the sample's first three coordinates.
+// The 320 basis functions (one of them 0) fall into 84 blocks of one (l_a, l_b), 1 to 9 functions each, and within a
+// block every product X_x Y_y belongs to one component c and to nearly all of its functions: 8658
+// products in all, and dense coefficient lists of 36864 entries where the expansion has 31802 terms.
+// So a product is formed once and multiplied into the block's sums, one FMA per entry with the
+// coefficient in a scalar register, and two LDS reads serve a block's 4.3 entries instead of one
+// term.  Four products at a time (a quad): their indices and coefficients are one contiguous scalar
+// read.  The 287 harmonics of 64 samples take 73 KB (FP32) or 147 KB (FP64) of
+// LDS: two workgroups or one per CU.
+// Bound: vector issue, 45 k FMAs and products per sample (about 60 k with the radial functions and
+// harmonics; two thirds of the rate), where the term-by-term loop over 31802 terms was bound by its
+// 64 k LDS reads: 12289 x 1024 samples in FP32 122.7 -> 28.6 ms (103 -> 440 M samples/s).
 //   ch4co2_cf_rows_kernel one wavefront per trajectory: c_k = mu(0).mu(t_k), the sample checks of
 //                         correlation_eval (src/hawaii.c:2181-2236) in sample order, the CF rows
 //                         the reduction reads; a failed check marks the trajectory.
@@ -29,52 +34,129 @@
 // three-term recurrence in l at fixed m.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cstring>
+#include <map>
+#include <set>
+#include <utility>
+#include <vector>
+
 #include "ch4co2_dipole_tables.h"
 #include "hh_engine.h"
 #include "hh_systems.h"
 
 namespace hh {
 
-constexpr int kDipWaves = 4;   // wavefronts per dipole workgroup
+// wavefronts per dipole workgroup: with two workgroups per CU (FP32) eight each, with one (FP64)
+// sixteen, so four wavefronts per SIMD cover the scalar reads' latency.  196624 samples of 64 in FP32
+// take 42.9, 28.6 and 36.3 ms with 4, 8 and 16; 200000 points in FP64 2.10, 1.31 and 1.04 ms.
+template <typename P>
+constexpr int kDipWaves = sizeof(P) == 4 ? 8 : 16;
+constexpr int kDipBlocks = 84; // (l_a, l_b) blocks
+constexpr int kDipMaxNB = 9;   // basis functions of the largest block
+constexpr int kDipQuads = 2304, kDipCoefs = 39936;   // quads of products and their coefficients (upper bounds)
+
+typedef unsigned int dip_u4 __attribute__((ext_vector_type(4)));
+
+// One block: its basis functions are rows [pos, pos + nb) of the radial table; the quads of component
+// c are [quad[c], quad[c + 1]), the coefficients of quad q the 4 nb values from coef0 + 4 nb (q -
+// quad[0]), function-major.
+struct DipBlock {
+    int nb, pos, coef0, pad;
+    int quad[4];
+};
 
 template <typename P>
 struct Ch4Co2DipTables {
-    P radial[HH_CH4CO2_NINT + 1][HH_CH4CO2_NB][4];   // row NINT: the tail (c4, c5, c6, 0)
-    P coef[HH_CH4CO2_NTERMS];
-    unsigned xy[HH_CH4CO2_NTERMS];   // x | y << 8 (32-bit: read with scalar loads)
-    int start[HH_CH4CO2_NB][4];
+    P radial[HH_CH4CO2_NINT + 1][HH_CH4CO2_NB][4];   // in block order; row NINT: the tail (c4, c5, c6, 0)
+    P coef[kDipCoefs];
+    dip_u4 xy[kDipQuads];        // x | y << 16 of a quad's products
+    DipBlock block[kDipBlocks];  // in wavefront order
+    int wave0[kDipWaves<P> + 1];    // wavefront w takes blocks [wave0[w], wave0[w + 1])
     double bounds[HH_CH4CO2_NINT];
     double centre[HH_CH4CO2_NINT];
-    int bsplit[kDipWaves + 1];   // wavefront w takes basis functions [bsplit[w], bsplit[w + 1])
 };
 
 template <typename P>
 void fill_ch4co2_tables(Ch4Co2DipTables<P>& t)
 {
+    // l of an X index (l^2 ..) and of a Y index (even l: l (l - 1) / 2 ..)
+    auto la = [](int x) { int l = 0; while ((l + 1) * (l + 1) <= x) ++l; return l; };
+    auto lb = [](int y) { int l = 0; while ((l + 2) * (l + 1) / 2 <= y) l += 2; return l; };
+    struct Host {
+        std::vector<int> fn;                        // basis functions
+        std::vector<std::pair<int, int>> prod[3];   // products (x, y) of each component
+        long cost = 0;
+    };
+    std::map<std::pair<int, int>, Host> blocks;
+    for (int b = 0; b < HH_CH4CO2_NB; ++b)
+        if (HH_CH4CO2_START[b][3] > HH_CH4CO2_START[b][0]) {
+            const unsigned xy = HH_CH4CO2_XY[HH_CH4CO2_START[b][0]];
+            blocks[{la(xy & 0xff), lb(xy >> 8)}].fn.push_back(b);
+        }
+    std::vector<Host*> order;
+    for (auto& kv : blocks) {
+        Host& h = kv.second;
+        h.cost = 24 + 12 * (long)h.fn.size();
+        for (int c = 0; c < 3; ++c) {
+            std::set<std::pair<int, int>> used;
+            for (int b : h.fn)
+                for (int e = HH_CH4CO2_START[b][c]; e < HH_CH4CO2_START[b][c + 1]; ++e)
+                    used.insert({(int)(HH_CH4CO2_XY[e] & 0xff), (int)(HH_CH4CO2_XY[e] >> 8)});
+            h.prod[c].assign(used.begin(), used.end());
+            h.cost += (long)(h.prod[c].size() + 3) / 4 * (8 + 4 * (long)h.fn.size());
+        }
+        order.push_back(&h);
+    }
+    // blocks to wavefronts: the costliest first, each to the least loaded wavefront
+    std::stable_sort(order.begin(), order.end(), [](const Host* a, const Host* b) { return a->cost > b->cost; });
+    constexpr int waves = kDipWaves<P>;
+    std::vector<Host*> share[waves];
+    long load[waves] = {};
+    for (Host* h : order) {
+        const int w = (int)(std::min_element(load, load + waves) - load);
+        share[w].push_back(h);
+        load[w] += h->cost;
+    }
+    std::memset(&t, 0, sizeof t);
+    int nblk = 0, pos = 0, quad = 0, coef = 0;
+    for (int w = 0; w < waves; ++w) {
+        t.wave0[w] = nblk;
+        for (const Host* h : share[w]) {
+            const int nb = (int)h->fn.size();
+            DipBlock& bl = t.block[nblk++];
+            bl.nb = nb;
+            bl.pos = pos;
+            bl.coef0 = coef;
+            for (int j = 0; j < nb; ++j, ++pos) {
+                const int b = h->fn[j];
+                for (int k = 0; k < HH_CH4CO2_NINT; ++k)
+                    for (int i = 0; i < 4; ++i) t.radial[k][pos][i] = (P)HH_CH4CO2_RADIAL[k][b][i];
+                for (int i = 0; i < 3; ++i) t.radial[HH_CH4CO2_NINT][pos][i] = (P)HH_CH4CO2_TAIL[b][i];
+            }
+            for (int c = 0; c < 3; ++c) {
+                bl.quad[c] = quad;
+                for (size_t p0 = 0; p0 < h->prod[c].size(); p0 += 4, ++quad, coef += 4 * nb)
+                    for (int u = 0; u < 4; ++u) {
+                        if (p0 + u >= h->prod[c].size()) continue;   // padded: coefficients 0
+                        const std::pair<int, int> xy = h->prod[c][p0 + u];
+                        t.xy[quad][u] = (unsigned)xy.first | (unsigned)xy.second << 16;
+                        for (int j = 0; j < nb; ++j) {
+                            const int b = h->fn[j];
+                            for (int e = HH_CH4CO2_START[b][c]; e < HH_CH4CO2_START[b][c + 1]; ++e)
+                                if ((int)(HH_CH4CO2_XY[e] & 0xff) == xy.first && (int)(HH_CH4CO2_XY[e] >> 8) == xy.second)
+                                    t.coef[coef + 4 * j + u] += (P)HH_CH4CO2_COEF[e];
+                        }
+                    }
+            }
+            bl.quad[3] = quad;
+        }
+    }
+    t.wave0[waves] = nblk;
     for (int k = 0; k < HH_CH4CO2_NINT; ++k) {
         t.bounds[k] = HH_CH4CO2_BOUNDS[k];
         t.centre[k] = HH_CH4CO2_CENTRE[k];
-        for (int b = 0; b < HH_CH4CO2_NB; ++b)
-            for (int j = 0; j < 4; ++j) t.radial[k][b][j] = (P)HH_CH4CO2_RADIAL[k][b][j];
     }
-    for (int b = 0; b < HH_CH4CO2_NB; ++b) {
-        for (int j = 0; j < 3; ++j) t.radial[HH_CH4CO2_NINT][b][j] = (P)HH_CH4CO2_TAIL[b][j];
-        t.radial[HH_CH4CO2_NINT][b][3] = P(0);
-        for (int c = 0; c < 4; ++c) t.start[b][c] = HH_CH4CO2_START[b][c];
-    }
-    for (int i = 0; i < HH_CH4CO2_NTERMS; ++i) {
-        t.coef[i] = (P)HH_CH4CO2_COEF[i];
-        t.xy[i] = HH_CH4CO2_XY[i];
-    }
-    // contiguous basis-function ranges of about equal term counts
-    t.bsplit[0] = 0;
-    int b = 0;
-    for (int w = 1; w < kDipWaves; ++w) {
-        const long long goal = (long long)HH_CH4CO2_NTERMS * w / kDipWaves;
-        while (b < HH_CH4CO2_NB && HH_CH4CO2_START[b][3] <= goal) ++b;
-        t.bsplit[w] = b;
-    }
-    t.bsplit[kDipWaves] = HH_CH4CO2_NB;
 }
 
 size_t ch4co2_table_bytes(bool f32) { return f32 ? sizeof(Ch4Co2DipTables<float>) : sizeof(Ch4Co2DipTables<double>); }
@@ -106,7 +188,7 @@ __device__ __forceinline__ void harmonics(const P* v, P (*out)[64], int lane, in
             wr = t;
             dfact *= P(2 * m - 1);
         }
-        if (m % kDipWaves != wave) continue;   // this order belongs to another wavefront
+        if (m % kDipWaves<P> != wave) continue;   // this order belongs to another wavefront
         // Q_l^m = d^m P_l / dx^m: Q_m^m = (2m - 1)!!, Q_{m+1}^m = (2m + 1) x Q_m^m,
         // (l - m) Q_l^m = (2l - 1) x Q_{l-1}^m - (l + m - 1) Q_{l-2}^m
         P q0 = P(0), q1 = dfact;
@@ -130,15 +212,52 @@ __device__ __forceinline__ void harmonics(const P* v, P (*out)[64], int lane, in
     }
 }
 
-// One workgroup = 64 consecutive samples of one trajectory (blockIdx.y), kDipWaves wavefronts;
+// mu[c] += sum over the block's functions j of r_j(R) sum over the products of coef X_x Y_y, for the
+// lane's sample
+template <typename P, int NB>
+__device__ __forceinline__ void dipole_block(const Ch4Co2DipTables<P>* __restrict__ tb, const DipBlock& bl,
+                                             const P (*sX)[64], const P (*sY)[64], int lane, int kint, P t, P ir, P ir4,
+                                             bool tail, P (&mu)[3])
+{
+    P r[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        const P* rc = tb->radial[kint][bl.pos + j];
+        r[j] = tail ? (rc[0] + (rc[1] + rc[2] * ir) * ir) * ir4 : ((rc[3] * t + rc[2]) * t + rc[1]) * t + rc[0];
+    }
+    const int q0 = bl.quad[0];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        P acc[NB];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[j] = P(0);
+#pragma unroll 2
+        for (int q = bl.quad[c]; q < bl.quad[c + 1]; ++q) {
+            const dip_u4 xy = tb->xy[q];
+            const P* cf = tb->coef + (bl.coef0 + 4 * NB * (q - q0));   // by index: stays a scalar address
+            P p[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) p[u] = sX[xy[u] & 0xffffu][lane] * sY[xy[u] >> 16][lane];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int j = 0; j < NB; ++j) acc[j] += cf[4 * j + u] * p[u];
+        }
+#pragma unroll
+        for (int j = 0; j < NB; ++j) mu[c] += acc[j] * r[j];
+    }
+}
+
+// One workgroup = 64 consecutive samples of one trajectory (blockIdx.y), kDipWaves<P> wavefronts;
 // coordinates rec[8] per sample (Phi, Theta, R, phi1, theta1, psi1, phi2, theta2) are replaced by
 // (mu_x, mu_y, mu_z).
 template <typename P>
-__global__ void __launch_bounds__(64 * kDipWaves) ch4co2_dipole_kernel(JobDesc jb, const Ch4Co2DipTables<P>* __restrict__ tb)
+__global__ void __launch_bounds__(64 * kDipWaves<P>) ch4co2_dipole_kernel(JobDesc jb, const Ch4Co2DipTables<P>* __restrict__ tb)
 {
     __shared__ P sX[HH_CH4CO2_NX][64];
     __shared__ P sY[HH_CH4CO2_NY][64];
-    __shared__ P sMu[kDipWaves][3][64];
+    P (*sMu)[3][64] = reinterpret_cast<P (*)[3][64]>(&sX[0][0]);   // once the harmonics have been read
+    static_assert(kDipWaves<P> * 3 <= HH_CH4CO2_NX, "the partial dipoles fit the harmonics' place");
     const long long item = blockIdx.y;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -186,23 +305,26 @@ __global__ void __launch_bounds__(64 * kDipWaves) ch4co2_dipole_kernel(JobDesc j
     const P ir = (P)(1.0 / R), ir4 = ir * ir * ir * ir;
     const bool tail = kint == HH_CH4CO2_NINT;
     P mu[3] = {P(0), P(0), P(0)};
-    const int b0 = tb->bsplit[wave], b1 = tb->bsplit[wave + 1];
+    const int b0 = tb->wave0[wave], b1 = tb->wave0[wave + 1];
 #pragma unroll 1
-    for (int bf = b0; bf < b1; ++bf) {
-        const P* rc = tb->radial[kint][bf];
-        const P r = tail ? (rc[0] + (rc[1] + rc[2] * ir) * ir) * ir4 : ((rc[3] * t + rc[2]) * t + rc[1]) * t + rc[0];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const int t0 = tb->start[bf][c], t1 = tb->start[bf][c + 1];
-            P s = P(0);
-#pragma unroll 8
-            for (int e = t0; e < t1; ++e) {
-                const unsigned xy = tb->xy[e];
-                s += tb->coef[e] * (sX[xy & 0xffu][lane] * sY[xy >> 8][lane]);
-            }
-            mu[c] += s * r;
+    for (int b = b0; b < b1; ++b) {
+        const DipBlock bl = tb->block[b];
+        switch (bl.nb) {
+#define HH_DIP_CASE(NB) \
+    case NB: dipole_block<P, NB>(tb, bl, sX, sY, lane, kint, t, ir, ir4, tail, mu); break;
+            HH_DIP_CASE(1)
+            HH_DIP_CASE(2)
+            HH_DIP_CASE(3)
+            HH_DIP_CASE(4)
+            HH_DIP_CASE(5)
+            HH_DIP_CASE(6)
+            HH_DIP_CASE(7)
+            HH_DIP_CASE(8)
+#undef HH_DIP_CASE
+        default: dipole_block<P, kDipMaxNB>(tb, bl, sX, sY, lane, kint, t, ir, ir4, tail, mu); break;
         }
     }
+    __syncthreads();
 #pragma unroll
     for (int c = 0; c < 3; ++c) sMu[wave][c][lane] = mu[c];
     __syncthreads();
@@ -212,7 +334,7 @@ __global__ void __launch_bounds__(64 * kDipWaves) ch4co2_dipole_kernel(JobDesc j
     for (int c = 0; c < 3; ++c) {
         P m = sMu[0][c][lane];
 #pragma unroll
-        for (int w = 1; w < kDipWaves; ++w) m += sMu[w][c][lane];
+        for (int w = 1; w < kDipWaves<P>; ++w) m += sMu[w][c][lane];
         mu[c] = m;
     }
     // mu_lab = Sz(phi1)^T Sx(theta1)^T Sz(psi1)^T mu
@@ -304,7 +426,7 @@ hipError_t run_ch4co2_eval_dipole(const double* y, long long n, double* records,
     jd.len = len;
     jd.n_items = 1;
     jd.L = (int)n;
-    hipLaunchKernelGGL(ch4co2_dipole_kernel<double>, dim3((unsigned)((n + 63) / 64), 1), dim3(64 * kDipWaves), 0, st, jd,
+    hipLaunchKernelGGL(ch4co2_dipole_kernel<double>, dim3((unsigned)((n + 63) / 64), 1), dim3(64 * kDipWaves<double>), 0, st, jd,
                        static_cast<const Ch4Co2DipTables<double>*>(tables));
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(ch4co2_dipole_out_kernel, dim3(g), dim3(256), 0, st, records, n, out);
@@ -315,10 +437,10 @@ hipError_t run_ch4co2_cf_rows(const JobDesc& jd, const void* tables, bool f32, h
 {
     const dim3 grid((unsigned)((jd.L + 63) / 64), (unsigned)jd.n_items);
     if (f32)
-        hipLaunchKernelGGL(ch4co2_dipole_kernel<float>, grid, dim3(64 * kDipWaves), 0, st, jd,
+        hipLaunchKernelGGL(ch4co2_dipole_kernel<float>, grid, dim3(64 * kDipWaves<float>), 0, st, jd,
                            static_cast<const Ch4Co2DipTables<float>*>(tables));
     else
-        hipLaunchKernelGGL(ch4co2_dipole_kernel<double>, grid, dim3(64 * kDipWaves), 0, st, jd,
+        hipLaunchKernelGGL(ch4co2_dipole_kernel<double>, grid, dim3(64 * kDipWaves<double>), 0, st, jd,
                            static_cast<const Ch4Co2DipTables<double>*>(tables));
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
