@@ -27,8 +27,8 @@ SOURCES = [
     # the integrators' arithmetic is what their expressions say (a * b + c inside one expression
     # becomes one FMA, nothing across statements), so kernels of different shape (one item per
     # thread, the lane pool, stage vectors in LDS or in the buffer arena) compute the same bits
-    ("hh_kernels.hip", DEVICE + ["-ffp-contract=on"]),
-    # constants hoisted out of the row kernel's loops would take all its registers
+    # (constants hoisted out of their loops would take all the registers)
+    ("hh_kernels.hip", DEVICE + ["-ffp-contract=on", "-mllvm", "-disable-machine-licm"]),
     ("hh_rows.hip", DEVICE + ["-ffp-contract=on", "-mllvm", "-disable-machine-licm"]),
     ("hh_aux.hip", DEVICE),
     ("hh_pipnn.hip", DEVICE),

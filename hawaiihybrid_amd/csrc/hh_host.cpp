@@ -46,6 +46,10 @@ namespace {
 template <typename P>
 void fill_tables(hh::Co2ArTables<P>& t)
 {
+    for (int k = 0; k < 122; ++k) {
+        t.branch[k] = 0;
+        for (int b = 0; b < 31; ++b) t.branch[k] += 0.25 * k >= HH_CO2AR_BOUNDS[b] ? 1 : 0;
+    }
     for (int b = 0; b < 32; ++b) {
         t.center[b] = HH_CO2AR_CENTER[b];
         for (int s = 0; s < 6; ++s)

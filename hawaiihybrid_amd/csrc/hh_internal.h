@@ -233,8 +233,16 @@ namespace hh {
 // the surface constants of a system for the device kernels (f32: the FP32 tables of CO2-Ar)
 inline SysConst sysconst(const hh_engine* e, const hh_system& sys, bool f32)
 {
-    SysConst sc{sys.mu, sys.I, (f32 && sys.system == HH_SYS_CO2AR) ? e->tab32.p : e->tab64.p, {0.0, 0.0, 0.0}};
-    for (int i = 0; i < 3; ++i) sc.IR[i] = sys.I_rotor[i];
+    SysConst sc{};
+    sc.mu = sys.mu;
+    sc.I = sys.I;
+    sc.tables = (f32 && sys.system == HH_SYS_CO2AR) ? e->tab32.p : e->tab64.p;
+    sc.imu = 1.0 / sys.mu;
+    sc.iI = sys.I != 0.0 ? 1.0 / sys.I : 0.0;
+    for (int i = 0; i < 3; ++i) {
+        sc.IR[i] = sys.I_rotor[i];
+        sc.iIR[i] = sys.I_rotor[i] != 0.0 ? 1.0 / sys.I_rotor[i] : 0.0;
+    }
     return sc;
 }
 // the ensemble CF of a finished job into cf_out (on the engine stream)

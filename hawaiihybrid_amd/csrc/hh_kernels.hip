@@ -382,15 +382,10 @@ __device__ __forceinline__ int dop853_attempt(const SysConst& sc, const JobDesc&
         for (int i = 0; i < N; ++i) {
             yn[i] = ln.y[i] + h * be[0][i];
             const double sk = jb.atol + jb.rtol * fmax(fabs(ln.y[i]), fabs(yn[i])) + ((i & 1) ? floor_p : 0.0);
-            if constexpr (sizeof(P) == 4) {
-                // FP32 surfaces: one Newton-refined reciprocal per component (see rcp_nr)
-                const double isk = rcp_nr(sk), e5 = be[1][i] * isk, e3 = be[2][i] * isk;
-                err += e5 * e5;
-                err2 += e3 * e3;
-            } else {
-                err += (be[1][i] / sk) * (be[1][i] / sk);
-                err2 += (be[2][i] / sk) * (be[2][i] / sk);
-            }
+            const double isk = recip<P>(sk);
+            const double e5 = divide<P>(be[1][i], sk, isk), e3 = divide<P>(be[2][i], sk, isk);
+            err += e5 * e5;
+            err2 += e3 * e3;
         }
     }
     double deno = err + 0.01 * err2;

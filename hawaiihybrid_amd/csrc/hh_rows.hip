@@ -15,9 +15,9 @@
 // whichever kernel integrates it, and the two share the slot format: a slice of a pool can run on
 // either.  The rows of a grid hold the slots of ranks 0, 1, ... of a repacked pool.
 //
-// Bound: a lone wavefront's instruction issue (about 520 instructions per FP64 CO2-Ar right-hand
-// side).  One trajectory's right-hand side: 2.3 -> 1.0 us; 1153 CO2-Ar trajectories in FP64 (L = 1024)
-// 45.3 -> 21.7 ms, 4096 He-Ar ones (L = 2048) 7.7 -> 4.3 ms.
+// Bound: a lone wavefront's instruction issue (one in 4.4 cycles).  1153 CO2-Ar trajectories in FP64
+// (L = 1024): 42 ms on the lane kernel, 21 ms with every lane evaluating both series of a sincos and
+// all components, 17 ms in this form; 4096 He-Ar ones (L = 2048) 7.4, 4.2 and 3.9 ms.
 #include <hip/hip_runtime.h>
 
 #include <utility>
@@ -53,6 +53,31 @@ __device__ __forceinline__ long long bcast(long long v)
     return __builtin_bit_cast(long long, bcast<L>(__builtin_bit_cast(double, v)));
 }
 
+// the value of another lane of the row by a DPP control: within pairs (even lane's, odd lane's, the
+// partner's) or two lanes down
+enum RowMove : int { PAIR_EVEN = 0xa0, PAIR_ODD = 0xf5, PAIR_SWAP = 0xb1, QUAD_SWAP2 = 0x4e, HALF_MIRROR = 0x141, DOWN2 = 0x112 };
+template <int CTRL>
+__device__ __forceinline__ float row_move(float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double row_move(double v)
+{
+    const rw_v2u u = __builtin_bit_cast(rw_v2u, v);
+    return __builtin_bit_cast(double, rw_v2u{(unsigned)__builtin_amdgcn_mov_dpp((int)u.x, CTRL, 0xf, 0xf, true),
+                                             (unsigned)__builtin_amdgcn_mov_dpp((int)u.y, CTRL, 0xf, 0xf, true)});
+}
+
+// slot_sum of lanes 0..5's values (lanes 6 and 7 hold 0, lanes 8..15 the same again), in every lane
+template <typename P>
+__device__ __forceinline__ P row_slot_sum(P t)
+{
+    t += row_move<PAIR_SWAP>(t);
+    t += row_move<QUAD_SWAP2>(t);
+    return t + row_move<HALF_MIRROR>(t);
+}
+
 // out[i] = lane i's value, i < N
 template <typename T, int N, int... I>
 __device__ __forceinline__ void gather_impl(T v, T (&out)[N], std::integer_sequence<int, I...>)
@@ -65,7 +90,7 @@ __device__ __forceinline__ void gather(T v, T (&out)[N])
     gather_impl<T, N>(v, out, std::make_integer_sequence<int, N>{});
 }
 
-// v[comp] by selects; the empty asm keeps the values in registers (the compiler would turn the
+// CH4-CO2: v[comp] by selects; the empty asm keeps the values in registers (the compiler would turn the
 // selects into an indexed load of an array in scratch)
 template <int N>
 __device__ __forceinline__ double pick(const double (&v)[N], int comp)
@@ -80,12 +105,17 @@ __device__ __forceinline__ double pick(const double (&v)[N], int comp)
     return r;
 }
 
-// What a lane keeps for the whole kernel: its component and the reciprocals of the constants
-// (uniform), and for CH4-CO2 its site pair (lane l < 15: CO2 site l / 5, CH4 site l % 5).
+// What a lane keeps for the whole kernel: its component, the coefficients of its half of the sine and
+// cosine (even lanes the sine's series, odd lanes the cosine's), for FP32 CO2-Ar its slot's Legendre
+// recurrence (the steps past the slot's order repeat the value), for CH4-CO2 its site pair (lane l < 15:
+// CO2 site l / 5, CH4 site l % 5).
 template <int SYS, typename P>
 struct RowCtx {
     int lane, comp;      // lane of the row; component (the last one again past QP)
-    double imu, iI, i0, i1;
+    double w[8];         // FP64 series in r^2, highest order last
+    float wf[5];         // FP32 series
+    double kin;          // the lane's constant factor: 1/mu or 1/I
+    P alpha[SYS == SYS_CO2AR && sizeof(P) == 4 ? 5 : 1], beta[SYS == SYS_CO2AR && sizeof(P) == 4 ? 5 : 1], gamma[SYS == SYS_CO2AR && sizeof(P) == 4 ? 5 : 1];
     P sgn, s2, e4, h0, h1, h2;
     P* scratch;          // CH4-CO2: the row's LDS scratch [5][16]
 };
@@ -96,13 +126,32 @@ __device__ __forceinline__ RowCtx<SYS, P> row_ctx(const SysConst& sc, P* scratch
     RowCtx<SYS, P> cx{};
     cx.lane = (int)(threadIdx.x & 15);
     cx.comp = min(cx.lane, SysTraits<SYS>::QP - 1);
-    cx.imu = 1.0 / sc.mu;
-    cx.iI = SYS == SYS_HEAR ? 0.0 : 1.0 / sc.I;
     cx.scratch = scratch;
+    const bool odd = cx.lane & 1;
+    // the coefficients of sincos_p
+    constexpr double ws[8] = {-1.0 / 6, 1.0 / 120, -1.0 / 5040, 1.0 / 362880, -1.0 / 39916800, 1.0 / 6227020800.0,
+                              -1.0 / 1307674368000.0, 1.0 / 355687428096000.0};
+    constexpr double wc[8] = {-0.5, 1.0 / 24, -1.0 / 720, 1.0 / 40320, -1.0 / 3628800, 1.0 / 479001600.0,
+                              -1.0 / 87178291200.0, 1.0 / 20922789888000.0};
+    constexpr float fs[5] = {-1.0f / 6, 1.0f / 120, -1.0f / 5040, 1.0f / 362880, 0.0f};
+    constexpr float fc[5] = {-0.5f, 1.0f / 24, -1.0f / 720, 1.0f / 40320, -1.0f / 3628800};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) cx.w[i] = odd ? wc[i] : ws[i];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) cx.wf[i] = odd ? fc[i] : fs[i];
+    cx.kin = cx.lane >= 6 ? sc.iI : sc.imu;
+    if constexpr (SYS == SYS_CO2AR && sizeof(P) == 4) {
+        const int slot = cx.lane & 7;
+#pragma unroll
+        for (int t = 0; t < 5; ++t) {
+            const LegendreEven k = legendre_even_step(t);
+            cx.alpha[t] = t < slot ? P(k.alpha) : P(0);
+            cx.beta[t] = t < slot ? P(k.beta) : P(-1);
+            cx.gamma[t] = t < slot ? P(k.gamma) : P(0);
+        }
+    }
     if constexpr (SYS == SYS_CH4CO2) {
         using namespace ch4co2;
-        cx.i0 = 1.0 / sc.IR[0];
-        cx.i1 = 1.0 / sc.IR[1];
         const int l = min(cx.lane, 14), j = l / 5, i = l % 5;
         const P hs = P(kRCH / 1.7320508075688772);
 #pragma unroll
@@ -128,80 +177,76 @@ __device__ __forceinline__ RowCtx<SYS, P> row_ctx(const SysConst& sc, P* scratch
     return cx;
 }
 
+// sincos_p of an angle that both lanes of a pair hold: the even lane gets the sine, the odd lane the
+// cosine
+template <int SYS, typename P>
+__device__ __forceinline__ void row_sincos(const RowCtx<SYS, P>& cx, const Reduced& red, double& v)
+{
+    const bool odd = cx.lane & 1;
+    const double r2 = red.r * red.r;
+    double w = cx.w[6] + r2 * cx.w[7];
+#pragma unroll
+    for (int i = 5; i >= 0; --i) w = cx.w[i] + r2 * w;
+    const double base = odd ? 1.0 : red.r;   // sin: r + (r r2) w, cos: 1 + r2 w
+    v = base + base * r2 * w;
+    const double other = row_move<PAIR_SWAP>(v);
+    v = (red.q & 1) ? other : v;
+    rw_v2u u = __builtin_bit_cast(rw_v2u, v);
+    u.y ^= (unsigned)((red.q + (odd ? 1 : 0)) & 2) << 30;
+    v = __builtin_bit_cast(double, u);
+}
+
+template <int SYS, typename P>
+__device__ __forceinline__ void row_sincos(const RowCtx<SYS, P>& cx, const Reduced& red, float& v)
+{
+    const bool odd = cx.lane & 1;
+    const float r = (float)red.r, r2 = r * r;
+    float w = cx.wf[3] + r2 * cx.wf[4];
+#pragma unroll
+    for (int i = 2; i >= 0; --i) w = cx.wf[i] + r2 * w;
+    const float base = odd ? 1.0f : r;
+    v = base + base * r2 * w;
+    const float other = row_move<PAIR_SWAP>(v);
+    v = (red.q & 1) ? other : v;
+    v = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) ^ ((unsigned)((red.q + (odd ? 1 : 0)) & 2) << 30));
+}
+
 // ------------------------------------------------------------------ right-hand sides
 // The component of Hamilton's equations of the calling lane; y: the lane's component of the
-// state.  noise as in rhs().  Each branch follows rhs<SYS, P> expression by expression.
+// state.  noise as in rhs().  Coordinates sit in the even lanes, their momenta in the odd ones; each
+// branch follows rhs<SYS, P> expression by expression.
 template <int SYS, typename P>
 __device__ __forceinline__ double row_rhs(const SysConst& sc, const RowCtx<SYS, P>& cx, double y, double& noise)
 {
-    constexpr int N = SysTraits<SYS>::QP;
     noise = 0.0;
-    double yd[N];
-    double s, c;                      // every lane's own sine and cosine; the angles' lanes are read
-    sincos_p<double>(y, &s, &c);
-    P sP, cP;                         // and in the surfaces' precision
-    if constexpr (sizeof(P) == 8) {
-        sP = s;
-        cP = c;
-    } else {
-        sincos_p<P>(y, &sP, &cP);
+    const int lane = cx.lane;
+    const bool odd = lane & 1;
+    double ang = row_move<PAIR_EVEN>(y);              // the pair's coordinate in both lanes
+    const double p_next = row_move<PAIR_ODD>(y);      // and its momentum
+    if constexpr (SYS == SYS_CO2AR && sizeof(P) == 4) {
+        const double d = bcast<0>(y) - bcast<6>(y);   // Phi - phi1
+        ang = lane < 2 ? d : ang;
     }
+    const Reduced red = reduce_pio2(ang);
+    double t;                                         // even lane: sine, odd lane: cosine
+    row_sincos(cx, red, t);
+    P tp;                                             // and in the surfaces' precision
+    if constexpr (sizeof(P) == 8)
+        tp = t;
+    else
+        row_sincos(cx, red, tp);
     const double R = bcast<4>(y);
-    if constexpr (SYS == SYS_HEAR) {
-        const double x = kHearB * R;
-        const double arg = cx.lane == 0 ? -x : -kHearA1 * R - kHearA2 * R * R;
-        const double ex = exp(arg);
-        double dV[3];
-        dV[0] = 0.0;
-        dV[1] = 0.0;
-        dV[2] = hear_dV_exps(R, bcast<0>(ex), bcast<1>(ex));
-        const double r = recip<P>(cx.lane == 4 ? y : s);
-        pair_eom(bcast<1>(y), bcast<3>(y), bcast<5>(y), bcast<2>(c), cx.imu, bcast<4>(r), bcast<2>(r), dV, yd);
-    } else if constexpr (SYS == SYS_CO2AR) {
-        const Co2ArTables<P>* tb = (const Co2ArTables<P>*)sc.tables;
-        // the lane's radial slot: value and derivative
-        const int b = co2ar_branch(R);
-        const int slot = min(cx.lane, 5);
-        const double rc = recip<P>(cx.lane == 4 ? y : s);
-        const double iR = bcast<4>(rc);
-        P v, dv;
-        if (b == 0) {
-            const P r = (P)R;
-            const P e = tb->pes_exp[slot][0] * exp(tb->pes_exp[slot][1] * r);
-            v = e;
-            dv = tb->pes_exp[slot][1] * e;
-        } else {
-            const P x = (P)(R - tb->center[b]);
-            const P sinv = (P)iR;
-            slot_eval<P>(tb->pes[b][slot], x, sinv, v, dv);
-        }
-        const double sT = bcast<2>(s), cT = bcast<2>(c), st = bcast<8>(s), ct = bcast<8>(c);
-        const Co2ArAngles<P> g = co2ar_angles<P>(bcast<0>(sP), bcast<0>(cP), (P)sT, (P)cT, bcast<6>(sP), bcast<6>(cP),
-                                                 (P)st, (P)ct);
-        P Pl[11], dPl[11];
-        legendre10<P>(g.c, Pl, dPl);
-        P vs[6], dvs[6];
-        gather<P, 6>(v, vs);
-        gather<P, 6>(dv, dvs);
-        P dVdR = P(0), dVdc = P(0), mag = P(0);
-#pragma unroll
-        for (int q = 0; q < 6; ++q) {
-            const P tR = dvs[q] * Pl[2 * q], tc = vs[q] * dPl[2 * q];
-            dVdR += tR;
-            dVdc += tc;
-            if constexpr (sizeof(P) == 4) mag += fabs(tR) + fabs(tc);
-        }
-        noise = sizeof(P) == 4 ? kF32NoiseUnits * (double)mag : 0.0;
-        double dV[5];
-        co2ar_gradient<P>(g, dVdR, dVdc, dV);
-        pair_eom(bcast<1>(y), bcast<3>(y), bcast<5>(y), cT, cx.imu, iR, bcast<2>(rc), dV, yd);
-        linear_rotor_eom(bcast<7>(y), bcast<9>(y), ct, cx.iI, bcast<8>(rc), dV[3], dV[4], yd + 6);
-    } else {
+    // reciprocals of the sines and, in lane 4, of R; in both lanes of a pair
+    const double rc = row_move<PAIR_EVEN>(recip<P>(lane == 4 ? y : t));
+    const double iR = bcast<4>(rc), is = bcast<2>(rc);
+    const double is2 = is * is, a = sc.imu * (iR * iR);
+    const double rad = radial_rate(bcast<1>(y), bcast<3>(y), is2, a);
+    if constexpr (SYS == SYS_CH4CO2) {
         Ch4Co2Frame<P> f;
-        const double sT = bcast<2>(s), cT = bcast<2>(c), s1 = bcast<8>(s), c1 = bcast<8>(c);
-        const double sp = bcast<10>(s), cp = bcast<10>(c), s2 = bcast<14>(s), c2 = bcast<14>(c);
-        f.sP = bcast<0>(sP), f.cP = bcast<0>(cP), f.sf = bcast<6>(sP), f.cf = bcast<6>(cP);
-        f.sP2 = bcast<12>(sP), f.cP2 = bcast<12>(cP);
+        const double sT = bcast<2>(t), cT = bcast<3>(t), s1 = bcast<8>(t), c1 = bcast<9>(t);
+        const double sp = bcast<10>(t), cp = bcast<11>(t), s2 = bcast<14>(t), c2 = bcast<15>(t);
+        f.sP = bcast<0>(tp), f.cP = bcast<1>(tp), f.sf = bcast<6>(tp), f.cf = bcast<7>(tp);
+        f.sP2 = bcast<12>(tp), f.cP2 = bcast<13>(tp);
         f.sT = (P)sT, f.cT = (P)cT, f.s1 = (P)s1, f.c1 = (P)c1, f.sp = (P)sp, f.cp = (P)cp, f.s2 = (P)s2, f.c2 = (P)c2;
         ch4co2_axes<P>(f);
         const P Rp = (P)R;
@@ -214,18 +259,18 @@ __device__ __forceinline__ double row_rhs(const SysConst& sc, const RowCtx<SYS, 
                             Rp * f.a[2] + sgn * P(kRCO) * f.b[2]};
             const P d0 = X[0] - cx.h0, d1 = X[1] - cx.h1, d2 = X[2] - cx.h2;
             const P r2 = d0 * d0 + d1 * d1 + d2 * d2;
-            const P ir2 = P(1) / r2;
+            const P ir2 = recip_p(r2);
             const P sr2 = cx.s2 * ir2, sr6 = sr2 * sr2 * sr2, sr12 = sr6 * sr6;
             const P w = cx.e4 * (P(-12) * sr12 + P(6) * sr6) * ir2;   // (dV/dr) / r
             P* sm = cx.scratch;
-            sm[cx.lane] = w;
-            sm[16 + cx.lane] = d0;
-            sm[32 + cx.lane] = d1;
-            sm[48 + cx.lane] = d2;
-            if constexpr (sizeof(P) == 4) sm[64 + cx.lane] = fabs(d0) + fabs(d1) + fabs(d2);
+            sm[lane] = w;
+            sm[16 + lane] = d0;
+            sm[32 + lane] = d1;
+            sm[48 + lane] = d2;
+            if constexpr (sizeof(P) == 4) sm[64 + lane] = fabs(d0) + fabs(d1) + fabs(d2);
             wave_share_sync();
             // lane 3 j + k sums component k of CO2 site j over the five CH4 sites, in site order
-            const int jk = min(cx.lane, 8), j = jk / 3, k = jk - 3 * j;
+            const int jk = min(lane, 8), j = jk / 3, k = jk - 3 * j;
             P g = P(0);
 #pragma unroll
             for (int i = 0; i < 5; ++i) g += sm[5 * j + i] * sm[16 + 16 * k + 5 * j + i];
@@ -251,15 +296,96 @@ __device__ __forceinline__ double row_rhs(const SysConst& sc, const RowCtx<SYS, 
         double dV[8];
         ch4co2_gradient<P>(f, Rp, gs, gd, dV);
         noise = ch4co2_noise<P>(Rp, mag);
-        const double rc = recip<P>(cx.lane == 4 ? y : s);
-        // the rotor's 1/sin(theta1) is a division in both precisions
-        const double is1 = sizeof(P) == 8 ? bcast<8>(rc) : 1.0 / s1;
-        pair_eom(bcast<1>(y), bcast<3>(y), bcast<5>(y), cT, cx.imu, bcast<4>(rc), bcast<2>(rc), dV, yd);
+        double yd[16];
+        yd[4] = bcast<5>(y) * sc.imu;
+        yd[5] = rad * iR - dV[2];
+        yd[0] = bcast<1>(y) * a * is2;
+        yd[1] = -dV[0];
+        yd[2] = bcast<3>(y) * a;
+        yd[3] = polar_rate(bcast<1>(y), cT, a, is2, is, dV[1]);
         const double m[6] = {0.0, bcast<7>(y), 0.0, bcast<9>(y), 0.0, bcast<11>(y)};
-        rotor_rhs(sc.IR, m, dV + 3, s1, c1, sp, cp, is1, cx.i0, cx.i1, yd + 6);
-        linear_rotor_eom(bcast<13>(y), bcast<15>(y), c2, cx.iI, bcast<14>(rc), dV[6], dV[7], yd + 12);
+        // the rotor's 1/sin(theta1) is FP64 in both precisions
+        rotor_rhs(sc.IR, sc.iIR, m, dV + 3, s1, c1, sp, cp, sizeof(P) == 8 ? bcast<8>(rc) : recip<double>(s1), yd + 6);
+        linear_rotor_eom(bcast<13>(y), bcast<15>(y), c2, sc.iI, bcast<14>(rc), dV[6], dV[7], yd + 12);
+        return pick<16>(yd, cx.comp);
+    } else {
+        double dV;                                    // odd lanes: dV/dq of their coordinate
+        double irot2 = 1.0;                           // CO2-Ar: 1/sin^2(theta1)
+        if constexpr (SYS == SYS_HEAR) {
+            const double x = kHearB * R;
+            const double arg = lane == 0 ? -x : -kHearA1 * R - kHearA2 * R * R;
+            const double ex = exp(arg);
+            const double dVR = hear_dV_exps(R, bcast<0>(ex), bcast<1>(ex));
+            dV = lane == 5 ? dVR : 0.0;
+        } else {
+            const Co2ArTables<P>* tb = (const Co2ArTables<P>*)sc.tables;
+            // the lane's radial slot: value and derivative
+            const int b = co2ar_branch<P>(tb, R);
+            const int slot = min(lane & 7, 5);
+            P v, dv;
+            if (b == 0) {
+                const P r = (P)R;
+                const P e = tb->pes_exp[slot][0] * exp(tb->pes_exp[slot][1] * r);
+                v = e;
+                dv = tb->pes_exp[slot][1] * e;
+            } else {
+                const P x = (P)(R - tb->center[b]);
+                slot_eval<P>(tb->pes[b][slot], x, (P)iR, v, dv);
+            }
+            const double sT = bcast<2>(t), cT = bcast<3>(t), st = bcast<8>(t), ct = bcast<9>(t);
+            P dVdR, dVdc;
+            Co2ArAngles<P> g;
+            if constexpr (sizeof(P) == 8) {
+                g = co2ar_angles<P>(bcast<0>(tp), bcast<1>(tp), sT, cT, bcast<6>(tp), bcast<7>(tp), st, ct);
+                P Pl[11], dPl[11];
+                legendre10<P>(g.c, Pl, dPl);
+                P vs[6], dvs[6];
+                gather<P, 6>(v, vs);
+                gather<P, 6>(dv, dvs);
+                dVdR = dVdc = P(0);
+#pragma unroll
+                for (int q = 0; q < 6; ++q) {
+                    const P tR = dvs[q] * Pl[2 * q], tc = vs[q] * dPl[2 * q];
+                    dVdR += tR;
+                    dVdc += tc;
+                }
+            } else {
+                g = co2ar_angles_difference<P>(bcast<0>(tp), bcast<1>(tp), (P)sT, (P)cT, (P)st, (P)ct);
+                // the slot's Legendre polynomial and its derivative (lanes 6 and 7 of each half: 0)
+                const P z = g.c * g.c;
+                P p0 = P(0), p1 = (lane & 7) < 6 ? P(1) : P(0), d0 = P(0), d1 = P(0);
+#pragma unroll
+                for (int q = 0; q < 5; ++q) legendre_step<P>(cx.alpha[q], cx.beta[q], cx.gamma[q], z, p0, p1, d0, d1);
+                const P tR = dv * p1, tc = v * d1;
+                dVdR = row_slot_sum<P>(tR);
+                const P c2 = g.c + g.c, ac2 = fabs(c2);
+                dVdc = row_slot_sum<P>(tc) * c2;
+                noise = kF32NoiseUnits * (double)row_slot_sum<P>(fabs(tc) * ac2 + fabs(tR));
+            }
+            P gl = lane == 3 ? g.dTheta : g.dPhi;
+            gl = lane == 9 ? g.dtheta : gl;
+            gl = lane == 7 ? g.dphi : gl;
+            const double gq = (double)(dVdc * gl);
+            dV = lane == 5 ? (double)dVdR : gq;
+            const double ist = bcast<8>(rc);
+            irot2 = ist * ist;
+        }
+        // even lanes: p a is2, p a, p / mu, p iI ist2, p iI; a factor 1 leaves the product as it is
+        const double ka = lane < 4 ? a : cx.kin;
+        double kb = lane == 0 ? is2 : 1.0;
+        kb = lane == 6 ? irot2 : kb;
+        const double coord = p_next * ka * kb;
+        // odd lanes: lanes 3 and 9 polar_rate (azimuthal momentum two lanes down, own cosine), lane 5 the
+        // radial rate; lanes 1 and 7 (a cyclic and a surface-driven azimuth) -dV
+        const double pa = row_move<DOWN2>(y);
+        const double i2 = lane == 3 ? is2 : irot2;
+        const double pol = pa * pa * t * ka * i2;
+        double num = lane == 5 ? rad : pol;
+        num = (lane == 1 || lane == 7) ? 0.0 : num;
+        const double mul = lane == 5 ? iR : rc;
+        const double momentum = num * mul - dV;
+        return odd ? momentum : coord;
     }
-    return pick<N>(yd, cx.comp);
 }
 
 // ------------------------------------------------------------------ a row's trajectory
@@ -587,15 +713,9 @@ __device__ __forceinline__ void row_step(const SysConst& sc, const RowCtx<SYS, P
             const double floor_p = fabs(h) * noise;
             yn = it.y + h * be0;
             const double sk = it.atol + it.rtol * fmax(fabs(it.y), fabs(yn)) + ((cx.comp & 1) ? floor_p : 0.0);
-            double e5, e3;
-            if constexpr (sizeof(P) == 4) {
-                const double isk = rcp_nr(sk);
-                e5 = be1 * isk, e3 = be2 * isk;
-            } else {
-                e5 = be1 / sk, e3 = be2 / sk;
-            }
-            double err = sum_squares<N>(e5);
-            const double err2 = sum_squares<N>(e3);
+            const double isk = recip<P>(sk);
+            double err = sum_squares<N>(divide<P>(be1, sk, isk));
+            const double err2 = sum_squares<N>(divide<P>(be2, sk, isk));
             double deno = err + 0.01 * err2;
             if (deno <= 0.0) deno = 1.0;
             err = fabs(h) * err * sqrt(1.0 / (N * deno));

@@ -38,6 +38,7 @@ struct Co2ArTables {
     P dipx[32][5][8];    // P_l^1 slots l = 2..10
     P dipz[32][6][8];    // P_l slots l = 0..10
     double center[32];
+    int branch[122];     // branch of R in [k/4, (k + 1)/4), k <= 120 (every bound is a multiple of 1/4)
 };
 
 struct SysConst {
@@ -45,7 +46,53 @@ struct SysConst {
     double I;            // linear-rotor moment of inertia (II[0] == II[1]); CH4-CO2: of CO2
     const void* tables;  // Co2ArTables<P>* for CO2-Ar
     double IR[3];        // CH4-CO2: principal moments of the rotor (CH4)
+    double imu, iI;      // 1/mu, 1/I
+    double iIR[3];       // 1/IR
 };
+
+// 1/x within an ulp: the hardware reciprocal estimate refined by two Newton steps (each at
+// least doubles the correct bits).  The engines with FP32 surfaces (P = float) use it.
+__device__ __forceinline__ double rcp_nr(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    double e = fma(-x, r, 1.0);
+    r = fma(r, e, r);
+    e = fma(-x, r, 1.0);
+    return fma(r, e, r);
+}
+
+// The FP64 engines' 1/x: one more residual step rounds to the division's value (the same bits for the
+// well-scaled arguments here: distances, sines, error scales) in 7 instructions instead of the scaled
+// division's 11.
+template <typename P>
+__device__ __forceinline__ double recip(double x)
+{
+    const double r = rcp_nr(x);
+    if constexpr (sizeof(P) == 4)
+        return r;
+    else
+        return fma(fma(-x, r, 1.0), r, r);
+}
+
+// a / b by b's reciprocal r: the division's bits in FP64 (a residual step), a product in the engines
+// with FP32 surfaces
+template <typename P>
+__device__ __forceinline__ double divide(double a, double b, double r)
+{
+    const double q = a * r;
+    if constexpr (sizeof(P) == 4)
+        return q;
+    else
+        return fma(fma(-b, q, a), r, q);
+}
+
+// 1/x in the surfaces' precision
+__device__ __forceinline__ double recip_p(double x) { return recip<double>(x); }
+__device__ __forceinline__ float recip_p(float x)
+{
+    const float r = __builtin_amdgcn_rcpf(x);
+    return fmaf(fmaf(-x, r, 1.0f), r, r);
+}
 
 // ------------------------------------------------------------------ He-Ar (PES-IDS/HeAr.h)
 // Tang-Toennies form V = A exp(-a1 R - a2 R^2) - sum_{n=3}^{8} C_2n f_2n(R)/R^2n with
@@ -59,7 +106,7 @@ __device__ __forceinline__ double hear_dV_exps(double R, double e, double ea)
     const double A = kHearA, a1 = kHearA1, a2 = kHearA2, b = kHearB;
     const double C[6] = {0.940835513e1, 0.165523018e3, 0.379715796e4, 0.1165179999e6, 0.466258000e7,
                          0.236861000e9};
-    const double x = b * R, inv = 1.0 / R, inv2 = inv * inv;
+    const double x = b * R, inv = recip<double>(R), inv2 = inv * inv;
     double term = 1.0, sum = 1.0;
     double dV = A * ea * (-a1 - 2.0 * a2 * R);
     double ip = inv2 * inv2;  // R^-4
@@ -114,38 +161,13 @@ __device__ __forceinline__ P hear_dip(P R)
     return exp(P(0.47293181) - P(0.40100613) * R - P(0.10292726) * r2) - P(148.55391) * inv7;
 }
 
-// 1/x within an ulp: the hardware reciprocal estimate refined by two Newton steps (each at
-// least doubles the correct bits).  The engines with FP32 surfaces (P = float) use it in place
-// of the correctly rounded FP64 division, which costs twice the instructions and a longer
-// dependent chain; the FP64 engines divide.
-__device__ __forceinline__ double rcp_nr(double x)
-{
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-x, r, 1.0);
-    return fma(r, e, r);
-}
-
-template <typename P>
-__device__ __forceinline__ double recip(double x)
-{
-    if constexpr (sizeof(P) == 4)
-        return rcp_nr(x);
-    else
-        return 1.0 / x;
-}
-
 // ------------------------------------------------------------------ CO2-Ar
-__device__ __forceinline__ int co2ar_branch(double R)
+// breakpoints 4.5, 4.75, ..., 10 (step 1/4), then 11, 12, 14, 16, 18, 20, 25, 30: a lookup at 4 R
+// (R * 4 is exact)
+template <typename P>
+__device__ __forceinline__ int co2ar_branch(const Co2ArTables<P>* __restrict__ tb, double R)
 {
-    // breakpoints 4.5, 4.75, ..., 10 (step 1/4), then 11, 12, 14, 16, 18, 20, 25, 30
-    if (R < 4.5) return 0;
-    if (R < 10.0) return 1 + (int)((R - 4.5) * 4.0);   // exact: R - 4.5 and *4 are exact here
-    int b = 23;
-    b += (R >= 11.0) + (R >= 12.0) + (R >= 14.0) + (R >= 16.0) + (R >= 18.0) + (R >= 20.0) + (R >= 25.0) +
-         (R >= 30.0);
-    return b;
+    return tb->branch[(int)fmin(fmax(R * 4.0, 0.0), 120.0)];
 }
 
 // sin and cos for the bounded angles of a trajectory (|x| < 1.6e6 rad).  Cody-Waite
@@ -168,9 +190,8 @@ __device__ __forceinline__ Reduced reduce_pio2(double x)
 }
 
 template <typename P>
-__device__ __forceinline__ void sincos_p(double x, P* s, P* c)
+__device__ __forceinline__ void sincos_reduced(const Reduced& red, P* s, P* c)
 {
-    const Reduced red = reduce_pio2(x);
     P sr, cr;
     if constexpr (sizeof(P) == 8) {
         const double r = red.r, r2 = r * r;
@@ -189,6 +210,12 @@ __device__ __forceinline__ void sincos_p(double x, P* s, P* c)
     *c = (red.q == 1 || red.q == 2) ? -c0 : c0;
 }
 
+template <typename P>
+__device__ __forceinline__ void sincos_p(double x, P* s, P* c)
+{
+    sincos_reduced<P>(reduce_pio2(x), s, c);
+}
+
 // Legendre P_l(c), P_l'(c), l = 0..10 (three-term recurrences, P'_{l+1} = P'_{l-1} + (2l+1) P_l)
 template <typename P>
 __device__ __forceinline__ void legendre10(P c, P* Pl, P* dPl)
@@ -204,14 +231,89 @@ __device__ __forceinline__ void legendre10(P c, P* Pl, P* dPl)
     }
 }
 
+// FP32 surfaces: even Legendre polynomials as functions of z = c^2, half the steps of legendre10: p_{l+2} = (alpha z - beta) p_l - gamma p_{l-2},
+// from x^2 P_l = A P_{l+2} + B P_l + C P_{l-2}, A = (l+1)(l+2) / ((2l+1)(2l+3)),
+// B = (2l^2+2l-1) / ((2l-1)(2l+3)), C = l(l-1) / ((2l-1)(2l+1)).
+struct LegendreEven {
+    double alpha, beta, gamma;
+};
+constexpr LegendreEven legendre_even_step(int t)   // l = 2t
+{
+    const double l = 2.0 * t, A = (l + 1) * (l + 2) / ((2 * l + 1) * (2 * l + 3));
+    const double B = (2 * l * l + 2 * l - 1) / ((2 * l - 1) * (2 * l + 3)), C = l * (l - 1) / ((2 * l - 1) * (2 * l + 1));
+    return {1.0 / A, B / A, C / A};
+}
+
+// one step of the recurrence and of its derivative in z
+template <typename P>
+__device__ __forceinline__ void legendre_step(P alpha, P beta, P gamma, P z, P& p0, P& p1, P& d0, P& d1)
+{
+    const P a = alpha * z - beta;
+    const P gp = gamma * p0, gd = gamma * d0 - alpha * p1;
+    p0 = p1;
+    d0 = d1;
+    p1 = a * p1 - gp;
+    d1 = a * d1 - gd;
+}
+
+// p[s] = P_{2s}(c), d[s] = dp/dz at z = c^2 (P_l'(c) = 2 c dp/dz), s = 0..5
+template <typename P>
+__device__ __forceinline__ void legendre_even(P z, P (&p)[6], P (&d)[6])
+{
+    P p0 = P(0), p1 = P(1), d0 = P(0), d1 = P(0);
+    p[0] = P(1);
+    d[0] = P(0);
+#pragma unroll
+    for (int t = 0; t < 5; ++t) {
+        const LegendreEven k = legendre_even_step(t);
+        legendre_step<P>(P(k.alpha), P(k.beta), P(k.gamma), z, p0, p1, d0, d1);
+        p[t + 1] = p1;
+        d[t + 1] = d1;
+    }
+}
+
+// the sum of six slots' terms, in the order in which a row of lanes adds them
+template <typename P>
+__device__ __forceinline__ P slot_sum(const P (&t)[6])
+{
+    const P a = t[0] + t[1], b = t[2] + t[3], c = t[4] + t[5];
+    const P ab = a + b;
+    return ab + c;
+}
+
 // radial slot value and derivative: centred cubic in x plus R^-4..R^-7 in s = 1/R
 template <typename P>
-__device__ __forceinline__ void slot_eval(const P* c, P x, P s, P& v, P& dv)
+__device__ __forceinline__ void slot_eval_terms(const P* c, P x, P s, P& v, P& dv)
 {
     const P s2 = s * s, s4 = s2 * s2;
     v = ((c[3] * x + c[2]) * x + c[1]) * x + c[0] + s4 * (((c[7] * s + c[6]) * s + c[5]) * s + c[4]);
     dv = (P(3) * c[3] * x + P(2) * c[2]) * x + c[1] -
          s4 * s * (((P(7) * c[7] * s + P(6) * c[6]) * s + P(5) * c[5]) * s + P(4) * c[4]);
+}
+
+// The same; FP32 surfaces take each polynomial by Horner's rule with its derivative (fewer
+// operations and no constants to load)
+template <typename P>
+__device__ __forceinline__ void slot_eval(const P* c, P x, P s, P& v, P& dv)
+{
+    if constexpr (sizeof(P) == 8) {
+        slot_eval_terms<P>(c, x, s, v, dv);
+        return;
+    }
+    P f = c[3] * x + c[2], df = c[3];
+    df = df * x + f;
+    f = f * x + c[1];
+    df = df * x + f;
+    f = f * x + c[0];
+    P g = c[7] * s + c[6], dg = c[7];
+    dg = dg * s + g;
+    g = g * s + c[5];
+    dg = dg * s + g;
+    g = g * s + c[4];
+    const P s2 = s * s, s4 = s2 * s2;
+    const P u = s * dg + P(4) * g;   // d(s^4 g)/dR = -s^5 (4 g + s g')
+    v = s4 * g + f;
+    dv = df - s4 * s * u;
 }
 
 template <typename P>
@@ -236,6 +338,8 @@ struct Co2ArAngles {
     P c, dPhi, dTheta, dphi, dtheta;
 };
 
+// FP64: from the unit vectors.  An orbiting pair's trajectory depends on the last bit of the FP64
+// surfaces, so this form and the order of the sums after it stay as they are.
 template <typename P>
 __device__ __forceinline__ Co2ArAngles<P> co2ar_angles(P sP, P cP, P sT, P cT, P sp, P cp, P st, P ct)
 {
@@ -249,6 +353,24 @@ __device__ __forceinline__ Co2ArAngles<P> co2ar_angles(P sP, P cP, P sT, P cT, P
     g.dTheta = cT * cP * ux + cT * sP * uy - sT * uz;  // dRhat/dTheta . u
     g.dphi = -Rx * uy + Ry * ux;                       // Rhat . du/dphi
     g.dtheta = ct * cp * Rx + ct * sp * Ry - st * Rz;  // Rhat . du/dtheta
+    return g;
+}
+
+// FP32: the surface depends on Phi and phi1 only through their difference (sD, cD its sine and
+// cosine), so dc/dphi1 = -dc/dPhi; three sincos instead of four and half the products.  With the even
+// Legendre recurrence and slot_eval's Horner form, a batch of 6 x 65536 mixed trajectories went from
+// 300 to 257 ms; rows against the FP64 engine's: median 2.74e-7 -> 2.68e-7, 99 % 1.57e-6 -> 1.55e-6.
+template <typename P>
+__device__ __forceinline__ Co2ArAngles<P> co2ar_angles_difference(P sD, P cD, P sT, P cT, P st, P ct)
+{
+    Co2ArAngles<P> g;
+    const P stC = st * cD, sTC = sT * cD, ss = sT * st;
+    const P c = sT * stC + cT * ct;
+    g.c = c > P(1) ? P(1) : (c < P(-1) ? P(-1) : c);
+    g.dPhi = -(ss * sD);
+    g.dphi = -g.dPhi;
+    g.dTheta = cT * stC - sT * ct;
+    g.dtheta = ct * sTC - cT * st;
     return g;
 }
 
@@ -269,7 +391,7 @@ __device__ __forceinline__ void co2ar_dpes(const Co2ArTables<P>* __restrict__ tb
                                            const Trig& tr, double* dV, double& noise)
 {
     const double R = y[4];
-    const int b = co2ar_branch(R);
+    const int b = co2ar_branch<P>(tb, R);
     // FP32: the radial coefficients of the point's branch are read from LDS first, so their
     // latency overlaps the angular part (one wait instead of one per slot)
     P cf[6][8];
@@ -283,42 +405,70 @@ __device__ __forceinline__ void co2ar_dpes(const Co2ArTables<P>* __restrict__ tb
         cen = tb->center[bb];
         __builtin_amdgcn_sched_barrier(0);
     }
-    P sP, cP, sp, cp;
-    sincos_p<P>(y[0], &sP, &cP);
-    sincos_p<P>(y[6], &sp, &cp);
-    const Co2ArAngles<P> g = co2ar_angles<P>(sP, cP, (P)tr.sT, (P)tr.cT, sp, cp, (P)tr.st, (P)tr.ct);
-    const P c = g.c;
-
-    P Pl[11], dPl[11];
-    legendre10<P>(c, Pl, dPl);
-
-    P dVdR = P(0), dVdc = P(0);
-    P mag = P(0);   // sum of |terms| (FP32 only)
-    if (b == 0) {
-        const P r = (P)R;
+    if constexpr (sizeof(P) == 8) {
+        P sP, cP, sp, cp;
+        sincos_p<P>(y[0], &sP, &cP);
+        sincos_p<P>(y[6], &sp, &cp);
+        const Co2ArAngles<P> g = co2ar_angles<P>(sP, cP, tr.sT, tr.cT, sp, cp, tr.st, tr.ct);
+        P Pl[11], dPl[11];
+        legendre10<P>(g.c, Pl, dPl);
+        P dVdR = P(0), dVdc = P(0);
+        if (b == 0) {
 #pragma unroll
-        for (int s = 0; s < 6; ++s) {
-            const P e = tb->pes_exp[s][0] * exp(tb->pes_exp[s][1] * r);
-            const P tR = tb->pes_exp[s][1] * e * Pl[2 * s], tc = e * dPl[2 * s];
-            dVdR += tR;
-            dVdc += tc;
-            if constexpr (sizeof(P) == 4) mag += fabs(tR) + fabs(tc);
+            for (int s = 0; s < 6; ++s) {
+                const P e = tb->pes_exp[s][0] * exp(tb->pes_exp[s][1] * R);
+                const P tR = tb->pes_exp[s][1] * e * Pl[2 * s], tc = e * dPl[2 * s];
+                dVdR += tR;
+                dVdc += tc;
+            }
+        } else {
+            const P x = R - tb->center[b];
+            const P sinv = recip<P>(R);
+#pragma unroll
+            for (int s = 0; s < 6; ++s) {
+                P v, dv;
+                slot_eval<P>(tb->pes[b][s], x, sinv, v, dv);
+                const P tR = dv * Pl[2 * s], tc = v * dPl[2 * s];
+                dVdR += tR;
+                dVdc += tc;
+            }
         }
+        noise = 0.0;
+        co2ar_gradient<P>(g, dVdR, dVdc, dV);
     } else {
-        const P x = (P)(R - (sizeof(P) == 4 ? cen : tb->center[b]));
-        const P sinv = (P)recip<P>(R);
+        P sD, cD;
+        sincos_p<P>(y[0] - y[6], &sD, &cD);
+        const Co2ArAngles<P> g = co2ar_angles_difference<P>(sD, cD, (P)tr.sT, (P)tr.cT, (P)tr.st, (P)tr.ct);
+        P Pl[6], dPl[6];
+        legendre_even<P>(g.c * g.c, Pl, dPl);
+        P tR[6], tc[6];
+        if (b == 0) {
+            const P r = (P)R;
 #pragma unroll
-        for (int s = 0; s < 6; ++s) {
-            P v, dv;
-            slot_eval<P>(sizeof(P) == 4 ? cf[s] : tb->pes[b][s], x, sinv, v, dv);
-            const P tR = dv * Pl[2 * s], tc = v * dPl[2 * s];
-            dVdR += tR;
-            dVdc += tc;
-            if constexpr (sizeof(P) == 4) mag += fabs(tR) + fabs(tc);
+            for (int s = 0; s < 6; ++s) {
+                const P e = tb->pes_exp[s][0] * exp(tb->pes_exp[s][1] * r);
+                tR[s] = tb->pes_exp[s][1] * e * Pl[s];
+                tc[s] = e * dPl[s];
+            }
+        } else {
+            const P x = (P)(R - cen);
+            const P sinv = (P)recip<P>(R);
+#pragma unroll
+            for (int s = 0; s < 6; ++s) {
+                P v, dv;
+                slot_eval<P>(cf[s], x, sinv, v, dv);
+                tR[s] = dv * Pl[s];
+                tc[s] = v * dPl[s];
+            }
         }
+        const P dVdR = slot_sum<P>(tR), dVdz = slot_sum<P>(tc);
+        const P c2 = g.c + g.c, ac2 = fabs(c2);
+        P mag[6];   // |terms|
+#pragma unroll
+        for (int s = 0; s < 6; ++s) mag[s] = fabs(tc[s]) * ac2 + fabs(tR[s]);
+        noise = kF32NoiseUnits * (double)slot_sum<P>(mag);
+        co2ar_gradient<P>(g, dVdR, dVdz * c2, dV);
     }
-    noise = sizeof(P) == 4 ? kF32NoiseUnits * (double)mag : 0.0;
-    co2ar_gradient<P>(g, dVdR, dVdc, dV);
 }
 
 template <typename P>
@@ -336,7 +486,7 @@ __device__ __forceinline__ P co2ar_pes(const Co2ArTables<P>* __restrict__ tb, co
     P Pl[11], dPl[11];
     legendre10<P>(c, Pl, dPl);
     const double R = y[4];
-    const int b = co2ar_branch(R);
+    const int b = co2ar_branch<P>(tb, R);
     P V = P(0);
     if (b == 0) {
 #pragma unroll
@@ -355,7 +505,7 @@ template <typename P>
 __device__ __forceinline__ void co2ar_dipole(const Co2ArTables<P>* __restrict__ tb, const double* y, P* mu)
 {
     const double R = y[4];
-    const int b = co2ar_branch(R);
+    const int b = co2ar_branch<P>(tb, R);
     // FP32: the branch's radial coefficients are read from LDS before the angular part (as in
     // co2ar_dpes)
     P cx[5][8], cz[6][8];
@@ -381,15 +531,26 @@ __device__ __forceinline__ void co2ar_dipole(const Co2ArTables<P>* __restrict__ 
     const P ux = st * cp, uy = st * sp, uz = ct;
     P c = Rx * ux + Ry * uy + Rz * uz;
     c = c > P(1) ? P(1) : (c < P(-1) ? P(-1) : c);
-    P Pl[11], dPl[11];
-    legendre10<P>(c, Pl, dPl);
+    P Pl[6], dPl[6];   // P_2s and P'_2s
+    if constexpr (sizeof(P) == 8) {
+        P all[11], dall[11];
+        legendre10<P>(c, all, dall);
+#pragma unroll
+        for (int s = 0; s < 6; ++s) {
+            Pl[s] = all[2 * s];
+            dPl[s] = dall[2 * s];
+        }
+    } else {
+        legendre_even<P>(c * c, Pl, dPl);   // d/dz: times 2 c below
+    }
     const P x = (P)(R - (sizeof(P) == 4 ? cen : tb->center[b]));
     const P sinv = (P)recip<P>(R);
     P gx = P(0), dz = P(0);
 #pragma unroll
-    for (int s = 0; s < 5; ++s) gx += slot_value<P>(sizeof(P) == 4 ? cx[s] : tb->dipx[b][s], x, sinv) * dPl[2 * s + 2];
+    for (int s = 0; s < 5; ++s) gx += slot_value<P>(sizeof(P) == 4 ? cx[s] : tb->dipx[b][s], x, sinv) * dPl[s + 1];
 #pragma unroll
-    for (int s = 0; s < 6; ++s) dz += slot_value<P>(sizeof(P) == 4 ? cz[s] : tb->dipz[b][s], x, sinv) * Pl[2 * s];
+    for (int s = 0; s < 6; ++s) dz += slot_value<P>(sizeof(P) == 4 ? cz[s] : tb->dipz[b][s], x, sinv) * Pl[s];
+    if constexpr (sizeof(P) == 4) gx *= c + c;
     // mu = dz Rhat - gx (u - c Rhat)
     mu[0] = dz * Rx - gx * (ux - c * Rx);
     mu[1] = dz * Ry - gx * (uy - c * Ry);
@@ -483,7 +644,7 @@ __device__ __forceinline__ P ch4co2_sites(P R, const P* a, const P* b, P* gs, P*
             const P h2 = i == 0 ? P(0) : hs * P(kH[i - 1][2]);
             const P d0 = X[0] - h0, d1 = X[1] - h1, d2 = X[2] - h2;
             const P r2 = d0 * d0 + d1 * d1 + d2 * d2;
-            const P ir2 = P(1) / r2;
+            const P ir2 = recip_p(r2);
             const P sr2 = s2 * ir2, sr6 = sr2 * sr2 * sr2, sr12 = sr6 * sr6;
             V += e4 * (sr12 - sr6);
             const P w = e4 * (P(-12) * sr12 + P(6) * sr6) * ir2;   // (dV/dr) / r
@@ -606,6 +767,18 @@ struct SysTraits<SYS_CH4CO2> {
     static constexpr int QP = 16;
 };
 
+// d(p_theta)/dt of a polar angle with azimuthal momentum p: k p^2 cos / sin^3 - dV, is = 1/sin
+__device__ __forceinline__ double polar_rate(double p, double c, double k, double is2, double is, double dV)
+{
+    return p * p * c * k * is2 * is - dV;
+}
+
+// d(p_R)/dt + dV/dR, without the factor 1/R; a = 1/(mu R^2)
+__device__ __forceinline__ double radial_rate(double pPhi, double pTheta, double is2, double a)
+{
+    return (pTheta * pTheta + pPhi * pPhi * is2) * a;
+}
+
 // intermolecular part of Hamilton's equations (src/hawaii.c:586-591): iR = 1/R, is = 1/sin(Theta),
 // dV = dV/d(Phi, Theta, R)
 __device__ __forceinline__ void pair_eom(double pPhi, double pTheta, double pR, double cT, double imu, double iR,
@@ -615,11 +788,11 @@ __device__ __forceinline__ void pair_eom(double pPhi, double pTheta, double pR, 
     const double is2 = is * is;
     const double a = imu * iR2;               // 1/(mu R^2)
     yd[4] = pR * imu;
-    yd[5] = (pTheta * pTheta + pPhi * pPhi * is2) * a * iR - dV[2];
+    yd[5] = radial_rate(pPhi, pTheta, is2, a) * iR - dV[2];
     yd[0] = pPhi * a * is2;
     yd[1] = -dV[0];
     yd[2] = pTheta * a;
-    yd[3] = pPhi * pPhi * cT * a * is2 * is - dV[1];
+    yd[3] = polar_rate(pPhi, cT, a, is2, is, dV[1]);
 }
 
 // linear rotor (src/hawaii.c:494-497): ist = 1/sin(theta), dVp = dV/dphi, dVt = dV/dtheta
@@ -630,26 +803,25 @@ __device__ __forceinline__ void linear_rotor_eom(double pphi, double ptheta, dou
     yd[0] = pphi * iI * ist2;
     yd[1] = -dVp;
     yd[2] = ptheta * iI;
-    yd[3] = pphi * pphi * ct * iI * ist2 * ist - dVt;
+    yd[3] = polar_rate(pphi, ct, iI, ist2, ist, dVt);
 }
 
 // rhsMonomer ROTOR (src/hawaii.c:505-531): monomer state m = (phi, pphi, theta, ptheta, psi, ppsi),
-// dV = dV/d(phi, theta, psi), sin/cos of theta and psi given; is = 1/sin(theta), i0 = 1/II[0],
-// i1 = 1/II[1]
-__device__ __forceinline__ void rotor_rhs(const double* II, const double* m, const double* dV, double st, double ct,
-                                          double sp, double cp, double is, double i0, double i1, double* d)
+// dV = dV/d(phi, theta, psi), sin/cos of theta and psi given; is = 1/sin(theta), iII = 1/II
+__device__ __forceinline__ void rotor_rhs(const double* II, const double* iII, const double* m, const double* dV,
+                                          double st, double ct, double sp, double cp, double is, double* d)
 {
     const double pPhi = m[1], pTheta = m[3], pPsi = m[5];
     const double t1 = (pPhi - pPsi * ct) * sp + pTheta * st * cp;
     const double t2 = (pPhi - pPsi * ct) * cp - pTheta * st * sp;
     const double t3 = pPhi * ct - pPsi, t4 = pPsi * ct - pPhi;
-    const double is2 = is * is;
+    const double is2 = is * is, i0 = iII[0], i1 = iII[1];
     d[0] = (t1 * sp * i0 + t2 * cp * i1) * is2;
     d[1] = -dV[0];
     d[2] = (t1 * cp * i0 - t2 * sp * i1) * is;
     d[3] = -t3 * (t4 * (II[0] - II[1]) * cp * cp + pTheta * (II[0] - II[1]) * st * sp * cp + t4 * II[1]) * i0 * i1 *
                is2 * is - dV[1];
-    d[4] = -(t1 * sp * i0 + t2 * cp * i1) * ct * is2 + pPsi / II[2];
+    d[4] = -(t1 * sp * i0 + t2 * cp * i1) * ct * is2 + divide<double>(pPsi, II[2], iII[2]);
     d[5] = t1 * t2 * (i1 - i0) * is2 - dV[2];
 }
 
@@ -661,7 +833,7 @@ __device__ __forceinline__ void rhs(const SysConst& sc, const double* __restrict
                                     double& noise)
 {
     noise = 0.0;
-    const double pPhi = y[1], Theta = y[2], pTheta = y[3], R = y[4], pR = y[5], mu = sc.mu;
+    const double pPhi = y[1], Theta = y[2], pTheta = y[3], R = y[4], pR = y[5];
     if constexpr (SYS == SYS_CH4CO2) {
         Ch4Co2Trig ct;
         sincos_p<double>(Theta, &ct.sT, &ct.cT);
@@ -670,9 +842,9 @@ __device__ __forceinline__ void rhs(const SysConst& sc, const double* __restrict
         sincos_p<double>(y[14], &ct.s2, &ct.c2);
         double dV[8];
         ch4co2_dpes<P>(y, ct, dV, noise);
-        pair_eom(pPhi, pTheta, pR, ct.cT, 1.0 / mu, recip<P>(R), recip<P>(ct.sT), dV, yd);
-        rotor_rhs(sc.IR, y + 6, dV + 3, ct.s1, ct.c1, ct.sp, ct.cp, 1.0 / ct.s1, 1.0 / sc.IR[0], 1.0 / sc.IR[1], yd + 6);
-        linear_rotor_eom(y[13], y[15], ct.c2, 1.0 / sc.I, recip<P>(ct.s2), dV[6], dV[7], yd + 12);
+        pair_eom(pPhi, pTheta, pR, ct.cT, sc.imu, recip<P>(R), recip<P>(ct.sT), dV, yd);
+        rotor_rhs(sc.IR, sc.iIR, y + 6, dV + 3, ct.s1, ct.c1, ct.sp, ct.cp, recip<double>(ct.s1), yd + 6);
+        linear_rotor_eom(y[13], y[15], ct.c2, sc.iI, recip<P>(ct.s2), dV[6], dV[7], yd + 12);
         return;
     }
     Trig tr;
@@ -686,9 +858,9 @@ __device__ __forceinline__ void rhs(const SysConst& sc, const double* __restrict
         sincos_p<double>(y[8], &tr.st, &tr.ct);
         co2ar_dpes<P>((const Co2ArTables<P>*)sc.tables, y, tr, dV, noise);
     }
-    pair_eom(pPhi, pTheta, pR, tr.cT, 1.0 / mu, recip<P>(R), recip<P>(tr.sT), dV, yd);
+    pair_eom(pPhi, pTheta, pR, tr.cT, sc.imu, recip<P>(R), recip<P>(tr.sT), dV, yd);
     if constexpr (SYS == SYS_CO2AR)
-        linear_rotor_eom(y[7], y[9], tr.ct, 1.0 / sc.I, recip<P>(tr.st), dV[3], dV[4], yd + 6);
+        linear_rotor_eom(y[7], y[9], tr.ct, sc.iI, recip<P>(tr.st), dV[3], dV[4], yd + 6);
 }
 
 template <int SYS, typename P>

@@ -270,7 +270,7 @@ extern "C" int hh_vegas(hh_engine* e, const hh_system* sys, const hh_vegas_param
     std::vector<double> grid((size_t)D * (kVegasBins + 1));
     for (int d = 0; d < D; ++d)
         for (int i = 0; i <= kVegasBins; ++i) grid[(size_t)d * (kVegasBins + 1) + i] = (double)i / kVegasBins;
-    SysConst sc{sys->mu, sys->I, e->tab64.p};
+    const SysConst sc = sysconst(e, *sys, false);
     VegasParams p{vp->T, vp->Rmin, vp->Rmax, vp->pair_state, vp->integrand, D, 0, vp->seed, vp->npoints};
     std::vector<double> host(3 + width_bins);
     double wsum = 0.0, wisum = 0.0, chi_a = 0.0;   // sums of weights, weighted values, weighted squares
