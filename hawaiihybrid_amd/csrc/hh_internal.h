@@ -156,8 +156,8 @@ struct LanePool {
     int cur = 0;
     // next: the queue head, then the number of items finished since the pool exists
     DevBuf arena, ring, ring_done, ring_orbit, ring_orbit_nrhs, next, scratch, sort_tmp;
-    // every pool's slices run on its own stream (default priority), so the slices of different
-    // pools (an FP64 orbit pool beside its mixed pool, classes of a serving mix) overlap
+    // of the present slice (not owned): the slices of different pools (an FP64 orbit pool beside its
+    // mixed pool, classes of a serving mix) overlap
     hipStream_t stream = nullptr;
     hipEvent_t slice_end = nullptr;
     double launch_ms = 0.0;         // summed durations of this pool's slice launches
@@ -187,15 +187,12 @@ struct LanePool {
     LanePool& operator=(const LanePool&) = delete;
     ~LanePool()
     {
+        if (slice_end) (void)hipEventSynchronize(slice_end);
         for (auto& g : graphs)
             if (g.exec) (void)hipGraphExecDestroy(g.exec);
         if (h_done) (void)hipHostFree(h_done);
         if (h_orbit) (void)hipHostFree(h_orbit);
         if (h_next) (void)hipHostFree(h_next);
-        if (stream) {
-            (void)hipStreamSynchronize(stream);
-            (void)hipStreamDestroy(stream);
-        }
         if (slice_end) (void)hipEventDestroy(slice_end);
     }
 };
@@ -207,6 +204,7 @@ struct hh_session;
 struct hh_engine {
     int device = 0;
     hipStream_t stream = nullptr;
+    hipStream_t pool_streams[3] = {nullptr, nullptr, nullptr};   // default priority; created on first use
     hipStream_t capture = nullptr;      // non-blocking stream used only to capture slice graphs
     bool use_graphs = false;            // HH_GRAPHS=1: slices as captured graphs (opt-in: see hh_pool.cpp)
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};

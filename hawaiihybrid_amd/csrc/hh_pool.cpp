@@ -54,7 +54,6 @@ int pool_get(hh_engine* e, PoolSet& set, const hh_system& sys, bool mixed, LaneP
         pl->scratch.ensure((size_t)(pl->S / 256 + 1) * sizeof(int)) != hipSuccess)
         return fail(HH_E_NOMEM, "cannot allocate a lane pool (%.1f MiB of slots and arena)",
                     (2.0 * sb + arena) / 1048576.0);
-    HH_CHECK(hipStreamCreateWithFlags(&pl->stream, hipStreamNonBlocking));
     HH_CHECK(hipEventCreate(&pl->slice_end));
     HH_CHECK(run_slots_clear(pl->view(0), e->stream));
     const unsigned long long z[2] = {0, 0};
@@ -299,22 +298,32 @@ SysConst pool_sysconst(const hh_engine* e, const LanePool& pl) { return sysconst
 // 0, 1024, 2048, 4096 and 8192 items, 1153 CO2-Ar trajectories in FP64 take 45.3, 24.1, 23.3, 22.9 and
 // 21.7 ms, 65536 mixed ones (their tail) 282, 185, 182, 184 and 170 ms, 12289 CH4-CO2 ones 356, 266,
 // 238, 225 and 208 ms, 4096 He-Ar ones 7.7, 6.0, 5.5, 4.2 and 4.3 ms.
+//
+// A mixed pool whose orbiting items go to an FP64 pool takes half of that, one wavefront per SIMD: two
+// fill the register file, and the FP64 pool's rows, which hold the longest trajectories, would wait for
+// them (65536 mixed CO2-Ar trajectories: 106 -> 95 ms).
 constexpr long long kRowLimit = 8192;
 
-long long row_limit(const LanePool& pl) { return std::min(kRowLimit, pl.S / 8); }
+bool hands_over(const LanePool& pl) { return pl.mixed && pl.sys != HH_SYS_HEAR; }
 
-// The grid for `left` items: one row per wavefront while they fit one wavefront, then two, per SIMD (a
-// lone row has no neighbours to diverge from), then two wavefronts per SIMD of two to four rows.
+long long row_limit(const LanePool& pl)
+{
+    const long long lim = std::min(kRowLimit, pl.S / 8);
+    return hands_over(pl) ? lim / 2 : lim;
+}
+
+// The grid for `left` items: one row per wavefront while they fit one wavefront then two per SIMD (a
+// lone row has no neighbours to diverge from), then two to four rows.
 struct RowPlan {
     int wgs, rows_used;
 };
 
-RowPlan row_plan(const hh_engine* e, long long left)
+RowPlan row_plan(const hh_engine* e, const LanePool& pl, long long left)
 {
-    const long long cus = e->prop.multiProcessorCount;   // a workgroup: one wavefront per SIMD
-    if (left <= 4 * cus) return {(int)cus, 1};
-    const long long waves = 8 * cus;
-    return {(int)(2 * cus), (int)std::min<long long>(4, (left + waves - 1) / waves)};
+    const int cus = e->prop.multiProcessorCount;   // a workgroup: one wavefront per SIMD
+    if (left <= 4LL * cus) return {cus, 1};
+    const int wgs = hands_over(pl) ? cus : 2 * cus;
+    return {wgs, (int)std::min<long long>(4, (left + 4LL * wgs - 1) / (4LL * wgs))};
 }
 
 // The items that `parent` handed over since its last orbit job, [parent.orbit_admitted, count)
@@ -376,6 +385,17 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
     }
     if (!run.empty()) {
         HH_CHECK(hipEventRecord(e->ev[0], e->stream));
+        // Streams are dealt out per step, not kept per pool: a process has four hardware queues, and with
+        // a stream per pool those of a mixed pool and of the FP64 pool of its orbiting items could share
+        // one and run in turn (65536 mixed CO2-Ar trajectories after a He-Ar call: 139 ms instead of 93).
+        // Three of the engine's own and its main stream carry up to four pools at once.
+        for (size_t k = 0; k < run.size(); ++k) {
+            run[k]->stream = e->stream;
+            if (k % 4 == 3) continue;
+            hipStream_t& st = e->pool_streams[k % 4];
+            if (!st) HH_CHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+            run[k]->stream = st;
+        }
         for (LanePool* pl : run) {
             PoolCtl ctl{};
             ctl.next = pl->next.as<unsigned long long>();
@@ -397,7 +417,7 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
                                         pl->stream));
                     pl->cur = 1 - pl->cur;
                 }
-                const RowPlan rp = row_plan(e, left);
+                const RowPlan rp = row_plan(e, *pl, left);
                 HH_CHECK(run_rows(pl->sys, pl->mixed, pool_sysconst(e, *pl), pl->ring.as<JobDesc>(), ctl,
                                   pl->view(pl->cur), rp.wgs, rp.rows_used, pl->stream));
             } else if (e->use_graphs) {
@@ -409,9 +429,11 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
             }
             pl->live_slots = true;
             HH_CHECK(hipEventRecord(pl->slice_end, pl->stream));
-            HH_CHECK(hipStreamWaitEvent(e->stream, pl->slice_end, 0));
             if (launches) ++*launches;
         }
+        // after every launch: a wait queued between two would hold back a pool that shares the engine
+        // stream or its hardware queue
+        for (LanePool* pl : run) HH_CHECK(hipStreamWaitEvent(e->stream, pl->slice_end, 0));
         HH_CHECK(hipEventRecord(e->ev[1], e->stream));
         HH_CHECK(hipStreamSynchronize(e->stream));
         float ms = 0.0f;
@@ -441,8 +463,13 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
             std::memcpy(orbit.data(), pl->h_orbit, pl->ring_cap * sizeof(int));
             next = *pl->h_next;
         } else {
-            HH_CHECK(hipMemcpy(done.data(), pl->ring_done.p, pl->ring_cap * sizeof(int), hipMemcpyDeviceToHost));
-            HH_CHECK(hipMemcpy(orbit.data(), pl->ring_orbit.p, pl->ring_cap * sizeof(int), hipMemcpyDeviceToHost));
+            // the ring slots in flight (all of them when they wrap around)
+            int s0 = (int)(pl->inflight.front()->seq % pl->ring_cap), s1 = (int)(pl->inflight.back()->seq % pl->ring_cap);
+            if (s1 < s0) s0 = 0, s1 = pl->ring_cap - 1;
+            const size_t nb = (size_t)(s1 - s0 + 1) * sizeof(int);
+            HH_CHECK(hipMemcpy(done.data() + s0, pl->ring_done.as<int>() + s0, nb, hipMemcpyDeviceToHost));
+            if (hands_over(*pl))
+                HH_CHECK(hipMemcpy(orbit.data() + s0, pl->ring_orbit.as<int>() + s0, nb, hipMemcpyDeviceToHost));
             HH_CHECK(hipMemcpy(&next, pl->next.p, sizeof next, hipMemcpyDeviceToHost));
         }
         // lanes that found the queue empty advanced the head past the end; none of those
