@@ -22,149 +22,287 @@ namespace hh {
 constexpr double kPI = 3.14159265358979323846;
 
 // ------------------------------------------------------------------ CF -> SF
-// The pack kernel only reads cf (thread k > n needs the original cf[2n - k] that thread 2n - k
-// would otherwise be overwriting); the in-place apodization of the input that the reference
-// performs is written by sf_unpack_kernel, after the transform.
-__global__ void __launch_bounds__(256) sf_pack_kernel(const double* __restrict__ cf, long n, double dt,
-                                                      double2* __restrict__ z)
+// The reference packs the n apodized samples v into a Hermitian sequence of 2n complex values and keeps
+// n of the transform's 2n values, which are real: sf_j ~ v_0 + 2 sum_k v_k cos(pi k (2j + 1) / 2n).
+// That is a complex transform of n points (Makhoul 1980) of
+//   V_k = e^{i pi k / 2n} (v_k - i v_{n-k}), v_n = 0,   x_j = sum_k V_k e^{2 pi i jk / n}
+// whose real parts x_0, x_1, ... are sf_0, sf_2, ... and, from the end, sf_1, sf_3, ...  (The x are real, so
+// n/2 points would do, for 2 us less of a call's 44 at n = 4096, but the imaginary parts take half of the
+// rounding errors' squares with them: error in the 2-norm 2.5e-16 to 3.5e-16 from n = 2^10 to 2^20, against
+// 1.8e-16 to 2.7e-16 here and 2.0e-16 to 2.8e-16 with radix-2 stages over the 2n points.)
+//
+// The points run as Stockham passes of radix R over global memory, each R-point transform in LDS by
+// eight points per thread (radix 8, the last step 2, 4 or 8): one workgroup does it all up to
+// n = 4096, beyond that it is as few passes as that allows (two up to n = 2^20).  The first pass makes
+// the V_k from cf as it loads them, the last one writes sf in order, nu and the apodized cf.
+// What bounds it: at n = 4096 the call's launch and wait and the instructions of one workgroup; at 2^20
+// points two passes over 16 MiB with a sincospi per point and pass.  Radix-2 stages with a sincospi per
+// butterfly took 65 us of kernels at n = 4096 and 245 us at 2^20; this takes
+// 15 us and 33 us.
+constexpr int kFftSingleLog = 12;   // one workgroup: 512 threads, 136 KiB of LDS
+constexpr int kFftPassLog = 10;     // a pass of 4 columns: 512 threads, 88 KiB
+constexpr int kFftColsLog = 2;      // columns of a workgroup: 64-byte rows of complex values
+constexpr double kSqrtHalf = 0.70710678118654752440;
+
+__device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ double2 cmul(double2 a, double2 b)
 {
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= 2 * n) return;
-    const double tmax = dt * n;
-    const double inv2n = 1.0 / (2.0 * n);
-    double s, c;
-    sincospi((double)k / (2.0 * n), &s, &c);   // e^{i pi k / 2n}
-    double v;
-    if (k < n) {
-        const double tc = dt * k, r = tc / tmax;
-        const double f = (1.0 - r * r) * (1.0 - r * r);
-        v = cf[k] * f;
-    } else if (k == n) {
-        z[k] = make_double2(0.0, 0.0);
-        return;
-    } else {
-        const long i = 2 * n - k;
-        const double tc = dt * i, r = tc / tmax;
-        v = -(cf[i] * ((1.0 - r * r) * (1.0 - r * r)));
+    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+__device__ __forceinline__ double2 ctimes_i(double2 a) { return make_double2(-a.y, a.x); }
+__device__ __forceinline__ double2 cispi(double x)
+{
+    double2 w;
+    sincospi(x, &w.y, &w.x);
+    return w;
+}
+
+// backward transforms (e^{+i}) of 2, 4 and 8 points, in place
+__device__ __forceinline__ void dft4(double2& a, double2& b, double2& c, double2& d)
+{
+    const double2 s = cadd(a, c), t = csub(a, c), u = cadd(b, d), v = ctimes_i(csub(b, d));
+    a = cadd(s, u);
+    b = cadd(t, v);
+    c = csub(s, u);
+    d = csub(t, v);
+}
+
+__device__ __forceinline__ void dft8(double2* v)
+{
+    double2 e[4], o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        e[i] = cadd(v[i], v[i + 4]);
+        o[i] = csub(v[i], v[i + 4]);
     }
-    z[k] = make_double2(v * c * inv2n, v * s * inv2n);
+    o[1] = make_double2((o[1].x - o[1].y) * kSqrtHalf, (o[1].x + o[1].y) * kSqrtHalf);
+    o[2] = ctimes_i(o[2]);
+    o[3] = make_double2(-(o[3].x + o[3].y) * kSqrtHalf, (o[3].x - o[3].y) * kSqrtHalf);
+    dft4(e[0], e[1], e[2], e[3]);
+    dft4(o[0], o[1], o[2], o[3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        v[2 * i] = e[i];
+        v[2 * i + 1] = o[i];
+    }
 }
 
-// one radix-2 Stockham stage over global memory: len = 2^stage * 2
-__global__ void __launch_bounds__(256) fft_stage_kernel(const double2* __restrict__ in, double2* __restrict__ out,
-                                                        long M, long half_len)
+// x (1 - r^2)^2, r = k/n (exact: n is a power of two), the window with its rounding error
+__device__ __forceinline__ double connes(double x, long k, double inv_n)
 {
-    const long j = (long)blockIdx.x * blockDim.x + threadIdx.x;   // butterfly index, M/2 of them
-    if (j >= M / 2) return;
-    const long k = j % half_len;        // position inside the sub-transform
-    const long g = j / half_len;        // sub-transform group
-    // Stockham: inputs a = in[j], b = in[j + M/2]; outputs to out[g*2*half_len + k] and + half_len
-    const double2 a = in[j], b = in[j + M / 2];
-    double s, c;
-    sincospi((double)k / (double)half_len, &s, &c);   // backward: w = e^{+i pi k / half_len}
-    const double2 wb = make_double2(b.x * c - b.y * s, b.x * s + b.y * c);
-    out[g * 2 * half_len + k] = make_double2(a.x + wb.x, a.y + wb.y);
-    out[g * 2 * half_len + k + half_len] = make_double2(a.x - wb.x, a.y - wb.y);
+    const double r = (double)k * inv_n, p = r * r, f = 1.0 - p;
+    const double fl = (-p - (f - 1.0)) - fma(r, r, -p);
+    const double g = f * f, gl = fma(f, f, -g) + 2.0 * f * fl;
+    return fma(x, g, x * gl);
 }
 
-// whole transform in LDS for M <= 8192 complex values (128 KiB)
-__global__ void __launch_bounds__(1024) fft_lds_kernel(const double2* __restrict__ in, double2* __restrict__ out,
-                                                       long M)
+// One Stockham pass of radix R = 2^logr, after passes of a combined radix 2^logl, for the 2^logc columns
+// of this workgroup.  A thread holds rows q = b + i R/8 of one column.
+template <bool FIRST, bool LAST>
+__global__ void __launch_bounds__(512) sf_pass_kernel(double* cf, const double2* __restrict__ in,
+                                                       double2* __restrict__ out, double* __restrict__ nu,
+                                                       double* __restrict__ sf, int logn, double dt, int logr, int logl,
+                                                       int logc)
 {
     extern __shared__ double2 sm[];
-    double2* a = sm;
-    for (long i = threadIdx.x; i < M; i += blockDim.x) a[i] = in[i];
-    __syncthreads();
-    // in place: bit reversal, then decimation-in-time radix-2 butterflies
-    int logM = 0;
-    while ((1L << logM) < M) ++logM;
-    for (long i = threadIdx.x; i < M; i += blockDim.x) {
-        long r = 0, x = i;
-        for (int b = 0; b < logM; ++b) {
-            r = (r << 1) | (x & 1);
-            x >>= 1;
+    const long n = 1L << logn;
+    const int t = threadIdx.x, c = t & ((1 << logc) - 1), b = t >> logc, eighth = 1 << (logr - 3);
+    const int logcols = logn - logr;
+    const long L = 1L << logl;
+    // Workgroups go to the eight XCDs in turn: neighbouring tiles, which share cache lines, go to one
+    // (n = 2^20: 42 -> 33 us)
+    const long tile = gridDim.x % 8 ? blockIdx.x : (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+    // a pass's columns j; in the last pass half of a workgroup's columns mirror the other half
+    const int half = 1 << logc >> 1;
+    long j;
+    if (LAST && half)
+        j = c < half ? tile * half + c : (1L << logcols) - 1 - (tile * half + c - half);
+    else
+        j = (tile << logc) + c;
+    const long k0 = j & (L - 1);
+    auto slot = [&](int q, int col) { return ((q + (q >> 3)) << logc) + col; };
+
+    double2 v[8];
+    if constexpr (FIRST) {
+        const double inv_n = 1.0 / (double)n;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const long k = j + ((long)(b + i * eighth) << logcols);
+            const double v0 = connes(cf[k], k, inv_n), v1 = k ? connes(cf[n - k], n - k, inv_n) : 0.0;
+            v[i] = cmul(cispi((double)k * (0.5 * inv_n)), make_double2(v0, -v1));
         }
-        if (r > i) {
-            const double2 t = a[i];
-            a[i] = a[r];
-            a[r] = t;
+    } else {
+        const double unit = 2.0 / (double)(L << logr);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int q = b + i * eighth;
+            v[i] = cmul(in[j + ((long)q << logcols)], cispi((double)(q * k0) * unit));
         }
     }
-    __syncthreads();
-    for (long half = 1; half < M; half <<= 1) {
-        for (long j = threadIdx.x; j < M / 2; j += blockDim.x) {
-            const long k = j % half;
-            const long i0 = (j / half) * 2 * half + k, i1 = i0 + half;
-            double s, c;
-            sincospi((double)k / (double)half, &s, &c);
-            const double2 u = a[i0], v = a[i1];
-            const double2 w = make_double2(v.x * c - v.y * s, v.x * s + v.y * c);
-            a[i0] = make_double2(u.x + w.x, u.y + w.y);
-            a[i1] = make_double2(u.x - w.x, u.y - w.y);
+    // the roots e^{2 pi i q / R} of the steps
+    double2* root = sm + ((1 << logr) + (1 << (logr - 3)) << logc);
+    const double rel = 2.0 / (double)(1 << logr);
+    for (int q = t; q < 1 << logr; q += blockDim.x) root[q] = cispi((double)q * rel);
+
+    for (int lg = 0;;) {
+        const int rest = logr - lg;
+        if (rest >= 3) {
+            if (lg) {
+                const int k = (b & ((1 << lg) - 1)) << (logr - lg - 3);
+#pragma unroll
+                for (int i = 1; i < 8; ++i) v[i] = cmul(v[i], root[i * k]);
+            }
+            dft8(v);
+            if (rest == 3) break;
+        } else {
+            // radix 4 or 2: butterflies of the rows b + u R/8
+            if (rest == 2) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                    for (int i = 1; i < 4; ++i) v[2 * i + u] = cmul(v[2 * i + u], root[i * (b + u * eighth)]);
+                    dft4(v[u], v[2 + u], v[4 + u], v[6 + u]);
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const double2 x = cmul(v[4 + u], root[b + u * eighth]);
+                    v[4 + u] = csub(v[u], x);
+                    v[u] = cadd(v[u], x);
+                }
+            }
+            break;
         }
+        const int k = b & ((1 << lg) - 1), g = b >> lg;
+        if (lg) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sm[slot((g << (lg + 3)) + k + (i << lg), c)] = v[i];
         __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = sm[slot(b + i * eighth, c)];
+        lg += 3;
     }
-    for (long i = threadIdx.x; i < M; i += blockDim.x) out[i] = a[i];
+
+    if constexpr (!LAST) {
+        const long o = ((j >> logl) << (logl + logr)) + k0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) out[o + ((long)(b + i * eighth) << logl)] = v[i];
+    } else {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sm[slot(b + i * eighth, c)] = v[i];
+        __syncthreads();
+        const double LightSpeed_cm = 2.99792458e10, ATU = 2.4188843265857e-17;
+        const double ADIPMOMU = 8.4783536255e-30, EPSILON0 = 8.8541878128e-12;
+        const double Xscale = 1.0 / LightSpeed_cm / ATU / 2.0 / kPI;
+        const double Yscale = ATU * ADIPMOMU * ADIPMOMU / (4.0 * kPI * EPSILON0);
+        const double tmax = n * dt;
+        // tmax / pi * Yscale / 2n with its rounding error
+        const double q0 = tmax / kPI, q1 = fma(-q0, kPI, tmax) / kPI, inv2n = 0.5 / n;
+        const double s0 = q0 * Yscale * inv2n, s1 = (fma(q0, Yscale, -(q0 * Yscale)) + q1 * Yscale) * inv2n;
+        auto scaled = [&](double x) { return fma(x, s0, x * s1); };
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = t + i * blockDim.x;
+            const int col = half ? e & (half - 1) : 0, q = half ? e >> (logc - 1) : e;
+            long m = (half ? tile * half + col : 0) + ((long)q << logl);
+            double y = sm[slot(q, col)].x, ym = sm[slot((1 << logr) - 1 - q, half + col)].x;
+            if (m >= n / 2) {
+                m = n - 1 - m;
+                const double s = y;
+                y = ym;
+                ym = s;
+            }
+            sf[2 * m] = scaled(y);
+            sf[2 * m + 1] = scaled(ym);
+        }
+        const double itmax = recip<double>(tmax);
+#pragma unroll 4
+        for (int i = 0; i < 8; ++i) {
+            const long k = ((long)blockIdx.x * 8 + i) * blockDim.x + t;
+            // Connes apodization of the input in place, as the reference does (src/hawaii.c:5581): no
+            // workgroup reads cf any more
+            const double r = divide<double>(dt * k, tmax, itmax);
+            cf[k] *= (1.0 - r * r) * (1.0 - r * r);
+            nu[k] = divide<double>(k * kPI, tmax, itmax) * Xscale;
+        }
+    }
 }
 
-__global__ void __launch_bounds__(256) sf_unpack_kernel(const double2* __restrict__ Z, long n, double dt,
-                                                        double* __restrict__ nu, double* __restrict__ sf,
-                                                        double* __restrict__ cf)
+// n = 2, 4: the cosine sum itself
+__global__ void __launch_bounds__(64) sf_direct_kernel(double* cf, double* __restrict__ nu, double* __restrict__ sf,
+                                                       int n, double dt)
 {
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    {
-        // Connes apodization of the input in place, as the reference does (src/hawaii.c:5581)
-        const double r = (dt * k) / (dt * n);
-        cf[k] *= (1.0 - r * r) * (1.0 - r * r);
-    }
+    const int j = threadIdx.x;
+    double x[4], acc = 0.0;
+    for (int k = 0; k < n; ++k) x[k] = cf[k];
+    __syncthreads();
+    if (j >= n) return;
+    for (int k = 0; k < n; ++k)
+        acc += (k ? 2.0 : 1.0) * connes(x[k], k, 1.0 / n) * cospi((double)(k * (2 * j + 1)) / (2.0 * n));
     const double LightSpeed_cm = 2.99792458e10, ATU = 2.4188843265857e-17;
     const double ADIPMOMU = 8.4783536255e-30, EPSILON0 = 8.8541878128e-12;
     const double Xscale = 1.0 / LightSpeed_cm / ATU / 2.0 / kPI;
     const double Yscale = ATU * ADIPMOMU * ADIPMOMU / (4.0 * kPI * EPSILON0);
-    const double tmax = n * dt;
-    nu[k] = k * kPI / tmax * Xscale;
-    sf[k] = Z[k].x * tmax / kPI * Yscale;
+    const double tmax = n * dt, r = (dt * j) / (dt * n);
+    cf[j] *= (1.0 - r * r) * (1.0 - r * r);
+    nu[j] = j * kPI / tmax * Xscale;
+    sf[j] = acc * (tmax / kPI * Yscale / (2.0 * n));
+}
+
+// Global passes of a transform of 2^logn points: as many as it takes at 2^kFftPassLog points each
+int sf_passes(int logn) { return logn <= kFftSingleLog ? 1 : (logn + kFftPassLog - 1) / kFftPassLog; }
+
+size_t sf_work_bytes(long n, int which)
+{
+    int logn = 0;
+    while ((1L << logn) < n) ++logn;
+    return sf_passes(logn) > 1 + which ? (size_t)n * sizeof(double2) : 0;
 }
 
 hipError_t run_cf_to_sf(double* cf, long n, double dt, double2* work_a, double2* work_b, double* nu, double* sf,
-                        hipStream_t st, bool lds_ok)
+                        hipStream_t st)
 {
-    const long M = 2 * n;
-    hipLaunchKernelGGL(sf_pack_kernel, dim3((unsigned)((M + 255) / 256)), dim3(256), 0, st, cf, n, dt, work_a);
-    double2* res = work_a;
-    if (M <= 8192 && lds_ok) {
-        const size_t lds = M * sizeof(double2);
+    int logn = 0;
+    while ((1L << logn) < n) ++logn;
+    if (n <= 4) {
+        hipLaunchKernelGGL(sf_direct_kernel, dim3(1), dim3(64), 0, st, cf, nu, sf, (int)n, dt);
+        return hipGetLastError();
+    }
+    const int passes = sf_passes(logn);
+    double2 *src = work_b, *dst = work_a;
+    int logl = 0;
+    for (int p = 0; p < passes; ++p) {
+        const int logr = (logn - logl + passes - p - 1) / (passes - p), logc = passes == 1 ? 0 : kFftColsLog;
+        const bool first = p == 0, last = p == passes - 1;
+        auto k = first ? (last ? sf_pass_kernel<true, true> : sf_pass_kernel<true, false>)
+                       : (last ? sf_pass_kernel<false, true> : sf_pass_kernel<false, false>);
+        const int points = 1 << (logr + logc);
+        const size_t lds = (size_t)(points + points / 8 + (1 << logr)) * sizeof(double2);
         if (lds > 65536) {
-            hipError_t e = hipFuncSetAttribute((const void*)fft_lds_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)lds);
+            const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     (int)lds);
             if (e != hipSuccess) return e;
         }
-        hipLaunchKernelGGL(fft_lds_kernel, dim3(1), dim3(1024), lds, st, work_a, work_b, M);
-        res = work_b;
-    } else {
-        double2 *src = work_a, *dst = work_b;
-        for (long half = 1; half < M; half <<= 1) {
-            hipLaunchKernelGGL(fft_stage_kernel, dim3((unsigned)((M / 2 + 255) / 256)), dim3(256), 0, st, src, dst, M,
-                               half);
-            double2* t = src;
-            src = dst;
-            dst = t;
-        }
-        res = src;
+        hipLaunchKernelGGL(k, dim3((unsigned)(n >> (logr + logc))), dim3(points / 8), lds, st, cf, src, dst, nu,
+                           sf, logn, dt, logr, logl, logc);
+        logl += logr;
+        double2* x = src;
+        src = dst;
+        dst = x;
     }
-    hipLaunchKernelGGL(sf_unpack_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, res, n, dt, nu, sf, cf);
     return hipGetLastError();
 }
 
 // ------------------------------------------------------------------ CF -> SF without allocation
-// The two 2n-point work sequences of the transform live in a file-scope device array instead of
-// engine-allocated buffers, for callers that cannot allocate (graph capture, tight serving loops).
+// The n-point work sequence of the transform lives in a file-scope device array instead of an
+// engine-allocated buffer, for callers that cannot allocate (graph capture, tight serving loops).
 // Every device holds its own copy; its address comes from hipGetSymbolAddress once per device
 // (noalloc_scratch_address, at engine creation) and only that address is passed to kernels: the
 // array's name in host code is a host-side stand-in, not a device address.  Calls that overlap on
 // one device share the array and race.
-__device__ __align__(256) double2 scratch[2 * 2 * kCfToSfNoAllocMaxN];
+__device__ __align__(256) double2 scratch[kCfToSfNoAllocMaxN];
 
 hipError_t noalloc_scratch_address(void** ptr)
 {

@@ -705,12 +705,10 @@ int hh_cf_to_sf(hh_engine* e, double* cf_dev, long n, double dt, double* nu_dev,
     if (dt <= 0) return fail(HH_E_INVALID, "sampling time must be positive");
     std::lock_guard<std::recursive_mutex> lock(e->mu);
     HH_CHECK(hipSetDevice(e->device));
-    HH_CHECK(e->fft_a.ensure(2 * n * sizeof(double2)));
-    HH_CHECK(e->fft_b.ensure(2 * n * sizeof(double2)));
-    const bool lds_ok = (size_t)(2 * n) * sizeof(double2) <= e->prop.sharedMemPerBlock;
+    HH_CHECK(e->fft_a.ensure(hh::sf_work_bytes(n, 0)));
+    HH_CHECK(e->fft_b.ensure(hh::sf_work_bytes(n, 1)));
     HH_CHECK(hipEventRecord(e->ev[0], e->stream));
-    HH_CHECK(hh::run_cf_to_sf(cf_dev, n, dt, e->fft_a.as<double2>(), e->fft_b.as<double2>(), nu_dev, sf_dev, e->stream,
-                              lds_ok));
+    HH_CHECK(hh::run_cf_to_sf(cf_dev, n, dt, e->fft_a.as<double2>(), e->fft_b.as<double2>(), nu_dev, sf_dev, e->stream));
     HH_CHECK(hipEventRecord(e->ev[1], e->stream));
     HH_CHECK(hipStreamSynchronize(e->stream));
     if (ms) {
@@ -731,10 +729,8 @@ int hh_cf_to_sf_noalloc(hh_engine* e, double* cf_dev, long n, double dt, double*
     if (dt <= 0) return fail(HH_E_INVALID, "sampling time must be positive");
     std::lock_guard<std::recursive_mutex> lock(e->mu);
     HH_CHECK(hipSetDevice(e->device));
-    double2* a = static_cast<double2*>(e->noalloc_scratch);
-    double2* b = a + 2 * hh::kCfToSfNoAllocMaxN;
-    const bool lds_ok = (size_t)(2 * n) * sizeof(double2) <= e->prop.sharedMemPerBlock;
-    HH_CHECK(hh::run_cf_to_sf(cf_dev, n, dt, a, b, nu_dev, sf_dev, e->stream, lds_ok));
+    HH_CHECK(hh::run_cf_to_sf(cf_dev, n, dt, static_cast<double2*>(e->noalloc_scratch), nullptr, nu_dev, sf_dev,
+                              e->stream));
     HH_CHECK(hipStreamSynchronize(e->stream));
     return HH_OK;
 }

@@ -65,7 +65,9 @@ int zimm_max_length();
 hipError_t run_zimm_reduce(const JobDesc& jb, double ppf, const double2* tw, double* psum, double* pcomp,
                            double* cf_out, hipStream_t st);
 hipError_t run_cf_to_sf(double* cf, long n, double dt, double2* work_a, double2* work_b, double* nu, double* sf,
-                        hipStream_t st, bool lds_ok);
+                        hipStream_t st);
+// bytes of its work_a (which = 0) and work_b (1)
+size_t sf_work_bytes(long n, int which);
 // hh_cf_to_sf_noalloc: the device address of its static work array on the current device
 hipError_t noalloc_scratch_address(void** ptr);
 hipError_t run_m0(int sys, const SysConst& sc, const M0Params& p, uint32_t seed, long nstreams, long npoints,
