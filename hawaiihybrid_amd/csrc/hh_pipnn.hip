@@ -7,8 +7,9 @@
 // examples/correlation_n2_ar.cpp:11-75.
 //
 // One wavefront evaluates 64 phase points per block.  Every lane computes the polynomial
-// features of its own point in FP32 (pip_n2ar.h), 16 at a time (one k-block), standardises
-// them and stages them in LDS as BF16 (high, and low part in the split mode).  The network
+// features of its own point in FP32 (pip_n2ar.h), 16 at a time (one k-block), and makes them
+// BF16 operands (high, and low part in the split mode): through LDS for the energy, by swapping
+// half-wavefronts for the dipole.  The network
 // runs with the points as the columns of v_mfma_f32_32x32x16_bf16 tiles: D[unit][point] =
 // W^T[unit][k] X^T[k][point], weights as the A operand (pre-swizzled 16-byte lane fragments
 // in global memory, L2-resident), features as the B operand.  The accumulator of one layer
@@ -19,7 +20,8 @@
 //
 // Every network is evaluated as a deviation from its value at the reference point where all
 // polynomials vanish (infinite separation; QModel::forward_inf): with x = (p - mean)/scale and
-// x_ref = -mean/scale, the first layer takes dx = p/scale and starts its accumulator from
+// x_ref = -mean/scale, the first layer takes dx = p/scale (the dipole's p, with 1/scale in its
+// weights) and starts its accumulator from
 // z_ref = W^T x_ref + b, each hidden layer passes dh = act(z) - act(z_ref), and the last layer
 // yields d(out) = out - out_ref directly.  The references are computed once on the host in FP64.
 // The BF16 operands then carry only the deviations, so their rounding scales with the signal
@@ -45,18 +47,12 @@ namespace hh {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr double kLN2 = 2.07856749;   // N2 bond length, bohr (src/constants.h:80)
 
 // ------------------------------------------------------------------ device helpers
-__device__ __forceinline__ unsigned bf16_bits(float x)
-{
-    unsigned u = __float_as_uint(x);
-    u += 0x7fffu + ((u >> 16) & 1u);   // round to nearest even
-    return u >> 16;
-}
-__device__ __forceinline__ float bf16_value(unsigned h) { return __uint_as_float(h << 16); }
-
 __device__ __forceinline__ f32x16 mfma16(const u32x4& a, const u32x4& b, const f32x16& c)
 {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
@@ -73,17 +69,18 @@ __device__ __forceinline__ float activate(float x)
     }
 }
 
-// 8 floats -> 8 BF16 (high part) and their residuals (low part)
+// 8 floats -> 8 BF16 (high part) and their residuals (low part); two a conversion (v_cvt_pk_bf16_f32,
+// round to nearest even)
 template <int SPLIT>
 __device__ __forceinline__ void pack8(const float* v, u32x4& hi, u32x4& lo)
 {
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-        const unsigned h0 = bf16_bits(v[2 * w]), h1 = bf16_bits(v[2 * w + 1]);
-        hi[w] = h0 | (h1 << 16);
+        const f32x2 x = {v[2 * w], v[2 * w + 1]};
+        hi[w] = __builtin_bit_cast(unsigned, __builtin_convertvector(x, bf16x2));
         if constexpr (SPLIT) {
-            const unsigned l0 = bf16_bits(v[2 * w] - bf16_value(h0)), l1 = bf16_bits(v[2 * w + 1] - bf16_value(h1));
-            lo[w] = l0 | (l1 << 16);
+            const f32x2 r = {x[0] - __uint_as_float(hi[w] << 16), x[1] - __uint_as_float(hi[w] & 0xffff0000u)};
+            lo[w] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
         }
     }
 }
@@ -210,32 +207,19 @@ __device__ __forceinline__ void pes_variables(const Frame& f, float* y)
     }
 }
 
-// dipole sites (xyz4q_from_bf): N1 (a s, 0, a c), N2 = -N1, N1' (a c, 0, -a s), N2' = -N1', Ar (0, 0, R)
-struct Sites {
-    double x[5], z[5];
-};
-__device__ __forceinline__ Sites sites_of(const Frame& f)
+// dipole sites (xyz4q_from_bf): N1 (as, 0, ac), N2 = -N1, N1' (ac, 0, -as), N2' = -N1', Ar (0, 0, R), with
+// as = a sin(theta_m), ac = a cos(theta_m).  The variables exp(-r_ij / a0), i < j, are those of two fixed
+// distances (N1-N2 and N1'-N2' 2a, the others sqrt(2) a: the host's, in the model) and of the four to Ar.
+__device__ __forceinline__ void dipole_variables(double as, double ac, double R, double inv_a0, float y2a, float yr2a,
+                                                 float* y)
 {
-    const double a = 0.5 * kLN2, c = f.c, s = sqrt(fmax(1.0 - c * c, 0.0));
-    Sites S;
-    S.x[0] = a * s; S.z[0] = a * c;
-    S.x[1] = -a * s; S.z[1] = -a * c;
-    S.x[2] = a * c; S.z[2] = -a * s;
-    S.x[3] = -a * c; S.z[3] = a * s;
-    S.x[4] = 0.0; S.z[4] = f.R;
-    return S;
-}
-
-__device__ __forceinline__ void dipole_variables(const Sites& S, double a0, float* y)
-{
-    int k = 0;
-#pragma unroll
-    for (int i = 0; i < 5; ++i)
-#pragma unroll
-        for (int j = i + 1; j < 5; ++j, ++k) {
-            const double dx = S.x[i] - S.x[j], dz = S.z[i] - S.z[j];
-            y[k] = (float)exp(-sqrt(dx * dx + dz * dz) / a0);
-        }
+    auto v = [&](double x, double z) { return (float)exp(-sqrt(x * x + (z - R) * (z - R)) * inv_a0); };
+    y[0] = y[7] = y2a;
+    y[1] = y[2] = y[4] = y[5] = yr2a;
+    y[3] = v(as, ac);
+    y[6] = v(as, -ac);
+    y[8] = v(ac, -as);
+    y[9] = v(ac, as);
 }
 
 // ------------------------------------------------------------------ model parameters
@@ -248,12 +232,24 @@ struct PesDev {
 };
 
 struct DipModelDev {
-    LayerDev L1, L2;        // 308 -> 40 (2 n-tiles, 20 k-blocks), 40 -> 5 (1 n-tile, 3 k-blocks)
-    const float* xinv;      // [320]
+    LayerDev L1, L2;        // 308 -> 40 (2 n-tiles, 20 k-blocks; the weights hold 1 / scale), 40 -> 5 (1, 3)
+    double inv_a0;
+    float y2a, yr2a;        // exp(-2a / a0), exp(-sqrt(2) a / a0)
 };
 struct DipDev {
     DipModelDev m[2];
 };
+
+// exchanges a's upper half-wavefront with b's lower one
+__device__ __forceinline__ void swap_halves(u32x4& a, u32x4& b)
+{
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const auto r = __builtin_amdgcn_permlane32_swap(a[w], b[w], false, false);
+        a[w] = r[0];
+        b[w] = r[1];
+    }
+}
 
 // stage the 16 input deviations p/scale of k-block kb of this lane's point into LDS
 template <int SPLIT>
@@ -321,54 +317,49 @@ __global__ __launch_bounds__(64) void pipnn_pes_kernel(PesDev<NH + 1> m, const d
 }
 
 // ------------------------------------------------------------------ dipole kernel
+// Bound by vector instructions: 2 x 308 polynomials a point, their conversion to BF16 and 40 SiLUs a
+// model, beside 8000 matrix-core cycles a wavefront.  So the conversion is the hardware's, the scale is in
+// the weights, the distances inside the molecule are constants, the operands change lanes in registers, and
+// the k-blocks are unrolled (they share products of the variables; in a loop over a switch they need 30
+// spilled registers more).  2^20 points in the split mode, both kernels: 920 -> 240 us.  Two wavefronts
+// per SIMD; three (168 registers, 92 spilled) take 390 us.
 template <int SPLIT>
-__global__ __launch_bounds__(64) void pipnn_dip_kernel(DipDev d, const double* __restrict__ q, long n,
-                                                       double* __restrict__ mu)
+__global__ __launch_bounds__(64, 2) void pipnn_dip_kernel(DipDev d, const double* __restrict__ q, long n,
+                                                          double* __restrict__ mu)
 {
-    __shared__ u32x4 fh[64][2], fl[64][2];
     __shared__ float qs[64][5];
     const int lane = threadIdx.x, half = lane >> 5;
     const long i = (long)blockIdx.x * 64 + lane;
     const long ii = i < n ? i : n - 1;
-    double R, c;
-    {
-        const Frame f = frame_of(q, n, ii);
-        R = f.R;
-        c = f.c;
-    }
+    const Frame f = frame_of(q, n, ii);
+    const double ac = 0.5 * kLN2 * f.c, as = 0.5 * kLN2 * sqrt(fmax(1.0 - f.c * f.c, 0.0));
     // blended body-frame dipole: (1 - w) mu_short + w mu_long
-    const double w = quintic_switch(R, 9.5, 12.5);
+    const double w = quintic_switch(f.R, 9.5, 12.5);
     double dx = 0.0, dz = 0.0;
 #pragma unroll 1
     for (int model = 0; model < 2; ++model) {
         const DipModelDev& M = d.m[model];
         float y[10];
-        {
-            Frame f;
-            f.R = R;
-            f.c = c;
-            dipole_variables(sites_of(f), model == 0 ? 2.0 : 6.0, y);
-        }
+        dipole_variables(as, ac, f.R, M.inv_a0, M.y2a, M.yr2a, y);
         f32x16 acc[2][2];
         bias_init<2>(M.L1.bias, acc[0], lane);
         bias_init<2>(M.L1.bias, acc[1], lane);
-#pragma unroll 1
+#pragma unroll 20
         for (int kb = 0; kb < 20; ++kb) {
             float p[16];
             pip_n2ar_dip_block<float>(kb, y, p);
-            __syncthreads();   // the previous block's operands have been read
-            stage_features<SPLIT>(p, M.xinv, kb, fh, fl, lane);
-            __syncthreads();
+            // lane l holds its point's features 0..7 and 8..15; swapped between the half-wavefronts they are
+            // the operands of points 0..31 and 32..63
+            u32x4 bh[2], bl[2];
+            pack8<SPLIT>(p, bh[0], bl[0]);
+            pack8<SPLIT>(p + 8, bh[1], bl[1]);
+            swap_halves(bh[0], bh[1]);
+            if constexpr (SPLIT) swap_halves(bl[0], bl[1]);
             // subnets 0, 1 (units 0..31) read polynomials 0..237 (k-blocks 0..14);
             // subnet 2 (units 32..39) reads 238..307 (k-blocks 14..19)
             const int nt0 = kb <= 14 ? 0 : 1, nt1 = kb >= 14 ? 2 : 1;
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int pt = 32 * t + (lane & 31);
-                const u32x4 bh = fh[pt][half];
-                const u32x4 bl = SPLIT ? fl[pt][half] : bh;
-                kblock<2, 20, SPLIT>(M.L1.A, kb, bh, bl, acc[t], lane, nt0, nt1);
-            }
+            for (int t = 0; t < 2; ++t) kblock<2, 20, SPLIT>(M.L1.A, kb, bh[t], bl[t], acc[t], lane, nt0, nt1);
         }
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -389,25 +380,14 @@ __global__ __launch_bounds__(64) void pipnn_dip_kernel(DipDev d, const double* _
         }
         __syncthreads();
         {
-            Frame f;
-            f.R = R;
-            f.c = c;
-            const Sites S = sites_of(f);
-            double ax = 0.0, az = 0.0;
-#pragma unroll
-            for (int a = 0; a < 5; ++a) {
-                const double dq = (double)qs[lane][a];
-                ax += dq * S.x[a];
-                az += dq * S.z[a];
-            }
+            const double q0 = qs[lane][0], q1 = qs[lane][1], q2 = qs[lane][2], q3 = qs[lane][3], q4 = qs[lane][4];
             const double wm = model == 0 ? 1.0 - w : w;
-            dx += wm * ax;
-            dz += wm * az;
+            dx += wm * ((q0 - q1) * as + (q2 - q3) * ac);
+            dz += wm * ((q0 - q1) * ac - (q2 - q3) * as + q4 * f.R);
         }
         __syncthreads();
     }
     if (i >= n) return;
-    const Frame f = frame_of(q, n, i);
 #pragma unroll
     for (int k = 0; k < 3; ++k) mu[k * n + i] = dz * f.Rh[k] + dx * f.ex[k];
 }
@@ -593,7 +573,6 @@ int hh_pipnn_create(hh_engine* e, const hh_pipnn_desc* d, int precision, hh_pipn
     // dipole: subnets merged block-diagonally; layer 1 308 (pad 320) -> 40 (pad 64),
     // layer 2 40 (pad 48) -> 5 (pad 32)
     StagedLayer dl[2][2] = {};
-    size_t dxi[2] = {0, 0};
     if (has_dip) {
         for (int m = 0; m < 2; ++m) {
             std::vector<double> W1T((size_t)64 * 320, 0.0), W2T((size_t)32 * 48, 0.0), b1(64, 0.0), b2(32, 0.0);
@@ -615,11 +594,10 @@ int hh_pipnn_create(hh_engine* e, const hh_pipnn_desc* d, int precision, hh_pipn
             std::vector<double> xref(320, 0.0);
             for (int k = 0; k < kPipDip; ++k) xref[k] = -d->dip_xmean[m][k] / d->dip_xscale[m][k];
             const std::vector<double> z1 = affine(W1T, 64, 320, xref, b1);
+            for (int j = 0; j < 64; ++j)
+                for (int k = 0; k < kPipDip; ++k) W1T[(size_t)j * 320 + k] /= d->dip_xscale[m][k];
             dl[m][0] = stage_layer(blob, W1T, 64, 320, false, z1, false, HH_ACT_SILU);
             dl[m][1] = stage_layer(blob, W2T, 32, 48, true, std::vector<double>(32, 0.0), true, HH_ACT_SILU);
-            std::vector<float> di(320, 0.0f);
-            for (int k = 0; k < kPipDip; ++k) di[k] = (float)(1.0 / d->dip_xscale[m][k]);
-            dxi[m] = stage(blob, di.data(), di.size() * 4);
         }
     }
 
@@ -654,7 +632,10 @@ int hh_pipnn_create(hh_engine* e, const hh_pipnn_desc* d, int precision, hh_pipn
         for (int m = 0; m < 2; ++m) {
             M->dip.m[m].L1 = view(dl[m][0]);
             M->dip.m[m].L2 = view(dl[m][1]);
-            M->dip.m[m].xinv = reinterpret_cast<const float*>(base + dxi[m]);
+            const double a = 0.5 * kLN2, a0 = m == 0 ? 2.0 : 6.0;
+            M->dip.m[m].inv_a0 = 1.0 / a0;
+            M->dip.m[m].y2a = (float)std::exp(-2.0 * a / a0);
+            M->dip.m[m].yr2a = (float)std::exp(-std::sqrt(2.0) * a / a0);
         }
     *out = M;
     return HH_OK;

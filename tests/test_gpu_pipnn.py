@@ -105,3 +105,16 @@ def test_rejects_unsupported_shape(setup):
     import hawaiihybrid_amd as H
     with pytest.raises(H.HHError):
         n2ar.PipNN(s["eng"], pes_layers=n2ar.synthetic_pes(96), with_dipole=False, weights=s["W"])
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n", [1, 31, 33, 63, 65])
+def test_points_do_not_depend_on_their_neighbours(setup, prec, n):
+    """Batches that end within a wavefront or one of its halves: the same bits as the same points of a
+    large batch, at whatever lanes they fall there."""
+    s = setup
+    model = s["n2ar"].PipNN(s["eng"], precision=prec, weights=s["W"])
+    E, mu, _ = model.eval(s["qd"])
+    Ep, mup, _ = model.eval(s["qd"][:, 100:100 + n].contiguous())
+    assert np.array_equal(Ep.cpu().numpy(), E[100:100 + n].cpu().numpy())
+    assert np.array_equal(mup.cpu().numpy(), mu[:, 100:100 + n].cpu().numpy())
