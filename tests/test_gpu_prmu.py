@@ -108,3 +108,18 @@ def test_prmu_fft_lengths(eng, L):
         want += coeff * (-y0[5] / O.MU_HEAR) * O.prmu_power(x, dt, nfreq)
     got = sf.cpu().numpy()
     assert np.linalg.norm(got - want) / np.linalg.norm(want) < 1e-9
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33])
+def test_prmu_sums_in_trajectory_order(eng, n):
+    """The sum over trajectories around the number of loads in flight: the bits of one call per trajectory
+    added into the same spectrum."""
+    L, nfreq, R0 = 512, 200, 12.0
+    smp = H.Sampler(H.IC_R0_INJECT, H.PAIR_FREE, 300.0, 4.0, 40.0, H.PESMIN_HEAR, R0)
+    ic, _, _ = H.sample_ics(H.he_ar(), smp, 37, n)
+    p = H.PrmuParams(1e-12, 1e-12, 200.0, R0, L, nfreq, H.PREC_FP64, 0, 0)
+    sf = eng.prmu(H.he_ar(), p, eng.to_device_soa(ic))[0]
+    one = eng.torch.zeros(nfreq, dtype=eng.torch.float64, device="cuda:0")
+    for t in range(n):
+        eng.prmu(H.he_ar(), p, eng.to_device_soa(ic[t:t + 1]), one)
+    assert np.array_equal(sf.cpu().numpy(), one.cpu().numpy())
