@@ -81,3 +81,15 @@ def test_session_admission_by_device_memory(eng):
     assert ia.state == H.REQ_DONE and ib.state == H.REQ_DONE
     assert ib.admit_ms >= ia.done_ms - 1e-6
     assert ibig.state == H.REQ_FAILED and b"memory" in ibig.error
+
+
+@pytest.mark.parametrize("nstreams", [1, 63, 300])
+def test_m0_in_slices_equals_m0_in_one(eng, nstreams):
+    """M0 whose streams stop at a slice's end with part of a batch of generator words drawn, over several
+    generations of the words: the bits of the run in one launch."""
+    smp = H.Sampler(H.IC_REJECTION, 1, 300.0, 4.0, 40.0, H.PESMIN_HEAR, 0.0)
+    m_ref, q_ref, _ = eng.m0(H.he_ar(), smp, 9, nstreams * 301, nstreams)
+    s = H.Session(eng, slice_ms=0.1)
+    info = s.poll(s.submit_m0(H.he_ar(), smp, 9, nstreams * 301, nstreams), 100000.0)
+    s.close()
+    assert info.state == H.REQ_DONE and info.m0 == m_ref and info.m0_err == q_ref
