@@ -1181,37 +1181,44 @@ __global__ void __launch_bounds__(256) cf_reduce_final_kernel(int L, int nchunks
 
 // CORRELATION_ARRAY: the same sums with a weight per trajectory and satellite temperature,
 // wr[t * ntemp + st] (Boltzmann reweight times the temperature's partition-function ratio);
-// blockIdx.z is the temperature.  Partial sums psum[(st * nchunks + c) * L + k].
+// blockIdx.z is a group of NT temperatures, so the rows are read once a group and, kReduceUnroll items
+// in flight, bound by their latency (20000 trajectories of both halves, L = 1024, eight temperatures:
+// a temperature per workgroup, an item at a time, 420 us; this 262).
+// Partial sums psum[(st * nchunks + c) * L + k].
+template <int HALVES, int NT>
 __global__ void __launch_bounds__(256) cf_reduce_weighted_partial_kernel(JobDesc jb, long long chunk, int ntemp,
                                                                          const double* __restrict__ wr,
                                                                          double* __restrict__ psum,
                                                                          double* __restrict__ pcomp)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int c = blockIdx.y, st = blockIdx.z;
+    const int c = blockIdx.y, st0 = blockIdx.z * NT;
     if (k >= jb.L) return;
     const long long t0 = (long long)c * chunk;
     long long t1 = t0 + chunk;
     if (t1 > jb.ntraj) t1 = jb.ntraj;
-    double s = 0.0, cc = 0.0;
-    for (long long t = t0; t < t1; ++t) {
-        double v;
-        if (jb.halves == 2) {
-            const long long a = 2 * t, b = 2 * t + 1;
-            if (dropped(jb.status[a], jb.status[b])) continue;
-            const double cf = k < jb.len[a] ? jb.rows[a * jb.L + k] : 0.0;
-            const double cb = k < jb.len[b] ? jb.rows[b * jb.L + k] : 0.0;
-            v = 0.5 * (cf + cb) * kALU * kALU * kALU;
-        } else {
-            if (dropped(jb.status[t], jb.status[t])) continue;
-            const double cf = k < jb.len[t] ? jb.rows[t * jb.L + k] : 0.0;
-            v = cf * kALU * kALU * kALU;
+    double s[NT], cc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) s[j] = cc[j] = 0.0;
+    for (long long t = t0; t < t1; t += kReduceUnroll) {
+        double v[kReduceUnroll];
+#pragma unroll
+        for (int u = 0; u < kReduceUnroll; ++u) v[u] = reduce_value<HALVES>(jb, t + u, t1, k);
+#pragma unroll
+        for (int u = 0; u < kReduceUnroll; ++u) {
+            if (t + u >= t1 || dropped(jb.status[HALVES * (t + u)], jb.status[HALVES * (t + u) + HALVES - 1])) continue;
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                neumaier_add(s[j], cc[j], wr[(t + u) * ntemp + min(st0 + j, ntemp - 1)] * v[u]);
         }
-        neumaier_add(s, cc, wr[t * ntemp + st] * v);
     }
-    const long long o = ((long long)st * gridDim.y + c) * jb.L + k;
-    psum[o] = s;
-    pcomp[o] = cc;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        if (st0 + j >= ntemp) break;
+        const long long o = ((long long)(st0 + j) * gridDim.y + c) * jb.L + k;
+        psum[o] = s[j];
+        pcomp[o] = cc[j];
+    }
 }
 
 // cf_out[st * L + k] = sum over chunks / nstar[st] (0 where nstar is 0: no trajectory carries
@@ -1225,10 +1232,20 @@ __global__ void __launch_bounds__(256) cf_reduce_weighted_final_kernel(int L, in
     const int st = blockIdx.y;
     if (k >= L) return;
     double s = 0.0, cc = 0.0;
-    for (int c = 0; c < nchunks; ++c) {
-        const long long o = ((long long)st * nchunks + c) * L + k;
-        neumaier_add(s, cc, psum[o]);
-        cc += pcomp[o];
+    for (int c = 0; c < nchunks; c += kReduceUnroll) {
+        double ps[kReduceUnroll], pc[kReduceUnroll];
+#pragma unroll
+        for (int u = 0; u < kReduceUnroll; ++u) {
+            const bool in = c + u < nchunks;
+            const long long o = ((long long)st * nchunks + (in ? c + u : nchunks - 1)) * L + k;
+            ps[u] = in ? psum[o] : 0.0;
+            pc[u] = in ? pcomp[o] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < kReduceUnroll; ++u) {
+            neumaier_add(s, cc, ps[u]);
+            cc += pc[u];
+        }
     }
     cf_out[(long long)st * L + k] = nstar[st] > 0.0 ? (s + cc) / nstar[st] : 0.0;
 }
@@ -1383,8 +1400,12 @@ LaneSlots slots_view(int sys, void* base, long long S)
 hipError_t run_reduce_weighted(const JobDesc& jb, int ntemp, const double* wr, const double* nstar, double* psum,
                                double* pcomp, long long chunk, int nchunks, double* cf_out, hipStream_t st)
 {
-    dim3 g1((jb.L + 255) / 256, nchunks, ntemp);
-    hipLaunchKernelGGL(cf_reduce_weighted_partial_kernel, g1, dim3(256), 0, st, jb, chunk, ntemp, wr, psum, pcomp);
+    // groups of eight temperatures, of four where there are no more
+    const int nt = ntemp > 4 ? 8 : 4;
+    auto k = jb.halves == 2 ? (nt == 8 ? cf_reduce_weighted_partial_kernel<2, 8> : cf_reduce_weighted_partial_kernel<2, 4>)
+                            : (nt == 8 ? cf_reduce_weighted_partial_kernel<1, 8> : cf_reduce_weighted_partial_kernel<1, 4>);
+    hipLaunchKernelGGL(k, dim3((jb.L + 255) / 256, nchunks, (ntemp + nt - 1) / nt), dim3(256), 0, st, jb, chunk, ntemp,
+                       wr, psum, pcomp);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(cf_reduce_weighted_final_kernel, dim3((jb.L + 255) / 256, ntemp), dim3(256), 0, st, jb.L,

@@ -71,3 +71,24 @@ def test_array_rejects_bad_input(eng):
         eng.cf_array(H.he_ar(), p, x, 100.0, H.PAIR_FREE, H.PESMIN_HEAR, [])
     with pytest.raises(H.HHError):
         eng.cf_array(H.he_ar(), H.cf_params(64, zimmermann=True), x, 100.0, H.PAIR_BOUND, H.PESMIN_HEAR, [50.0])
+
+
+@pytest.mark.parametrize("halves", [1, 2])
+@pytest.mark.parametrize("ntemp,n", [(1, 15), (4, 16), (5, 17), (8, 257), (9, 300)])
+def test_array_temperatures_do_not_depend_on_their_group(eng, ntemp, n, halves):
+    """The weighted sums of groups of temperatures, at the edges of a group, of the items in flight and of
+    a chunk of 256 items: the bits of each temperature on its own."""
+    import hawaiihybrid_amd as H
+    T = 100.0
+    smp = H.Sampler(H.IC_REJECTION, H.PAIR_BOUND, T, 4.0, 40.0, H.PESMIN_HEAR, 0.0)
+    x = eng.to_device_soa(H.sample_ics(H.he_ar(), smp, 13, n)[0])
+    p = H.cf_params(300, rtol=1e-12, halves=H.HALVES_BOTH if halves == 2 else H.HALVES_FORWARD,
+                    engine=H.ENGINE_BATCHED)
+    temps = [60.0 + 10.0 * k for k in range(ntemp)]
+    arr, nstar, _ = eng.cf_array(H.he_ar(), p, x, T, H.PAIR_BOUND, H.PESMIN_HEAR, temps)
+    arr = arr.cpu().numpy()
+    assert np.all(np.isfinite(arr)) and np.any(arr != 0.0)
+    for k, Ts in enumerate(temps):
+        one, ns, _ = eng.cf_array(H.he_ar(), p, x, T, H.PAIR_BOUND, H.PESMIN_HEAR, [Ts])
+        assert ns[0] == nstar[k]
+        assert np.array_equal(one[0].cpu().numpy(), arr[k])
