@@ -110,17 +110,18 @@ def hbm_section(H, eng, stm, mixed_len, plain_len, plain_reduce_ms, L, prmu_ntra
                   `alone`: the first timed step's job reduced after the plain engine's
                   integration (nothing else on the device); `in_batch`: the K jobs of the timed
                   mixed batch, each reduced while the pools integrate the others.
-      prmu        the PR/mu spectrum pass (pack + Connes window, four-step FFT of two complex
-                  series per trajectory, power, accumulation) of He-Ar trajectories at FFT length
-                  prmu_L: pack reads 24 B per recorded sample and writes 32 B per point, each FFT
-                  step reads and writes 64 B per point, power reads 48 B and writes 8 B per kept
+      prmu        the PR/mu spectrum pass (Connes window, four-step FFT of two complex series per
+                  trajectory, power, accumulation) of He-Ar trajectories at FFT length prmu_L: the
+                  first FFT step reads 24 B per recorded sample and writes 32 B per point, the
+                  second reads and writes 64 B per point, power reads 48 B and writes 8 B per kept
                   frequency, accumulation reads 8 B per frequency and trajectory; time = the
                   engine's events around the pass (integration excluded).
-      cf_to_sf    idct_cf_to_sf of an sf_n-point CF (Connes window, IDCT via an M = 2n-point
-                  complex FFT): the pack kernel reads 8 B and writes 16 B per point of M, each of
-                  the log2(M) global radix-2 passes (M > 8192) reads and writes 32 B per point of
-                  M, the unpack kernel reads 16 B and writes 24 B per CF point; `bytes_algorithmic`
-                  is the transform's own input and output (8 B read, 16 B written per CF point)."""
+      cf_to_sf    idct_cf_to_sf of an sf_n-point CF (Connes window, IDCT via an n-point complex FFT
+                  in one pass up to n = 4096, else of up to 1024 points a pass): the first pass
+                  reads 16 B of the CF per point, the last one reads and writes the CF and writes
+                  nu and sf, 32 B, and 32 B per point are written and read between two passes;
+                  `bytes_algorithmic` is the transform's own input and output (8 B read, 16 B
+                  written per CF point)."""
     import torch
     out = {}
 
@@ -144,16 +145,15 @@ def hbm_section(H, eng, stm, mixed_len, plain_len, plain_reduce_ms, L, prmu_ntra
     _, counted, nc, st = eng.prmu(H.he_ar(), pp, x)
     rec = float(np.minimum(eng.items(0, prmu_ntraj, prmu_L)["len"], prmu_L).sum())
     nt = prmu_ntraj
-    pb = 24.0 * rec + nt * prmu_L * (32.0 + 2 * 64.0) + nt * nfreq * (48.0 + 8.0 + 8.0)
+    pb = 24.0 * rec + nt * prmu_L * (32.0 + 64.0) + nt * nfreq * (48.0 + 8.0 + 8.0)
     out["prmu_spectrum"] = dict(rate(pb, st.reduce_ms), trajectories=nt, fft_length=prmu_L, nfreq=nfreq)
     del x
     # CF -> SF
     cf = torch.rand(sf_n, dtype=torch.float64, device="cuda:0")
     eng.cf_to_sf(cf.clone(), 200.0)
     _, _, ms = eng.cf_to_sf(cf, 200.0)
-    M = 2 * sf_n
-    passes = int(math.log2(M)) if M > 8192 else 1
-    mb = 24.0 * M + passes * 32.0 * M + 40.0 * sf_n
+    passes = 1 if sf_n <= 4096 else -(-(sf_n.bit_length() - 1) // 10)
+    mb = (16.0 + 32.0 + (passes - 1) * 32.0) * sf_n
     out["cf_to_sf"] = dict(rate(mb, ms), points=sf_n, fft_passes=passes, bytes_algorithmic=24.0 * sf_n,
                            GBps_algorithmic=24.0 * sf_n / (ms * 1e-3) / 1e9)
     del cf
