@@ -33,7 +33,6 @@ counter runs into the pool kernel's bytes per launch (profiles/).
 """
 import argparse
 import json
-import math
 import os
 import sys
 import time
@@ -116,10 +115,10 @@ def hbm_section(H, eng, stm, mixed_len, plain_len, plain_reduce_ms, L, prmu_ntra
                   second reads and writes 64 B per point, power reads 48 B and writes 8 B per kept
                   frequency, accumulation reads 8 B per frequency and trajectory; time = the
                   engine's events around the pass (integration excluded).
-      cf_to_sf    idct_cf_to_sf of an sf_n-point CF (Connes window, IDCT via an n-point complex FFT
-                  in one pass up to n = 4096, else of up to 1024 points a pass): the first pass
-                  reads 16 B of the CF per point, the last one reads and writes the CF and writes
-                  nu and sf, 32 B, and 32 B per point are written and read between two passes;
+      cf_to_sf    idct_cf_to_sf of an sf_n-point CF (Connes window, IDCT via an M = 2n-point complex
+                  FFT of up to 2048 points a pass): the first pass reads 8 B of the CF per point of
+                  M, the last one reads and writes the CF and writes nu and sf, 32 B per CF point,
+                  and 32 B per point of M are written and read between two passes;
                   `bytes_algorithmic` is the transform's own input and output (8 B read, 16 B
                   written per CF point)."""
     import torch
@@ -152,8 +151,8 @@ def hbm_section(H, eng, stm, mixed_len, plain_len, plain_reduce_ms, L, prmu_ntra
     cf = torch.rand(sf_n, dtype=torch.float64, device="cuda:0")
     eng.cf_to_sf(cf.clone(), 200.0)
     _, _, ms = eng.cf_to_sf(cf, 200.0)
-    passes = 1 if sf_n <= 4096 else -(-(sf_n.bit_length() - 1) // 10)
-    mb = (16.0 + 32.0 + (passes - 1) * 32.0) * sf_n
+    passes = -(-sf_n.bit_length() // 11)
+    mb = (2 * 8.0 + 32.0 + (passes - 1) * 2 * 32.0) * sf_n
     out["cf_to_sf"] = dict(rate(mb, ms), points=sf_n, fft_passes=passes, bytes_algorithmic=24.0 * sf_n,
                            GBps_algorithmic=24.0 * sf_n / (ms * 1e-3) / 1e9)
     del cf

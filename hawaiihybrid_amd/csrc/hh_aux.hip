@@ -18,165 +18,141 @@ namespace hh {
 constexpr double kPI = 3.14159265358979323846;
 
 // ------------------------------------------------------------------ CF -> SF
-// The reference packs the n apodized samples v into a Hermitian sequence of 2n complex values and keeps
-// n of the transform's 2n values, which are real: sf_j ~ v_0 + 2 sum_k v_k cos(pi k (2j + 1) / 2n).
-// That is a complex transform of n points (Makhoul 1980) of
-//   V_k = e^{i pi k / 2n} (v_k - i v_{n-k}), v_n = 0,   x_j = sum_k V_k e^{2 pi i jk / n}
-// whose real parts x_0, x_1, ... are sf_0, sf_2, ... and, from the end, sf_1, sf_3, ...  (The x are real, so
-// n/2 points would do, for 2 us less of a call's 44 at n = 4096, but the imaginary parts take half of the
-// rounding errors' squares with them: error in the 2-norm 2.5e-16 to 3.5e-16 from n = 2^10 to 2^20, against
-// 1.8e-16 to 2.7e-16 here and 2.0e-16 to 2.8e-16 with radix-2 stages over the 2n points.)
+// The packed sequence of 2n complex values goes through radix-2 Stockham stages, up to eleven of them in a
+// pass over global memory, three at a time in registers with eight points per thread: one pass up to
+// n = 1024, two up to n = 2^21, with the packing in the first one's loads and the scaling, nu and the
+// apodized cf in the last one's stores.
 //
-// The points run as Stockham passes of radix R over global memory, each R-point transform in LDS by
-// eight points per thread (radix 8, the last step 2, 4 or 8): one workgroup does it all up to
-// n = 4096, beyond that it is as few passes as that allows (two up to n = 2^20).  The first pass makes
-// the V_k from cf as it loads them, the last one writes sf in order, nu and the apodized cf.
-// What bounds it: at n = 4096 the call's launch and wait and the instructions of one workgroup; at 2^20
-// points two passes over 16 MiB with a sincospi per point and pass.  Radix-2 stages with a sincospi per
-// butterfly took 65 us of kernels at n = 4096 and 245 us at 2^20; this takes
-// 15 us and 33 us.
-constexpr int kFftSingleLog = 12;   // one workgroup: 512 threads, 136 KiB of LDS
-constexpr int kFftPassLog = 10;     // a pass of 4 columns: 512 threads, 88 KiB
-constexpr int kFftColsLog = 2;      // columns of a workgroup: 64-byte rows of complex values
-constexpr double kSqrtHalf = 0.70710678118654752440;
+// The butterflies and their roots are those of a transform that runs a stage at a time, bit for bit.  A
+// transform of n points (the packed sequence is Hermitian) with radix-8 butterflies needs half of the time
+// in the kernels at n = 2^20 and 2 us less of a call at n = 4096, with an error in the 2-norm that is the same
+// within a tenth, 1.8e-16 to 2.8e-16 from n = 2^10 to 2^20; but where a long CF's peak is hundreds of times
+// the spectrum's root mean square, the peak's roundings decide the far wing, and two such transforms
+// differ there by up to 1e-13 of the root mean square.
+//
+// Bound by the butterflies' sincospi and the latency of the passes.  Kernels of a call, with a pass per stage
+// (or one workgroup for all of them at n = 4096) before and now: n = 2^20 245 and 58 us, n = 4096 65 and
+// 15 us.
+constexpr int kFftPassLog = 11;     // stages of a pass: up to 4096 points in two or more columns, 512 threads, 72 KiB
 
-__device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ double2 cmul(double2 a, double2 b)
-{
-    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ __forceinline__ double2 ctimes_i(double2 a) { return make_double2(-a.y, a.x); }
-__device__ __forceinline__ double2 cispi(double x)
-{
-    double2 w;
-    sincospi(x, &w.y, &w.x);
-    return w;
-}
+constexpr double kLightSpeed_cm = 2.99792458e10, kATU = 2.4188843265857e-17;
+constexpr double kADIPMOMU = 8.4783536255e-30, kEPSILON0 = 8.8541878128e-12;
+constexpr double kSfXscale = 1.0 / kLightSpeed_cm / kATU / 2.0 / kPI;
+constexpr double kSfYscale = kATU * kADIPMOMU * kADIPMOMU / (4.0 * kPI * kEPSILON0);
 
-// backward transforms (e^{+i}) of 2, 4 and 8 points, in place
-__device__ __forceinline__ void dft4(double2& a, double2& b, double2& c, double2& d)
+// nu_k, and the Connes apodization of the input in place, as the reference does (src/hawaii.c:5581): for
+// the last pass, when nobody reads cf any more
+__device__ __forceinline__ void sf_axis(double* cf, double* nu, long k, double dt, double tmax, double itmax)
 {
-    const double2 s = cadd(a, c), t = csub(a, c), u = cadd(b, d), v = ctimes_i(csub(b, d));
-    a = cadd(s, u);
-    b = cadd(t, v);
-    c = csub(s, u);
-    d = csub(t, v);
+    const double r = divide<double>(dt * k, tmax, itmax);
+    cf[k] *= (1.0 - r * r) * (1.0 - r * r);
+    nu[k] = divide<double>(k * kPI, tmax, itmax) * kSfXscale;
 }
 
-__device__ __forceinline__ void dft8(double2* v)
+// One radix-2 butterfly with the root e^{i pi k/half}: a + w b, a - w b
+__device__ __forceinline__ void butterfly(double2& a, double2& b, double k_over_half)
 {
-    double2 e[4], o[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        e[i] = cadd(v[i], v[i + 4]);
-        o[i] = csub(v[i], v[i + 4]);
-    }
-    o[1] = make_double2((o[1].x - o[1].y) * kSqrtHalf, (o[1].x + o[1].y) * kSqrtHalf);
-    o[2] = ctimes_i(o[2]);
-    o[3] = make_double2(-(o[3].x + o[3].y) * kSqrtHalf, (o[3].x - o[3].y) * kSqrtHalf);
-    dft4(e[0], e[1], e[2], e[3]);
-    dft4(o[0], o[1], o[2], o[3]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        v[2 * i] = e[i];
-        v[2 * i + 1] = o[i];
-    }
+    double s, c;
+    sincospi(k_over_half, &s, &c);
+    const double2 wb = make_double2(b.x * c - b.y * s, b.x * s + b.y * c);
+    const double2 u = a;
+    a = make_double2(u.x + wb.x, u.y + wb.y);
+    b = make_double2(u.x - wb.x, u.y - wb.y);
 }
 
-// x (1 - r^2)^2, r = k/n (exact: n is a power of two), the window with its rounding error
-__device__ __forceinline__ double connes(double x, long k, double inv_n)
-{
-    const double r = (double)k * inv_n, p = r * r, f = 1.0 - p;
-    const double fl = (-p - (f - 1.0)) - fma(r, r, -p);
-    const double g = f * f, gl = fma(f, f, -g) + 2.0 * f * fl;
-    return fma(x, g, x * gl);
-}
-
-// One Stockham pass of radix R = 2^logr, after passes of a combined radix 2^logl, for the 2^logc columns
-// of this workgroup.  A thread holds rows q = b + i R/8 of one column.
+// logr radix-2 Stockham stages over M = 2n = 2^logm points, after logl of them, for the 2^logc columns of this
+// workgroup: column j holds in[j + q M/R], R = 2^logr; its outputs are out[g L R + k0 + p L], L = 2^logl,
+// k0 = j % L, g = j / L.  A thread holds rows q = b + i R/8.
 template <bool FIRST, bool LAST>
-__global__ void __launch_bounds__(512) sf_pass_kernel(double* cf, const double2* __restrict__ in,
-                                                       double2* __restrict__ out, double* __restrict__ nu,
-                                                       double* __restrict__ sf, int logn, double dt, int logr, int logl,
-                                                       int logc)
+__global__ void __launch_bounds__(512) sf_stages_kernel(double* cf, const double2* __restrict__ in,
+                                                        double2* __restrict__ out, double* __restrict__ nu,
+                                                        double* __restrict__ sf, int logm, double dt, int logr, int logl,
+                                                        int logc)
 {
     extern __shared__ double2 sm[];
-    const long n = 1L << logn;
+    const long M = 1L << logm, n = M >> 1, L = 1L << logl;
     const int t = threadIdx.x, c = t & ((1 << logc) - 1), b = t >> logc, eighth = 1 << (logr - 3);
-    const int logcols = logn - logr;
-    const long L = 1L << logl;
+    const int logcols = logm - logr;
     // Workgroups go to the eight XCDs in turn: neighbouring tiles, which share cache lines, go to one
-    // (n = 2^20: 42 -> 33 us)
     const long tile = gridDim.x % 8 ? blockIdx.x : (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
-    // a pass's columns j; in the last pass half of a workgroup's columns mirror the other half
-    const int half = 1 << logc >> 1;
-    long j;
-    if (LAST && half)
-        j = c < half ? tile * half + c : (1L << logcols) - 1 - (tile * half + c - half);
-    else
-        j = (tile << logc) + c;
-    const long k0 = j & (L - 1);
-    auto slot = [&](int q, int col) { return ((q + (q >> 3)) << logc) + col; };
+    const long j = (tile << logc) + c, k0 = j & (L - 1);
+    auto slot = [&](int q) { return ((q + (q >> 3)) << logc) + c; };
+    const double tmax = dt * n;
 
     double2 v[8];
-    if constexpr (FIRST) {
-        const double inv_n = 1.0 / (double)n;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const long k = j + ((long)(b + i * eighth) << logcols);
-            const double v0 = connes(cf[k], k, inv_n), v1 = k ? connes(cf[n - k], n - k, inv_n) : 0.0;
-            v[i] = cmul(cispi((double)k * (0.5 * inv_n)), make_double2(v0, -v1));
-        }
-    } else {
-        const double unit = 2.0 / (double)(L << logr);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int q = b + i * eighth;
-            v[i] = cmul(in[j + ((long)q << logcols)], cispi((double)(q * k0) * unit));
+    for (int i = 0; i < 8; ++i) {
+        const long k = j + ((long)(b + i * eighth) << logcols);
+        if constexpr (FIRST) {
+            // the packed sequence: v_k e^{i pi k/2n}, 0 at n, -v_{2n-k} e^{i pi k/2n}
+            const double inv2n = 1.0 / (2.0 * n);
+            const long kk = k < n ? k : 2 * n - k;
+            const double tc = dt * kk, r = tc / tmax;
+            double x = 0.0;
+            if (k != n) x = cf[kk] * ((1.0 - r * r) * (1.0 - r * r));
+            if (k > n) x = -x;
+            double sn, cs;
+            sincospi((double)k / (2.0 * n), &sn, &cs);
+            v[i] = make_double2(x * cs * inv2n, x * sn * inv2n);
+        } else {
+            v[i] = in[k];
         }
     }
-    // the roots e^{2 pi i q / R} of the steps
-    double2* root = sm + ((1 << logr) + (1 << (logr - 3)) << logc);
-    const double rel = 2.0 / (double)(1 << logr);
-    for (int q = t; q < 1 << logr; q += blockDim.x) root[q] = cispi((double)q * rel);
 
+    // a stage over the pairs of local position k' with `half` = 2^lg local, L 2^lg global: root (k0 + k' L) / (L 2^lg)
+    auto root = [&](int kp, int lg) { return (double)(k0 + ((long)kp << logl)) * (1.0 / (double)(L << lg)); };
     for (int lg = 0;;) {
         const int rest = logr - lg;
         if (rest >= 3) {
-            if (lg) {
-                const int k = (b & ((1 << lg) - 1)) << (logr - lg - 3);
+            const int k = b & ((1 << lg) - 1), l = 1 << lg;
+            const double ra = root(k, lg), rb0 = root(k, lg + 1), rb1 = root(k + l, lg + 1);
 #pragma unroll
-                for (int i = 1; i < 8; ++i) v[i] = cmul(v[i], root[i * k]);
+            for (int i = 0; i < 4; ++i) butterfly(v[i], v[i + 4], ra);
+            // v[i]: first output of pair i, v[i + 4]: second (k' + l)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                butterfly(v[i], v[i + 2], rb0);
+                butterfly(v[i + 4], v[i + 6], rb1);
             }
-            dft8(v);
+            butterfly(v[0], v[1], root(k, lg + 2));
+            butterfly(v[4], v[5], root(k + l, lg + 2));
+            butterfly(v[2], v[3], root(k + 2 * l, lg + 2));
+            butterfly(v[6], v[7], root(k + 3 * l, lg + 2));
+            // output s = u + 2 w + 4 x is at v[4 u + 2 w + x]
+            double2 o[8];
+#pragma unroll
+            for (int s = 0; s < 8; ++s) o[s] = v[4 * (s & 1) + 2 * ((s >> 1) & 1) + (s >> 2)];
+#pragma unroll
+            for (int s = 0; s < 8; ++s) v[s] = o[s];
             if (rest == 3) break;
         } else {
-            // radix 4 or 2: butterflies of the rows b + u R/8
             if (rest == 2) {
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
-#pragma unroll
-                    for (int i = 1; i < 4; ++i) v[2 * i + u] = cmul(v[2 * i + u], root[i * (b + u * eighth)]);
-                    dft4(v[u], v[2 + u], v[4 + u], v[6 + u]);
+                    const int k = b + u * eighth, l = 1 << lg;
+                    double2 &e0 = v[u], &e1 = v[2 + u], &e2 = v[4 + u], &e3 = v[6 + u];
+                    const double ra = root(k, lg);
+                    butterfly(e0, e2, ra);
+                    butterfly(e1, e3, ra);
+                    butterfly(e0, e1, root(k, lg + 1));
+                    butterfly(e2, e3, root(k + l, lg + 1));
+                    const double2 x = e1;   // outputs 0, 2, 1, 3
+                    e1 = e2;
+                    e2 = x;
                 }
             } else {
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const double2 x = cmul(v[4 + u], root[b + u * eighth]);
-                    v[4 + u] = csub(v[u], x);
-                    v[u] = cadd(v[u], x);
-                }
+                for (int u = 0; u < 4; ++u) butterfly(v[u], v[4 + u], root(b + u * eighth, lg));
             }
             break;
         }
         const int k = b & ((1 << lg) - 1), g = b >> lg;
         if (lg) __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 8; ++i) sm[slot((g << (lg + 3)) + k + (i << lg), c)] = v[i];
+        for (int i = 0; i < 8; ++i) sm[slot((g << (lg + 3)) + k + (i << lg))] = v[i];
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = sm[slot(b + i * eighth, c)];
+        for (int i = 0; i < 8; ++i) v[i] = sm[slot(b + i * eighth)];
         lg += 3;
     }
 
@@ -185,104 +161,68 @@ __global__ void __launch_bounds__(512) sf_pass_kernel(double* cf, const double2*
 #pragma unroll
         for (int i = 0; i < 8; ++i) out[o + ((long)(b + i * eighth) << logl)] = v[i];
     } else {
-        __syncthreads();
+        const double tm = n * dt;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) sm[slot(b + i * eighth, c)] = v[i];
-        __syncthreads();
-        const double LightSpeed_cm = 2.99792458e10, ATU = 2.4188843265857e-17;
-        const double ADIPMOMU = 8.4783536255e-30, EPSILON0 = 8.8541878128e-12;
-        const double Xscale = 1.0 / LightSpeed_cm / ATU / 2.0 / kPI;
-        const double Yscale = ATU * ADIPMOMU * ADIPMOMU / (4.0 * kPI * EPSILON0);
-        const double tmax = n * dt;
-        // tmax / pi * Yscale / 2n with its rounding error
-        const double q0 = tmax / kPI, q1 = fma(-q0, kPI, tmax) / kPI, inv2n = 0.5 / n;
-        const double s0 = q0 * Yscale * inv2n, s1 = (fma(q0, Yscale, -(q0 * Yscale)) + q1 * Yscale) * inv2n;
-        auto scaled = [&](double x) { return fma(x, s0, x * s1); };
+        for (int i = 0; i < 4; ++i)   // the first n outputs: rows below R/2
+            sf[k0 + ((long)(b + i * eighth) << logl)] = v[i].x * tm / kPI * kSfYscale;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int e = t + i * blockDim.x;
-            const int col = half ? e & (half - 1) : 0, q = half ? e >> (logc - 1) : e;
-            long m = (half ? tile * half + col : 0) + ((long)q << logl);
-            double y = sm[slot(q, col)].x, ym = sm[slot((1 << logr) - 1 - q, half + col)].x;
-            if (m >= n / 2) {
-                m = n - 1 - m;
-                const double s = y;
-                y = ym;
-                ym = s;
-            }
-            sf[2 * m] = scaled(y);
-            sf[2 * m + 1] = scaled(ym);
-        }
-        const double itmax = recip<double>(tmax);
-#pragma unroll 4
-        for (int i = 0; i < 8; ++i) {
-            const long k = ((long)blockIdx.x * 8 + i) * blockDim.x + t;
-            // Connes apodization of the input in place, as the reference does (src/hawaii.c:5581): no
-            // workgroup reads cf any more
-            const double r = divide<double>(dt * k, tmax, itmax);
-            cf[k] *= (1.0 - r * r) * (1.0 - r * r);
-            nu[k] = divide<double>(k * kPI, tmax, itmax) * Xscale;
-        }
+        for (int i = 0; i < 4; ++i)
+            sf_axis(cf, nu, ((long)blockIdx.x * 4 + i) * blockDim.x + t, dt, tm, recip<double>(tm));
     }
 }
 
-// n = 2, 4: the cosine sum itself
+// n = 2: the cosine sum itself
 __global__ void __launch_bounds__(64) sf_direct_kernel(double* cf, double* __restrict__ nu, double* __restrict__ sf,
-                                                       int n, double dt)
+                                                       double dt)
 {
     const int j = threadIdx.x;
-    double x[4], acc = 0.0;
-    for (int k = 0; k < n; ++k) x[k] = cf[k];
+    const double x0 = cf[0], x1 = cf[1] * (0.75 * 0.75);   // the window at r = 0, 1/2
     __syncthreads();
-    if (j >= n) return;
-    for (int k = 0; k < n; ++k)
-        acc += (k ? 2.0 : 1.0) * connes(x[k], k, 1.0 / n) * cospi((double)(k * (2 * j + 1)) / (2.0 * n));
-    const double LightSpeed_cm = 2.99792458e10, ATU = 2.4188843265857e-17;
-    const double ADIPMOMU = 8.4783536255e-30, EPSILON0 = 8.8541878128e-12;
-    const double Xscale = 1.0 / LightSpeed_cm / ATU / 2.0 / kPI;
-    const double Yscale = ATU * ADIPMOMU * ADIPMOMU / (4.0 * kPI * EPSILON0);
-    const double tmax = n * dt, r = (dt * j) / (dt * n);
-    cf[j] *= (1.0 - r * r) * (1.0 - r * r);
-    nu[j] = j * kPI / tmax * Xscale;
-    sf[j] = acc * (tmax / kPI * Yscale / (2.0 * n));
+    if (j >= 2) return;
+    const double tmax = 2 * dt, c = 2.0 * x1 * cospi(0.25 * (2 * j + 1));
+    sf[j] = 0.25 * (x0 + c) * tmax / kPI * kSfYscale;
+    sf_axis(cf, nu, j, dt, tmax, recip<double>(tmax));
 }
 
-// Global passes of a transform of 2^logn points: as many as it takes at 2^kFftPassLog points each
-int sf_passes(int logn) { return logn <= kFftSingleLog ? 1 : (logn + kFftPassLog - 1) / kFftPassLog; }
+// Passes of the 2^logm-point transform: as many as it takes at 2^kFftPassLog points each
+int sf_passes(int logm) { return (logm + kFftPassLog - 1) / kFftPassLog; }
+
+int sf_log(long m)
+{
+    int l = 0;
+    while ((1L << l) < m) ++l;
+    return l;
+}
 
 size_t sf_work_bytes(long n, int which)
 {
-    int logn = 0;
-    while ((1L << logn) < n) ++logn;
-    return sf_passes(logn) > 1 + which ? (size_t)n * sizeof(double2) : 0;
+    return sf_passes(sf_log(2 * n)) > 1 + which ? (size_t)(2 * n) * sizeof(double2) : 0;
 }
 
 hipError_t run_cf_to_sf(double* cf, long n, double dt, double2* work_a, double2* work_b, double* nu, double* sf,
                         hipStream_t st)
 {
-    int logn = 0;
-    while ((1L << logn) < n) ++logn;
-    if (n <= 4) {
-        hipLaunchKernelGGL(sf_direct_kernel, dim3(1), dim3(64), 0, st, cf, nu, sf, (int)n, dt);
+    if (n == 2) {
+        hipLaunchKernelGGL(sf_direct_kernel, dim3(1), dim3(64), 0, st, cf, nu, sf, dt);
         return hipGetLastError();
     }
-    const int passes = sf_passes(logn);
+    const int logm = sf_log(2 * n), passes = sf_passes(logm);
     double2 *src = work_b, *dst = work_a;
     int logl = 0;
     for (int p = 0; p < passes; ++p) {
-        const int logr = (logn - logl + passes - p - 1) / (passes - p), logc = passes == 1 ? 0 : kFftColsLog;
+        const int logr = (logm - logl + passes - p - 1) / (passes - p);
+        const int logc = passes == 1 ? 0 : (logr == kFftPassLog ? 1 : 2);
         const bool first = p == 0, last = p == passes - 1;
-        auto k = first ? (last ? sf_pass_kernel<true, true> : sf_pass_kernel<true, false>)
-                       : (last ? sf_pass_kernel<false, true> : sf_pass_kernel<false, false>);
+        auto k = first ? (last ? sf_stages_kernel<true, true> : sf_stages_kernel<true, false>)
+                       : (last ? sf_stages_kernel<false, true> : sf_stages_kernel<false, false>);
         const int points = 1 << (logr + logc);
-        const size_t lds = (size_t)(points + points / 8 + (1 << logr)) * sizeof(double2);
+        const size_t lds = (size_t)(points + points / 8) * sizeof(double2);
         if (lds > 65536) {
-            const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                     (int)lds);
+            const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             if (e != hipSuccess) return e;
         }
-        hipLaunchKernelGGL(k, dim3((unsigned)(n >> (logr + logc))), dim3(points / 8), lds, st, cf, src, dst, nu,
-                           sf, logn, dt, logr, logl, logc);
+        hipLaunchKernelGGL(k, dim3((unsigned)(2 * n >> (logr + logc))), dim3(points / 8), lds, st, cf, src, dst, nu, sf,
+                           logm, dt, logr, logl, logc);
         logl += logr;
         double2* x = src;
         src = dst;
@@ -292,13 +232,13 @@ hipError_t run_cf_to_sf(double* cf, long n, double dt, double2* work_a, double2*
 }
 
 // ------------------------------------------------------------------ CF -> SF without allocation
-// The n-point work sequence of the transform lives in a file-scope device array instead of an
+// The 2n-point work sequence of the transform lives in a file-scope device array instead of an
 // engine-allocated buffer, for callers that cannot allocate (graph capture, tight serving loops).
 // Every device holds its own copy; its address comes from hipGetSymbolAddress once per device
 // (noalloc_scratch_address, at engine creation) and only that address is passed to kernels: the
 // array's name in host code is a host-side stand-in, not a device address.  Calls that overlap on
 // one device share the array and race.
-__device__ __align__(256) double2 scratch[kCfToSfNoAllocMaxN];
+__device__ __align__(256) double2 scratch[2 * kCfToSfNoAllocMaxN];
 
 hipError_t noalloc_scratch_address(void** ptr)
 {

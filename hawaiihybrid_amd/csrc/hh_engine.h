@@ -41,8 +41,8 @@ __host__ __device__ __forceinline__ bool dropped(int first, int last)
 // Rcut sphere, the squared impact parameter, and the transit time with a marked front tier.
 enum OrderKey : int { ORDER_TRANSIT_KEY = 0, ORDER_IMPACT_KEY = 1, ORDER_TIERED_KEY = 2 };
 
-// hh_cf_to_sf_noalloc: the largest transform length its static work array holds (an
-// n-point complex FP64 sequence: 1 MiB per device)
+// hh_cf_to_sf_noalloc: the largest transform length its static work array holds (a
+// 2n-point complex FP64 sequence: 2 MiB per device)
 constexpr long kCfToSfNoAllocMaxN = 65536;
 
 // One correlation-function job: a batch of trajectories sharing system, temperature-free

@@ -8,7 +8,9 @@
 //   * launches the ensemble reduction of every job whose items have all finished, so a job's
 //     CF does not wait for the slowest trajectory of other jobs,
 //   * repacks the slots once the queue is drained, spreading the remaining items over all
-//     wavefronts so the long tail of the ensemble runs with little divergence.
+//     wavefronts so the long tail of the ensemble runs with little divergence,
+//   * and runs the slices of a pool with a few thousand items left on the row kernel (a
+//     trajectory per 16 lanes, hh_rows.hip), which ends a long trajectory sooner.
 // Every item's arithmetic is independent of the slice boundaries and of its neighbours, and
 // each job's reduction has a fixed order, so a job's CF is the same bits alone or in a mix.
 #include <algorithm>
@@ -297,7 +299,8 @@ SysConst pool_sysconst(const hh_engine* e, const LanePool& pl) { return sysconst
 // the lane kernel still gains from every lane that is filled: measured on whole calls with limits of
 // 0, 1024, 2048, 4096 and 8192 items, 1153 CO2-Ar trajectories in FP64 take 45.3, 24.1, 23.3, 22.9 and
 // 21.7 ms, 65536 mixed ones (their tail) 282, 185, 182, 184 and 170 ms, 12289 CH4-CO2 ones 356, 266,
-// 238, 225 and 208 ms, 4096 He-Ar ones 7.7, 6.0, 5.5, 4.2 and 4.3 ms.
+// 238, 225 and 208 ms, 4096 He-Ar ones 7.7, 6.0, 5.5, 4.2 and 4.3 ms (with the row kernel's first form;
+// its later ones are faster still).
 //
 // A mixed pool whose orbiting items go to an FP64 pool takes half of that, one wavefront per SIMD: two
 // fill the register file, and the FP64 pool's rows, which hold the longest trajectories, would wait for
@@ -375,7 +378,7 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
 {
     if (progress) *progress = false;
     static const bool trace = std::getenv("HH_POOL_TRACE") != nullptr;   // progress lines on stderr
-    // 1. one slice of every pool with items in flight, each pool on its own stream so the
+    // 1. one slice of every pool with items in flight, each pool on a stream of the step so the
     //    slices of different pools share the device
     std::vector<LanePool*> run;
     for (auto& pp : set) {

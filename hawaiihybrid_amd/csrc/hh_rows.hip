@@ -17,7 +17,8 @@
 //
 // Bound: a lone wavefront's instruction issue (one in 4.4 cycles).  1153 CO2-Ar trajectories in FP64
 // (L = 1024): 42 ms on the lane kernel, 21 ms with every lane evaluating both series of a sincos and
-// all components, 17 ms in this form; 4096 He-Ar ones (L = 2048) 7.4, 4.2 and 3.9 ms.
+// all components, 18 ms in this form with the stages in a loop and 15 with them unrolled; 4096 He-Ar
+// ones (L = 2048) 7.4, 4.4, 4.2 and 3.3 ms.
 #include <hip/hip_runtime.h>
 
 #include <utility>

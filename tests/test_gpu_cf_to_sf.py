@@ -1,6 +1,6 @@
-"""CF -> SF at the edges of the transform's dispatch: the direct sum (n <= 4), one workgroup (its
-last step of radix 2, 4 and 8, from 16 points up to its largest), two passes at their smallest and
-largest, three passes.  Against the cosine transform in long double.
+"""CF -> SF at the edges of the transform's dispatch: the direct sum (n = 2), one pass from its
+smallest to its largest, with a last step of one, two and three stages, two passes at their smallest
+and largest, three passes.  Against the cosine transform in long double.
 
 A radix transform's error in the 2-norm is at most about (3 + 1) eps per doubling (a product with a
 rounded root, an addition); the bound below adds the input's window and the scaling, 8 eps."""
@@ -20,7 +20,7 @@ def eng():
     e.close()
 
 
-@pytest.mark.parametrize("logn", [1, 2, 3, 4, 5, 6, 11, 12, 13, 14, 16, 20, 21])
+@pytest.mark.parametrize("logn", [1, 2, 3, 4, 5, 9, 10, 11, 12, 13, 16, 20, 21, 22])
 def test_cf_to_sf_against_long_double(eng, logn):
     n, dt = 1 << logn, 200.0
     rng = np.random.default_rng(logn)
