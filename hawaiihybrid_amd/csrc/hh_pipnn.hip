@@ -20,8 +20,8 @@
 //
 // Every network is evaluated as a deviation from its value at the reference point where all
 // polynomials vanish (infinite separation; QModel::forward_inf): with x = (p - mean)/scale and
-// x_ref = -mean/scale, the first layer takes dx = p/scale (the dipole's p, with 1/scale in its
-// weights) and starts its accumulator from
+// x_ref = -mean/scale, the first layer takes dx = p/scale (in the dipole's split mode p, with
+// 1/scale in its weights) and starts its accumulator from
 // z_ref = W^T x_ref + b, each hidden layer passes dh = act(z) - act(z_ref), and the last layer
 // yields d(out) = out - out_ref directly.  The references are computed once on the host in FP64.
 // The BF16 operands then carry only the deviations, so their rounding scales with the signal
@@ -232,7 +232,8 @@ struct PesDev {
 };
 
 struct DipModelDev {
-    LayerDev L1, L2;        // 308 -> 40 (2 n-tiles, 20 k-blocks; the weights hold 1 / scale), 40 -> 5 (1, 3)
+    LayerDev L1, L2;        // 308 -> 40 (2 n-tiles, 20 k-blocks), 40 -> 5 (1 n-tile, 3 k-blocks)
+    const float* xinv;      // [320] 1 / scale; in the split mode L1's weights hold it
     double inv_a0;
     float y2a, yr2a;        // exp(-2a / a0), exp(-sqrt(2) a / a0)
 };
@@ -348,6 +349,12 @@ __global__ __launch_bounds__(64, 2) void pipnn_dip_kernel(DipDev d, const double
         for (int kb = 0; kb < 20; ++kb) {
             float p[16];
             pip_n2ar_dip_block<float>(kb, y, p);
+            if constexpr (!SPLIT) {
+                // one BF16 product: which weights round well decides the far dipole's error (with the scale
+                // in them its 99th percentile doubles), so they stay the network's
+#pragma unroll
+                for (int e = 0; e < 16; ++e) p[e] *= M.xinv[16 * kb + e];
+            }
             // lane l holds its point's features 0..7 and 8..15; swapped between the half-wavefronts they are
             // the operands of points 0..31 and 32..63
             u32x4 bh[2], bl[2];
@@ -573,6 +580,7 @@ int hh_pipnn_create(hh_engine* e, const hh_pipnn_desc* d, int precision, hh_pipn
     // dipole: subnets merged block-diagonally; layer 1 308 (pad 320) -> 40 (pad 64),
     // layer 2 40 (pad 48) -> 5 (pad 32)
     StagedLayer dl[2][2] = {};
+    size_t dxi[2] = {0, 0};
     if (has_dip) {
         for (int m = 0; m < 2; ++m) {
             std::vector<double> W1T((size_t)64 * 320, 0.0), W2T((size_t)32 * 48, 0.0), b1(64, 0.0), b2(32, 0.0);
@@ -594,8 +602,12 @@ int hh_pipnn_create(hh_engine* e, const hh_pipnn_desc* d, int precision, hh_pipn
             std::vector<double> xref(320, 0.0);
             for (int k = 0; k < kPipDip; ++k) xref[k] = -d->dip_xmean[m][k] / d->dip_xscale[m][k];
             const std::vector<double> z1 = affine(W1T, 64, 320, xref, b1);
-            for (int j = 0; j < 64; ++j)
-                for (int k = 0; k < kPipDip; ++k) W1T[(size_t)j * 320 + k] /= d->dip_xscale[m][k];
+            if (precision == HH_MLP_BF16X3)
+                for (int j = 0; j < 64; ++j)
+                    for (int k = 0; k < kPipDip; ++k) W1T[(size_t)j * 320 + k] /= d->dip_xscale[m][k];
+            std::vector<float> di(320, 0.0f);
+            for (int k = 0; k < kPipDip; ++k) di[k] = (float)(1.0 / d->dip_xscale[m][k]);
+            dxi[m] = stage(blob, di.data(), di.size() * 4);
             dl[m][0] = stage_layer(blob, W1T, 64, 320, false, z1, false, HH_ACT_SILU);
             dl[m][1] = stage_layer(blob, W2T, 32, 48, true, std::vector<double>(32, 0.0), true, HH_ACT_SILU);
         }
@@ -633,6 +645,7 @@ int hh_pipnn_create(hh_engine* e, const hh_pipnn_desc* d, int precision, hh_pipn
             M->dip.m[m].L1 = view(dl[m][0]);
             M->dip.m[m].L2 = view(dl[m][1]);
             const double a = 0.5 * kLN2, a0 = m == 0 ? 2.0 : 6.0;
+            M->dip.m[m].xinv = reinterpret_cast<const float*>(base + dxi[m]);
             M->dip.m[m].inv_a0 = 1.0 / a0;
             M->dip.m[m].y2a = (float)std::exp(-2.0 * a / a0);
             M->dip.m[m].yr2a = (float)std::exp(-std::sqrt(2.0) * a / a0);
