@@ -20,8 +20,7 @@
 //
 // Every network is evaluated as a deviation from its value at the reference point where all
 // polynomials vanish (infinite separation; QModel::forward_inf): with x = (p - mean)/scale and
-// x_ref = -mean/scale, the first layer takes dx = p/scale (in the dipole's split mode p, with
-// 1/scale in its weights) and starts its accumulator from
+// x_ref = -mean/scale, the first layer takes dx = p/scale and starts its accumulator from
 // z_ref = W^T x_ref + b, each hidden layer passes dh = act(z) - act(z_ref), and the last layer
 // yields d(out) = out - out_ref directly.  The references are computed once on the host in FP64.
 // The BF16 operands then carry only the deviations, so their rounding scales with the signal
@@ -210,10 +209,13 @@ __device__ __forceinline__ void pes_variables(const Frame& f, float* y)
 // dipole sites (xyz4q_from_bf): N1 (as, 0, ac), N2 = -N1, N1' (ac, 0, -as), N2' = -N1', Ar (0, 0, R), with
 // as = a sin(theta_m), ac = a cos(theta_m).  The variables exp(-r_ij / a0), i < j, are those of two fixed
 // distances (N1-N2 and N1'-N2' 2a, the others sqrt(2) a: the host's, in the model) and of the four to Ar.
-__device__ __forceinline__ void dipole_variables(double as, double ac, double R, double inv_a0, float y2a, float yr2a,
+__device__ __forceinline__ void dipole_variables(double as, double ac, double R, double a0, float y2a, float yr2a,
                                                  float* y)
 {
-    auto v = [&](double x, double z) { return (float)exp(-sqrt(x * x + (z - R) * (z - R)) * inv_a0); };
+    auto v = [&](double x, double z) {
+        const double dx = x, dz = z - R;
+        return (float)exp(-sqrt(dx * dx + dz * dz) / a0);
+    };
     y[0] = y[7] = y2a;
     y[1] = y[2] = y[4] = y[5] = yr2a;
     y[3] = v(as, ac);
@@ -233,8 +235,8 @@ struct PesDev {
 
 struct DipModelDev {
     LayerDev L1, L2;        // 308 -> 40 (2 n-tiles, 20 k-blocks), 40 -> 5 (1 n-tile, 3 k-blocks)
-    const float* xinv;      // [320] 1 / scale; in the split mode L1's weights hold it
-    double inv_a0;
+    const float* xinv;      // [320] 1 / scale
+    double a0;
     float y2a, yr2a;        // exp(-2a / a0), exp(-sqrt(2) a / a0)
 };
 struct DipDev {
@@ -319,11 +321,12 @@ __global__ __launch_bounds__(64) void pipnn_pes_kernel(PesDev<NH + 1> m, const d
 
 // ------------------------------------------------------------------ dipole kernel
 // Bound by vector instructions: 2 x 308 polynomials a point, their conversion to BF16 and 40 SiLUs a
-// model, beside 8000 matrix-core cycles a wavefront.  So the conversion is the hardware's, the scale is in
-// the weights, the distances inside the molecule are constants, the operands change lanes in registers, and
-// the k-blocks are unrolled (they share products of the variables; in a loop over a switch they need 30
-// spilled registers more).  2^20 points in the split mode, both kernels: 920 -> 240 us.  Two wavefronts
-// per SIMD; three (168 registers, 92 spilled) take 390 us.
+// model, beside 8000 matrix-core cycles a wavefront.  So the conversion is the hardware's, the distances
+// inside the molecule are constants, the operands change lanes in registers, and the k-blocks are unrolled
+// (they share products of the variables; in a loop over a switch they need 30 spilled registers more).  2^20
+// points in the split mode, both kernels: 920 -> 290 us, the same bits.  With 1/scale in the weights instead
+// of a product per feature 260 us, but other operands are rounded then and the dipoles move by 1.5e-3 of
+// their 2-norm.  Two wavefronts per SIMD; three spill.
 template <int SPLIT>
 __global__ __launch_bounds__(64, 2) void pipnn_dip_kernel(DipDev d, const double* __restrict__ q, long n,
                                                           double* __restrict__ mu)
@@ -341,7 +344,7 @@ __global__ __launch_bounds__(64, 2) void pipnn_dip_kernel(DipDev d, const double
     for (int model = 0; model < 2; ++model) {
         const DipModelDev& M = d.m[model];
         float y[10];
-        dipole_variables(as, ac, f.R, M.inv_a0, M.y2a, M.yr2a, y);
+        dipole_variables(as, ac, f.R, M.a0, M.y2a, M.yr2a, y);
         f32x16 acc[2][2];
         bias_init<2>(M.L1.bias, acc[0], lane);
         bias_init<2>(M.L1.bias, acc[1], lane);
@@ -349,12 +352,8 @@ __global__ __launch_bounds__(64, 2) void pipnn_dip_kernel(DipDev d, const double
         for (int kb = 0; kb < 20; ++kb) {
             float p[16];
             pip_n2ar_dip_block<float>(kb, y, p);
-            if constexpr (!SPLIT) {
-                // one BF16 product: which weights round well decides the far dipole's error (with the scale
-                // in them its 99th percentile doubles), so they stay the network's
 #pragma unroll
-                for (int e = 0; e < 16; ++e) p[e] *= M.xinv[16 * kb + e];
-            }
+            for (int e = 0; e < 16; ++e) p[e] *= M.xinv[16 * kb + e];
             // lane l holds its point's features 0..7 and 8..15; swapped between the half-wavefronts they are
             // the operands of points 0..31 and 32..63
             u32x4 bh[2], bl[2];
@@ -387,10 +386,18 @@ __global__ __launch_bounds__(64, 2) void pipnn_dip_kernel(DipDev d, const double
         }
         __syncthreads();
         {
-            const double q0 = qs[lane][0], q1 = qs[lane][1], q2 = qs[lane][2], q3 = qs[lane][3], q4 = qs[lane][4];
+            // the charges at their sites
+            const double X[5] = {as, -as, ac, -ac, 0.0}, Z[5] = {ac, -ac, -as, as, f.R};
+            double ax = 0.0, az = 0.0;
+#pragma unroll
+            for (int a = 0; a < 5; ++a) {
+                const double dq = (double)qs[lane][a];
+                ax += dq * X[a];
+                az += dq * Z[a];
+            }
             const double wm = model == 0 ? 1.0 - w : w;
-            dx += wm * ((q0 - q1) * as + (q2 - q3) * ac);
-            dz += wm * ((q0 - q1) * ac - (q2 - q3) * as + q4 * f.R);
+            dx += wm * ax;
+            dz += wm * az;
         }
         __syncthreads();
     }
@@ -602,9 +609,6 @@ int hh_pipnn_create(hh_engine* e, const hh_pipnn_desc* d, int precision, hh_pipn
             std::vector<double> xref(320, 0.0);
             for (int k = 0; k < kPipDip; ++k) xref[k] = -d->dip_xmean[m][k] / d->dip_xscale[m][k];
             const std::vector<double> z1 = affine(W1T, 64, 320, xref, b1);
-            if (precision == HH_MLP_BF16X3)
-                for (int j = 0; j < 64; ++j)
-                    for (int k = 0; k < kPipDip; ++k) W1T[(size_t)j * 320 + k] /= d->dip_xscale[m][k];
             std::vector<float> di(320, 0.0f);
             for (int k = 0; k < kPipDip; ++k) di[k] = (float)(1.0 / d->dip_xscale[m][k]);
             dxi[m] = stage(blob, di.data(), di.size() * 4);
@@ -646,7 +650,7 @@ int hh_pipnn_create(hh_engine* e, const hh_pipnn_desc* d, int precision, hh_pipn
             M->dip.m[m].L2 = view(dl[m][1]);
             const double a = 0.5 * kLN2, a0 = m == 0 ? 2.0 : 6.0;
             M->dip.m[m].xinv = reinterpret_cast<const float*>(base + dxi[m]);
-            M->dip.m[m].inv_a0 = 1.0 / a0;
+            M->dip.m[m].a0 = a0;
             M->dip.m[m].y2a = (float)std::exp(-2.0 * a / a0);
             M->dip.m[m].yr2a = (float)std::exp(-std::sqrt(2.0) * a / a0);
         }

@@ -50,6 +50,13 @@ DIP_REPS = [
     "148 139 138 137 136 135 134 128 126 123 089 078 038 037 036 019 018 016 013 889 788 778 388 377 338 "
     "337 336 199 188 166 133 119 118 116 113 088 033 008 003 888 333",
 ]
+# The dipole polynomials are rounded to BF16 pairs on the device, so an ulp in a few of them moves the dipoles by
+# 2e-5 of their 2-norm: their operations are written out.  The second product of an orbit is rounded, the
+# first one is added to it and then the others, an FMA each; the polynomials of this list round the first product
+# and add the second.
+DIP_FIRST_ROUNDED = {
+    5, 6, 9, 11, 14, 16, 18, 19, 22, 63, 94, 128, 133, 137, 140, 143, 182, 207, 242, 243, 244, 247, 249, 250,
+    251, 252, 253, 274, 289}
 # atom permutations generating each basis' group
 PES_GENS = [(1, 0, 2)]
 DIP_GENS = [[(0, 1, 3, 2, 4)], [(1, 0, 2, 3, 4)], [(1, 0, 2, 3, 4), (0, 1, 3, 2, 4)]]
@@ -97,7 +104,17 @@ def term(mono):
     return "*".join(f"y[{i}]" for i in mono)
 
 
-def emit_blocks(name, polys, lines):
+def fma_sum(monos, first_rounded):
+    order = [0, 1] if first_rounded else [1, 0]
+    if len(monos[0]) == 1:
+        return " + ".join(term(m) for m in monos)
+    expr = term(monos[order[0]])
+    for i in order[1:] + list(range(2, len(monos))):
+        expr = f"pip_fma({term(monos[i][:-1])}, y[{monos[i][-1]}], {expr})"
+    return expr
+
+
+def emit_blocks(name, polys, lines, first_rounded=None):
     nb = (len(polys) + 15) // 16
     lines.append(f"// {len(polys)} polynomials in {nb} blocks of 16 (zero-padded)")
     lines.append("template <typename T>")
@@ -110,6 +127,8 @@ def emit_blocks(name, polys, lines):
             k = 16 * b + j
             if k < len(polys) and polys[k]:
                 expr = " + ".join(term(m) for m in polys[k])
+                if first_rounded is not None and len(polys[k]) > 1:
+                    expr = fma_sum(polys[k], k in first_rounded)
             else:
                 expr = "T(0)"
             lines.append(f"        p[{j}] = {expr};")
@@ -141,12 +160,15 @@ def write_device_header(path):
         "",
         "namespace hh {",
         "",
+        "HH_PIP_FN float pip_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }",
+        "HH_PIP_FN double pip_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }",
+        "",
         f"constexpr int kPipPes = {len(pes)};",
         f"constexpr int kPipDip = {len(dip)};",
         "",
     ]
     emit_blocks("pip_n2ar_pes_block", pes, lines)
-    emit_blocks("pip_n2ar_dip_block", dip, lines)
+    emit_blocks("pip_n2ar_dip_block", dip, lines, DIP_FIRST_ROUNDED)
     lines.append("}  // namespace hh")
     with open(path, "w") as f:
         f.write("\n".join(lines) + "\n")
