@@ -377,14 +377,15 @@ __device__ __forceinline__ double row_rhs(const SysConst& sc, const RowCtx<SYS, 
         kb = lane == 6 ? irot2 : kb;
         const double coord = p_next * ka * kb;
         // odd lanes: lanes 3 and 9 polar_rate (azimuthal momentum two lanes down, own cosine), lane 5 the
-        // radial rate; lanes 1 and 7 (a cyclic and a surface-driven azimuth) -dV
+        // radial rate; lanes 1 and 7 (a cyclic and a surface-driven azimuth) -dV, whatever the reciprocal of their
+        // azimuth's sine is (at 0 a product with it is no number)
         const double pa = row_move<DOWN2>(y);
         const double i2 = lane == 3 ? is2 : irot2;
         const double pol = pa * pa * t * ka * i2;
-        double num = lane == 5 ? rad : pol;
-        num = (lane == 1 || lane == 7) ? 0.0 : num;
+        const double num = lane == 5 ? rad : pol;
         const double mul = lane == 5 ? iR : rc;
-        const double momentum = num * mul - dV;
+        double momentum = num * mul - dV;
+        momentum = (lane == 1 || lane == 7) ? -dV : momentum;
         return odd ? momentum : coord;
     }
 }

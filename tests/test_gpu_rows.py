@@ -5,7 +5,10 @@ A job alone runs on the row kernel from its first step; beside a filler of 9000 
 the same call it starts on the lane kernel and, depending on its items, ends on either.  Every
 item's row, length, status, right-hand-side count and energy drift, and the job's CF, must be equal
 bit for bit: both kernels run the same expressions in the same order.  Sizes: one row, less and more
-than a wavefront's four rows, more rows than wavefronts."""
+than a wavefront's four rows, more rows than wavefronts.
+
+An engine with graph-captured slices stays on the lane kernel at every size; against it, exact special values
+of the initial conditions."""
 import numpy as np
 import pytest
 
@@ -44,3 +47,43 @@ def test_row_kernel_gives_the_lane_kernel_bits(eng, which, prec, n):
     for key in ("len", "status", "nrhs", "e_drift", "rows"):
         assert np.array_equal(a[key], b[key]), key
     assert np.array_equal(alone[0].cpu().numpy(), beside[0].cpu().numpy())
+
+
+@pytest.fixture(scope="module")
+def lane_eng():
+    mp = pytest.MonkeyPatch()
+    mp.setenv("HH_GRAPHS", "1")   # read at creation
+    e = H.Engine(0)
+    mp.undo()
+    yield e
+    e.close()
+
+
+@pytest.mark.parametrize("which", ["hear", "co2ar", "ch4co2"])
+@pytest.mark.parametrize("prec", [H.PREC_FP64, H.PREC_MIXED])
+def test_angles_of_exactly_zero(eng, lane_eng, which, prec):
+    """Azimuths of exactly 0 or equal to each other, with and without azimuthal momentum (a planar or aligned
+    geometry): their sines are 0, and no equation of motion divides by them."""
+    make, T, pesmin, rmin = SYSTEMS[which]
+    L = 512
+    smp = H.Sampler(H.IC_R0_INJECT, H.PAIR_FREE, T, rmin, 40.0, pesmin, 15.0)
+    ic = H.sample_ics(make(), smp, 7, 8)[0]
+    azimuths = {"hear": [0], "co2ar": [0, 6], "ch4co2": [0, 6, 12]}[which]
+    ic[0:2, 0] = 0.0                    # Phi
+    ic[1, 1] = 0.0
+    for k in azimuths[1:]:
+        ic[2:4, k] = 0.0                # a monomer's azimuth
+        ic[3, k + 1] = 0.0
+        ic[4:6, k] = ic[4:6, 0]         # the same azimuth
+        ic[5, k + 1] = ic[5, 1]
+    ic[6:8, azimuths] = 0.0             # in a plane
+    ic[7, [k + 1 for k in azimuths]] = 0.0
+    p = H.cf_params(L, rtol=1e-10 if prec == H.PREC_MIXED else 1e-12, Rcut=20.0, precision=prec)
+    got = []
+    for e in (eng, lane_eng):
+        e.cf_run(make(), p, [e.to_device_soa(ic)])
+        got.append(e.items(0, 8, L, rows=True))
+    print(f"zero angles {which} prec {prec}: status {got[0]['status']} {got[1]['status']}", flush=True)
+    assert np.all(got[1]["status"] == 0)
+    for key in ("len", "status", "nrhs", "e_drift", "rows"):
+        assert np.array_equal(got[0][key], got[1][key]), key
