@@ -238,10 +238,10 @@ inline SysConst sysconst(const hh_engine* e, const hh_system& sys, bool f32)
     sc.I = sys.I;
     sc.tables = (f32 && sys.system == HH_SYS_CO2AR) ? e->tab32.p : e->tab64.p;
     sc.imu = 1.0 / sys.mu;
-    sc.iI = sys.I != 0.0 ? 1.0 / sys.I : 0.0;
+    sc.iI = 1.0 / sys.I;
     for (int i = 0; i < 3; ++i) {
         sc.IR[i] = sys.I_rotor[i];
-        sc.iIR[i] = sys.I_rotor[i] != 0.0 ? 1.0 / sys.I_rotor[i] : 0.0;
+        sc.iIR[i] = 1.0 / sys.I_rotor[i];
     }
     return sc;
 }

@@ -316,7 +316,7 @@ __device__ __forceinline__ double row_rhs(const SysConst& sc, const RowCtx<SYS, 
             const double x = kHearB * R;
             const double arg = lane == 0 ? -x : -kHearA1 * R - kHearA2 * R * R;
             const double ex = exp(arg);
-            const double dVR = hear_dV_exps(R, bcast<0>(ex), bcast<1>(ex));
+            const double dVR = hear_dV_exps(R, bcast<0>(ex), bcast<1>(ex), sizeof(P) == 8 ? iR : recip<double>(R));
             dV = lane == 5 ? dVR : 0.0;
         } else {
             const Co2ArTables<P>* tb = (const Co2ArTables<P>*)sc.tables;

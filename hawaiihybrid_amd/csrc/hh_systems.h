@@ -61,9 +61,10 @@ __device__ __forceinline__ double rcp_nr(double x)
     return fma(r, e, r);
 }
 
-// The FP64 engines' 1/x: one more residual step rounds to the division's value (the same bits for the
-// well-scaled arguments here: distances, sines, error scales) in 7 instructions instead of the scaled
-// division's 11.
+// The FP64 engines' 1/x: one more residual step rounds to the division's value in 7 instructions and one that
+// puts in the limits (0, infinities, NaN), instead of the scaled division's 11.  Rounding by a residual from a
+// reciprocal within an ulp: Markstein, "Computation of elementary functions on the IBM RISC System/6000
+// processor", IBM J. Res. Dev. 34 (1990).  The same bits for normal x below 2^1022.
 template <typename P>
 __device__ __forceinline__ double recip(double x)
 {
@@ -71,19 +72,21 @@ __device__ __forceinline__ double recip(double x)
     if constexpr (sizeof(P) == 4)
         return r;
     else
-        return fma(fma(-x, r, 1.0), r, r);
+        return __builtin_amdgcn_div_fixup(fma(fma(-x, r, 1.0), r, r), x, 1.0);
 }
 
-// a / b by b's reciprocal r: the division's bits in FP64 (a residual step), a product in the engines
-// with FP32 surfaces
+// a / b by b's reciprocal r: the division's bits in FP64 (a residual step, left out where the quotient is not
+// finite or b is not), a product in the engines with FP32 surfaces
 template <typename P>
 __device__ __forceinline__ double divide(double a, double b, double r)
 {
     const double q = a * r;
     if constexpr (sizeof(P) == 4)
         return q;
-    else
-        return fma(fma(-b, q, a), r, q);
+    else {
+        const double e = fma(-b, q, a);
+        return __builtin_isfinite(e) ? fma(e, r, q) : q;
+    }
 }
 
 // 1/x in the surfaces' precision
@@ -91,7 +94,7 @@ __device__ __forceinline__ double recip_p(double x) { return recip<double>(x); }
 __device__ __forceinline__ float recip_p(float x)
 {
     const float r = __builtin_amdgcn_rcpf(x);
-    return fmaf(fmaf(-x, r, 1.0f), r, r);
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-x, r, 1.0f), r, r), x, 1.0f);
 }
 
 // ------------------------------------------------------------------ He-Ar (PES-IDS/HeAr.h)
@@ -100,13 +103,13 @@ __device__ __forceinline__ float recip_p(float x)
 // engine mode: f_2n cancels to 1e-5 below R ~ 5 bohr, beyond what FP32 can carry.
 constexpr double kHearA = 0.2303058634e2, kHearA1 = 0.163051044e1, kHearA2 = 0.4680016e-1, kHearB = 0.16274792500000e1;
 
-// e = exp(-b R), ea = exp(-a1 R - a2 R^2)
-__device__ __forceinline__ double hear_dV_exps(double R, double e, double ea)
+// e = exp(-b R), ea = exp(-a1 R - a2 R^2), inv = 1/R
+__device__ __forceinline__ double hear_dV_exps(double R, double e, double ea, double inv)
 {
     const double A = kHearA, a1 = kHearA1, a2 = kHearA2, b = kHearB;
     const double C[6] = {0.940835513e1, 0.165523018e3, 0.379715796e4, 0.1165179999e6, 0.466258000e7,
                          0.236861000e9};
-    const double x = b * R, inv = recip<double>(R), inv2 = inv * inv;
+    const double x = b * R, inv2 = inv * inv;
     double term = 1.0, sum = 1.0;
     double dV = A * ea * (-a1 - 2.0 * a2 * R);
     double ip = inv2 * inv2;  // R^-4
@@ -128,7 +131,7 @@ __device__ __forceinline__ double hear_dV_exps(double R, double e, double ea)
 __device__ __forceinline__ double hear_dV(double R)
 {
     const double x = kHearB * R;
-    return hear_dV_exps(R, exp(-x), exp(-kHearA1 * R - kHearA2 * R * R));
+    return hear_dV_exps(R, exp(-x), exp(-kHearA1 * R - kHearA2 * R * R), recip<double>(R));
 }
 
 __device__ __forceinline__ double hear_V(double R)
