@@ -438,20 +438,22 @@ int hh::cf_run(hh_engine* e, const hh_system* sys, const hh_cf_params* p, int nj
         if (!pl->inflight.empty()) return fail(HH_E_BUSY, "lane pool of this class is in use");
         if (njobs > pl->ring_cap) return fail(HH_E_INVALID, "at most %d jobs per call", pl->ring_cap);
         std::vector<hh::PoolJob*> mine;
+        // After an error the pools go with their state: jobs admitted before it are in the queue, whose head
+        // would hand their items out to the next call's jobs, and an orbit pool holds jobs on this call's
+        // buffers.  The next call builds fresh ones.
+        auto drop_pools = [e](int code) {
+            (void)hipStreamSynchronize(e->stream);
+            e->pools.clear();
+            return code;
+        };
         for (int j = 0; j < njobs; ++j) {
             hh::PoolJob* pj = nullptr;
             rc = hh::pool_admit(e, *pl, *p, ic_dev[j], ntraj[j], cf_dev[j], 0, &pj, record);
-            if (rc < 0) {
-                while (!pl->inflight.empty()) pl->inflight.pop_back();
-                return rc;
-            }
+            if (rc < 0) return drop_pools(rc);
             mine.push_back(pj);
         }
         rc = hh::pool_order_group(e, *pl);
-        if (rc < 0) {
-            while (!pl->inflight.empty()) pl->inflight.pop_back();
-            return rc;
-        }
+        if (rc < 0) return drop_pools(rc);
         double kms = 0.0, rms = 0.0;
         int launches = 0;
         const double pool_ms0 = pl->launch_ms;
@@ -466,13 +468,7 @@ int hh::cf_run(hh_engine* e, const hh_system* sys, const hh_cf_params* p, int nj
             rc = hh::pool_step(e, e->pools, 5.0, &kms, &rms, &launches, &progress);
             if (rc == HH_OK && !progress)
                 rc = fail(HH_E_DEVICE, "hh_cf_run: jobs left with no work in flight (internal bookkeeping error)");
-            if (rc < 0) {
-                // drop the pools with their state (the orbit pool holds jobs on this call's
-                // buffers); the next call builds fresh ones
-                (void)hipStreamSynchronize(e->stream);
-                e->pools.clear();
-                return rc;
-            }
+            if (rc < 0) return drop_pools(rc);
         }
         for (hh::PoolJob* pj : mine) {
             e->last_jobs.push_back(pj->jd);

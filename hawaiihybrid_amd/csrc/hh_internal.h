@@ -100,8 +100,10 @@ struct DevBuf {
         hipError_t e = hipMalloc(&p, n);
         if (e == hipSuccess)
             bytes = n;
-        else
+        else {
             p = nullptr;
+            (void)hipGetLastError();   // reported here: the next launch is not the one that failed
+        }
         return e;
     }
     void release()
@@ -167,6 +169,7 @@ struct LanePool {
     std::deque<std::unique_ptr<PoolJob>> inflight;   // sequence order
     long long next_seq = 0;
     unsigned long long total = 0;   // items admitted
+    unsigned long long finished = 0;   // the device's count of finished items, seen after a slice
     bool drained_repacked = false;
     bool live_slots = false;        // a slice has left items in the lane slots
     long long unordered_seq = 0;    // first job not yet ordered (pool_order_group)
@@ -189,7 +192,7 @@ struct LanePool {
     LanePool& operator=(const LanePool&) = delete;
     ~LanePool()
     {
-        if (slice_end) (void)hipEventSynchronize(slice_end);
+        if (stream) (void)hipStreamSynchronize(stream);
         for (auto& g : graphs)
             if (g.exec) (void)hipGraphExecDestroy(g.exec);
         if (h_done) (void)hipHostFree(h_done);

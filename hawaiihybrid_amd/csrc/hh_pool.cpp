@@ -409,11 +409,11 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
             ctl.ring = pl->ring_cap;
             const long long limit = e->use_graphs ? 0 : row_limit(*pl);
             ctl.finished = pl->next.as<unsigned long long>() + 1;
-            ctl.finish_target = limit > 0 && pl->total > (unsigned long long)limit ? pl->total - limit : ~0ull;
             HH_CHECK(hipStreamWaitEvent(pl->stream, e->ev[0], 0));
             long long left = 0;
             for (auto& j : pl->inflight)
                 if (j->state == 0 && !j->items_done) left += j->jd.n_items - j->items_finished;
+            ctl.finish_target = limit > 0 ? pl->finished + (unsigned long long)std::max(left - limit, 0LL) : ~0ull;
             if (left <= limit) {
                 if (pl->live_slots) {
                     HH_CHECK(run_repack(pl->sys, pl->view(pl->cur), pl->view(1 - pl->cur), pl->scratch.as<int>(),
@@ -473,7 +473,10 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
             HH_CHECK(hipMemcpy(done.data() + s0, pl->ring_done.as<int>() + s0, nb, hipMemcpyDeviceToHost));
             if (hands_over(*pl))
                 HH_CHECK(hipMemcpy(orbit.data() + s0, pl->ring_orbit.as<int>() + s0, nb, hipMemcpyDeviceToHost));
-            HH_CHECK(hipMemcpy(&next, pl->next.p, sizeof next, hipMemcpyDeviceToHost));
+            unsigned long long head[2];   // the queue head, the items finished
+            HH_CHECK(hipMemcpy(head, pl->next.p, sizeof head, hipMemcpyDeviceToHost));
+            next = head[0];
+            pl->finished = head[1];
         }
         // lanes that found the queue empty advanced the head past the end; none of those
         // indices was handed out (every admission clamps the device head back to the end)

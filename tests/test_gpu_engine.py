@@ -363,3 +363,27 @@ def test_batched_surfaces_match_oracle(eng, which):
         f = np.zeros(y.shape[1])
         L.orc_rhs(so, O.ptr(np.ascontiguousarray(y[i])), O.ptr(f))
         assert np.allclose(F[:, i], f, rtol=1e-9, atol=1e-15)
+
+
+def test_a_call_that_cannot_be_admitted_leaves_nothing_behind():
+    """A call whose second job does not fit the device is refused after its first job was queued; the calls after
+    it must not see the queued items (their indices lie before every later job's)."""
+    import ctypes as C
+    smp = H.Sampler(H.IC_R0_INJECT, H.PAIR_FREE, 300.0, 4.0, 40.0, H.PESMIN_HEAR, 15.0)
+    ic, _, _ = H.sample_ics(H.he_ar(), smp, 11, 900)
+    p = H.cf_params(256, rtol=1e-12, Rcut=20.0, halves=H.HALVES_FORWARD, engine=H.ENGINE_BATCHED)
+    eng = H.Engine(0)
+    x = eng.to_device_soa(ic)
+    want = eng.cf_run(H.he_ar(), p, [x])[0][0].cpu().numpy()
+    eng.close()
+    eng = H.Engine(0)
+    out = [eng.torch.zeros(256, dtype=eng.torch.float64, device="cuda:0") for _ in range(2)]
+    vp = lambda ts: (C.c_void_p * 2)(*[t.data_ptr() for t in ts])
+    st = H.CFStats()
+    rc = H.lib().hh_cf_run(eng.h, C.byref(H.he_ar()), C.byref(p), 2, vp([x, x]), (C.c_long * 2)(900, 1 << 36), vp(out),
+                           C.byref(st))
+    assert rc < 0   # 2^36 trajectories of 256 samples: 140 TB
+    for _ in range(2):
+        got = eng.cf_run(H.he_ar(), p, [x])[0][0].cpu().numpy()
+        assert np.array_equal(got, want)
+    eng.close()
