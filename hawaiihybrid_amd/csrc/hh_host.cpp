@@ -463,9 +463,9 @@ int hh::cf_run(hh_engine* e, const hh_system* sys, const hh_cf_params* p, int nj
             for (hh::PoolJob* pj : mine) all &= pj->state == 2;
             if (all) break;
             bool progress = false;
-            // 5 ms slices: items handed over to FP64 start that much sooner (65536 mixed CO2-Ar
-            // trajectories take 118, 101, 95 and 97 ms with 20, 10, 5 and 3 ms)
-            rc = hh::pool_step(e, e->pools, 5.0, &kms, &rms, &launches, &progress);
+            // 5 ms slices, but for a deep queue: items handed over to FP64 start that much sooner (65536
+            // mixed CO2-Ar trajectories take 118, 101, 95 and 97 ms with 20, 10, 5 and 3 ms)
+            rc = hh::pool_step(e, e->pools, hh::pool_slice_ms(e->pools), &kms, &rms, &launches, &progress);
             if (rc == HH_OK && !progress)
                 rc = fail(HH_E_DEVICE, "hh_cf_run: jobs left with no work in flight (internal bookkeeping error)");
             if (rc < 0) return drop_pools(rc);

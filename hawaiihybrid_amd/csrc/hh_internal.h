@@ -169,6 +169,7 @@ struct LanePool {
     std::deque<std::unique_ptr<PoolJob>> inflight;   // sequence order
     long long next_seq = 0;
     unsigned long long total = 0;   // items admitted
+    unsigned long long head = 0;       // the queue head, seen after a slice
     unsigned long long finished = 0;   // the device's count of finished items, seen after a slice
     bool drained_repacked = false;
     bool live_slots = false;        // a slice has left items in the lane slots
@@ -279,10 +280,13 @@ int cf_run(hh_engine* e, const hh_system* sys, const hh_cf_params* p, int njobs,
 int pool_order_group(hh_engine* e, LanePool& pl);
 // true when the ring has room for one more job
 bool pool_has_room(const LanePool& pl);
-// one slice of every pool with work (each pool on its own stream, concurrently), then
+// the slice length of a synchronous call: long while a queue is deep
+double pool_slice_ms(const PoolSet& set);
+// one slice of every pool with work, then
 // admission of the items handed over to FP64 as orbit jobs, reductions of the jobs whose items
 // (orbit jobs included) are all done and repacking of drained pools; synchronises the engine
-// stream.  Jobs whose CF is final have state 2 afterwards; their orbit jobs are gone from the
+// stream.  The slices run on three streams of the engine and its main one, dealt out per step: up to
+// four pools at once, from the fifth on two share a stream and run in turn.  Jobs whose CF is final have state 2 afterwards; their orbit jobs are gone from the
 // orbit pool.  kernel_ms / reduce_ms accumulate device time.
 int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, double* reduce_ms,
               int* launches = nullptr, bool* progress = nullptr);

@@ -307,6 +307,25 @@ SysConst pool_sysconst(const hh_engine* e, const LanePool& pl) { return sysconst
 // them (65536 mixed CO2-Ar trajectories: 106 -> 95 ms).
 constexpr long long kRowLimit = 8192;
 
+// A queue of more than three fills of the lane slots: what counts is the rate at which the lane kernel takes
+// the items, and the time of a single trajectory passes beside them.  Then a synchronous call's slices are
+// long (every slice saves and restores all slots, and the host waits), and the FP64 pool of the orbiting items
+// stays on the lane kernel, which takes fewer instructions an item than a row.  Calls of 80, 20, 6 and 3 times
+// 65536 mixed CO2-Ar trajectories (a fill each), slices' device time: in 5 ms slices with the orbiting
+// items on rows throughout 908, 309, 189 and 98 ms; long slices alone 892 and 337 (80 and 20); both 866, 275, 174
+// and 101.  The line at two fills instead: 859, 267, 159 and 115 ms, at four 861, 259, 174 and 100.
+bool queue_deep(const LanePool& pl) { return pl.total - pl.head > 3ull * (unsigned long long)pl.S; }
+
+bool queue_deep(const PoolSet& set)
+{
+    return std::any_of(set.begin(), set.end(), [](const auto& p) { return queue_deep(*p); });
+}
+
+bool only_orbit_jobs(const LanePool& pl)
+{
+    return std::all_of(pl.inflight.begin(), pl.inflight.end(), [](const auto& j) { return j->parent != nullptr; });
+}
+
 bool hands_over(const LanePool& pl) { return pl.mixed && pl.sys != HH_SYS_HEAR; }
 
 long long row_limit(const LanePool& pl)
@@ -373,6 +392,8 @@ int admit_orbit_job(hh_engine* e, PoolSet& set, LanePool& parent_pool, PoolJob& 
 
 }  // namespace
 
+double pool_slice_ms(const PoolSet& set) { return queue_deep(set) ? 20.0 : 5.0; }
+
 int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, double* reduce_ms, int* launches,
               bool* progress)
 {
@@ -399,6 +420,7 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
             if (!st) HH_CHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
             run[k]->stream = st;
         }
+        const bool deep = queue_deep(set);
         for (LanePool* pl : run) {
             PoolCtl ctl{};
             ctl.next = pl->next.as<unsigned long long>();
@@ -407,7 +429,7 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
             ctl.last_seq = pl->inflight.back()->seq;
             ctl.ticks = (long long)(slice_ms * e->wall_khz);
             ctl.ring = pl->ring_cap;
-            const long long limit = e->use_graphs ? 0 : row_limit(*pl);
+            const long long limit = e->use_graphs || (deep && only_orbit_jobs(*pl)) ? 0 : row_limit(*pl);
             ctl.finished = pl->next.as<unsigned long long>() + 1;
             HH_CHECK(hipStreamWaitEvent(pl->stream, e->ev[0], 0));
             long long left = 0;
@@ -481,6 +503,7 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
         // lanes that found the queue empty advanced the head past the end; none of those
         // indices was handed out (every admission clamps the device head back to the end)
         if (next > pl->total) next = pl->total;
+        pl->head = next;
         prog.push_back({pl, next});
         for (auto& jp : pl->inflight) {
             PoolJob& j = *jp;

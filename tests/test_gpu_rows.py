@@ -7,6 +7,9 @@ item's row, length, status, right-hand-side count and energy drift, and the job'
 bit for bit: both kernels run the same expressions in the same order.  Sizes: one row, less and more
 than a wavefront's four rows, more rows than wavefronts.
 
+Beside a queue of more than three fills of the lane slots the orbiting items of a mixed pool stay on the
+FP64 lane kernel: the same bits again.
+
 An engine with graph-captured slices stays on the lane kernel at every size; against it, exact special values
 of the initial conditions."""
 import numpy as np
@@ -87,3 +90,25 @@ def test_angles_of_exactly_zero(eng, lane_eng, which, prec):
     assert np.all(got[1]["status"] == 0)
     for key in ("len", "status", "nrhs", "e_drift", "rows"):
         assert np.array_equal(got[0][key], got[1][key]), key
+
+
+@pytest.mark.parametrize("which", ["co2ar", "ch4co2"])
+def test_orbiting_items_beside_a_deep_queue(eng, which):
+    """The same trajectories in a call of their own (their orbiting ones in FP64 on rows) and in front of a queue
+    of four fills (on the lane kernel while the queue is deep, then on rows)."""
+    make, T, pesmin, rmin = SYSTEMS[which]
+    n, L = 3000, 512
+    smp = H.Sampler(H.IC_R0_INJECT, H.PAIR_FREE, 150.0, rmin, 40.0, pesmin, 15.0)
+    ic = H.sample_ics(make(), smp, 9, n)[0]
+    x = eng.to_device_soa(ic)
+    fill = x.repeat(1, -(-4 * 65536 // n)).contiguous()
+    p = H.cf_params(L, rtol=1e-10, Rcut=20.0, precision=H.PREC_MIXED)
+    alone, st = eng.cf_run(make(), p, [x])
+    a = eng.items(0, n, L, rows=True)
+    beside, std = eng.cf_run(make(), p, [x, fill])
+    b = eng.items(0, n, L, rows=True)
+    print(f"deep {which}: {st.n_orbit} of {n} orbiting, {std.launches} slices", flush=True)
+    assert st.n_orbit > 0
+    for key in ("len", "status", "nrhs", "e_drift", "rows"):
+        assert np.array_equal(a[key], b[key]), key
+    assert np.array_equal(alone[0].cpu().numpy(), beside[0].cpu().numpy())
