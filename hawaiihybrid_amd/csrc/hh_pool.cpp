@@ -328,10 +328,20 @@ bool only_orbit_jobs(const LanePool& pl)
 
 bool hands_over(const LanePool& pl) { return pl.mixed && pl.sys != HH_SYS_HEAR; }
 
-long long row_limit(const LanePool& pl)
+long long row_limit(const hh_engine* e, const PoolSet& set, const LanePool& pl)
 {
+    if (e->use_graphs || (queue_deep(set) && only_orbit_jobs(pl))) return 0;
     const long long lim = std::min(kRowLimit, pl.S / 8);
     return hands_over(pl) ? lim / 2 : lim;
+}
+
+// items in slots or queued
+long long items_left(const LanePool& pl)
+{
+    long long left = 0;
+    for (auto& j : pl.inflight)
+        if (j->state == 0 && !j->items_done) left += j->jd.n_items - j->items_finished;
+    return left;
 }
 
 // The grid for `left` items: one row per wavefront while they fit one wavefront then two per SIMD (a
@@ -420,7 +430,6 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
             if (!st) HH_CHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
             run[k]->stream = st;
         }
-        const bool deep = queue_deep(set);
         for (LanePool* pl : run) {
             PoolCtl ctl{};
             ctl.next = pl->next.as<unsigned long long>();
@@ -429,12 +438,9 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
             ctl.last_seq = pl->inflight.back()->seq;
             ctl.ticks = (long long)(slice_ms * e->wall_khz);
             ctl.ring = pl->ring_cap;
-            const long long limit = e->use_graphs || (deep && only_orbit_jobs(*pl)) ? 0 : row_limit(*pl);
+            const long long limit = row_limit(e, set, *pl), left = items_left(*pl);
             ctl.finished = pl->next.as<unsigned long long>() + 1;
             HH_CHECK(hipStreamWaitEvent(pl->stream, e->ev[0], 0));
-            long long left = 0;
-            for (auto& j : pl->inflight)
-                if (j->state == 0 && !j->items_done) left += j->jd.n_items - j->items_finished;
             ctl.finish_target = limit > 0 ? pl->finished + (unsigned long long)std::max(left - limit, 0LL) : ~0ull;
             if (left <= limit) {
                 if (pl->live_slots) {
@@ -558,7 +564,8 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
         }
     }
     // 4. repacking: once every pool's queue is drained (the bulk of the work has been handed out),
-    //    the items left in a pool are spread over its wavefronts
+    //    the items left in a pool are spread over its wavefronts; a slice of the row kernel does so before it
+    //    starts
     bool all_drained = true;
     for (const Progress& g : prog) all_drained &= g.next >= g.pl->total;
     for (const Progress& g : prog) {
@@ -568,7 +575,7 @@ int pool_step(hh_engine* e, PoolSet& set, double slice_ms, double* kernel_ms, do
         if (integrating && all_drained && e->use_graphs) {
             // the next slice's graph spreads them over the wavefronts
             pl->repack_pending = true;
-        } else if (integrating && all_drained) {
+        } else if (integrating && all_drained && items_left(*pl) > row_limit(e, set, *pl)) {
             HH_CHECK(run_repack(pl->sys, pl->view(pl->cur), pl->view(1 - pl->cur), pl->scratch.as<int>(), e->stream));
             pl->cur = 1 - pl->cur;
             launched = true;
