@@ -34,14 +34,7 @@
 // three-term recurrence in l at fixed m.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-#include <cstring>
-#include <map>
-#include <set>
-#include <utility>
-#include <vector>
-
-#include "ch4co2_dipole_tables.h"
+#include "ch4co2_dipole_layout.h"
 #include "hh_engine.h"
 #include "hh_systems.h"
 
@@ -52,121 +45,30 @@ namespace hh {
 // take 42.9, 28.6 and 36.3 ms with 4, 8 and 16; 200000 points in FP64 2.10, 1.31 and 1.04 ms.
 template <typename P>
 constexpr int kDipWaves = sizeof(P) == 4 ? 8 : 16;
-constexpr int kDipBlocks = 84; // (l_a, l_b) blocks
 constexpr int kDipMaxNB = 9;   // basis functions of the largest block
-constexpr int kDipQuads = 2304, kDipCoefs = 39936;   // quads of products and their coefficients (upper bounds)
 
 typedef unsigned int dip_u4 __attribute__((ext_vector_type(4)));
 
-// One block: its basis functions are rows [pos, pos + nb) of the radial table; the quads of component
-// c are [quad[c], quad[c + 1]), the coefficients of quad q the 4 nb values from coef0 + 4 nb (q -
-// quad[0]), function-major.
-struct DipBlock {
-    int nb, pos, coef0, pad;
-    int quad[4];
-};
-
 template <typename P>
 struct Ch4Co2DipTables {
+    using Real = P;
+    // (l_a, l_b) blocks; quads of products and their coefficients (2250 and 38112 of the present expansion)
+    static constexpr int kWaves = kDipWaves<P>, kBlocks = 84, kMaxNB = kDipMaxNB, kQuads = 2304, kCoefs = 39936;
     P radial[HH_CH4CO2_NINT + 1][HH_CH4CO2_NB][4];   // in block order; row NINT: the tail (c4, c5, c6, 0)
-    P coef[kDipCoefs];
-    dip_u4 xy[kDipQuads];        // x | y << 16 of a quad's products
-    DipBlock block[kDipBlocks];  // in wavefront order
-    int wave0[kDipWaves<P> + 1];    // wavefront w takes blocks [wave0[w], wave0[w + 1])
+    P coef[kCoefs];
+    dip_u4 xy[kQuads];        // x | y << 16 of a quad's products
+    DipBlock block[kBlocks];     // in wavefront order
+    int wave0[kWaves + 1];       // wavefront w takes blocks [wave0[w], wave0[w + 1])
     double bounds[HH_CH4CO2_NINT];
     double centre[HH_CH4CO2_NINT];
 };
 
-template <typename P>
-void fill_ch4co2_tables(Ch4Co2DipTables<P>& t)
-{
-    // l of an X index (l^2 ..) and of a Y index (even l: l (l - 1) / 2 ..)
-    auto la = [](int x) { int l = 0; while ((l + 1) * (l + 1) <= x) ++l; return l; };
-    auto lb = [](int y) { int l = 0; while ((l + 2) * (l + 1) / 2 <= y) l += 2; return l; };
-    struct Host {
-        std::vector<int> fn;                        // basis functions
-        std::vector<std::pair<int, int>> prod[3];   // products (x, y) of each component
-        long cost = 0;
-    };
-    std::map<std::pair<int, int>, Host> blocks;
-    for (int b = 0; b < HH_CH4CO2_NB; ++b)
-        if (HH_CH4CO2_START[b][3] > HH_CH4CO2_START[b][0]) {
-            const unsigned xy = HH_CH4CO2_XY[HH_CH4CO2_START[b][0]];
-            blocks[{la(xy & 0xff), lb(xy >> 8)}].fn.push_back(b);
-        }
-    std::vector<Host*> order;
-    for (auto& kv : blocks) {
-        Host& h = kv.second;
-        h.cost = 24 + 12 * (long)h.fn.size();
-        for (int c = 0; c < 3; ++c) {
-            std::set<std::pair<int, int>> used;
-            for (int b : h.fn)
-                for (int e = HH_CH4CO2_START[b][c]; e < HH_CH4CO2_START[b][c + 1]; ++e)
-                    used.insert({(int)(HH_CH4CO2_XY[e] & 0xff), (int)(HH_CH4CO2_XY[e] >> 8)});
-            h.prod[c].assign(used.begin(), used.end());
-            h.cost += (long)(h.prod[c].size() + 3) / 4 * (8 + 4 * (long)h.fn.size());
-        }
-        order.push_back(&h);
-    }
-    // blocks to wavefronts: the costliest first, each to the least loaded wavefront
-    std::stable_sort(order.begin(), order.end(), [](const Host* a, const Host* b) { return a->cost > b->cost; });
-    constexpr int waves = kDipWaves<P>;
-    std::vector<Host*> share[waves];
-    long load[waves] = {};
-    for (Host* h : order) {
-        const int w = (int)(std::min_element(load, load + waves) - load);
-        share[w].push_back(h);
-        load[w] += h->cost;
-    }
-    std::memset(&t, 0, sizeof t);
-    int nblk = 0, pos = 0, quad = 0, coef = 0;
-    for (int w = 0; w < waves; ++w) {
-        t.wave0[w] = nblk;
-        for (const Host* h : share[w]) {
-            const int nb = (int)h->fn.size();
-            DipBlock& bl = t.block[nblk++];
-            bl.nb = nb;
-            bl.pos = pos;
-            bl.coef0 = coef;
-            for (int j = 0; j < nb; ++j, ++pos) {
-                const int b = h->fn[j];
-                for (int k = 0; k < HH_CH4CO2_NINT; ++k)
-                    for (int i = 0; i < 4; ++i) t.radial[k][pos][i] = (P)HH_CH4CO2_RADIAL[k][b][i];
-                for (int i = 0; i < 3; ++i) t.radial[HH_CH4CO2_NINT][pos][i] = (P)HH_CH4CO2_TAIL[b][i];
-            }
-            for (int c = 0; c < 3; ++c) {
-                bl.quad[c] = quad;
-                for (size_t p0 = 0; p0 < h->prod[c].size(); p0 += 4, ++quad, coef += 4 * nb)
-                    for (int u = 0; u < 4; ++u) {
-                        if (p0 + u >= h->prod[c].size()) continue;   // padded: coefficients 0
-                        const std::pair<int, int> xy = h->prod[c][p0 + u];
-                        t.xy[quad][u] = (unsigned)xy.first | (unsigned)xy.second << 16;
-                        for (int j = 0; j < nb; ++j) {
-                            const int b = h->fn[j];
-                            for (int e = HH_CH4CO2_START[b][c]; e < HH_CH4CO2_START[b][c + 1]; ++e)
-                                if ((int)(HH_CH4CO2_XY[e] & 0xff) == xy.first && (int)(HH_CH4CO2_XY[e] >> 8) == xy.second)
-                                    t.coef[coef + 4 * j + u] += (P)HH_CH4CO2_COEF[e];
-                        }
-                    }
-            }
-            bl.quad[3] = quad;
-        }
-    }
-    t.wave0[waves] = nblk;
-    for (int k = 0; k < HH_CH4CO2_NINT; ++k) {
-        t.bounds[k] = HH_CH4CO2_BOUNDS[k];
-        t.centre[k] = HH_CH4CO2_CENTRE[k];
-    }
-}
-
 size_t ch4co2_table_bytes(bool f32) { return f32 ? sizeof(Ch4Co2DipTables<float>) : sizeof(Ch4Co2DipTables<double>); }
 
-void ch4co2_tables_host(bool f32, void* out)
+bool ch4co2_tables_host(bool f32, void* out)
 {
-    if (f32)
-        fill_ch4co2_tables(*static_cast<Ch4Co2DipTables<float>*>(out));
-    else
-        fill_ch4co2_tables(*static_cast<Ch4Co2DipTables<double>*>(out));
+    return f32 ? fill_ch4co2_tables(*static_cast<Ch4Co2DipTables<float>*>(out))
+               : fill_ch4co2_tables(*static_cast<Ch4Co2DipTables<double>*>(out));
 }
 
 // P_l^m {1, cos, sin} of direction v for l <= LMAX (only even l when EVEN) into column `lane` of

@@ -353,7 +353,10 @@ int hh_engine_create(int device, hh_engine** out)
         for (int f32 = 0; f32 < 2; ++f32) {
             const size_t nb = hh::ch4co2_table_bytes(f32);
             std::vector<char> host(nb);
-            hh::ch4co2_tables_host(f32, host.data());
+            if (!hh::ch4co2_tables_host(f32, host.data())) {
+                hh_engine_destroy(e);
+                return fail(HH_E_UNSUPPORTED, "the CH4-CO2 dipole expansion does not fit the dipole pass's tables");
+            }
             hh::DevBuf& d = f32 ? e->ch4tab32 : e->ch4tab64;
             if (d.ensure(nb) != hipSuccess || hipMemcpy(d.p, host.data(), nb, hipMemcpyHostToDevice) != hipSuccess) {
                 hh_engine_destroy(e);

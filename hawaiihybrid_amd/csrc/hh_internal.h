@@ -38,7 +38,8 @@ hipError_t run_eval(int sys, const SysConst& sc, int what, const double* y, long
 // CH4-CO2 dipole tables (hh_ch4co2.hip): bytes and host image in FP32 or FP64; the dipole pass of a
 // record-3 job (dipoles over its coordinate rows, then the CF rows jd.cf_rows with the sample checks)
 size_t ch4co2_table_bytes(bool f32);
-void ch4co2_tables_host(bool f32, void* out);
+// false: the expansion does not fit the table's bounds
+bool ch4co2_tables_host(bool f32, void* out);
 hipError_t run_ch4co2_cf_rows(const JobDesc& jd, const void* tables, bool f32, hipStream_t st);
 // CH4-CO2 lab dipoles at n phase points (SoA [16][n]) into out[3][n] (FP64 tables); records holds
 // 8 n doubles of scratch, len one int
