@@ -11,7 +11,8 @@ Beside a queue of more than three fills of the lane slots the orbiting items of 
 FP64 lane kernel: the same bits again.
 
 An engine with graph-captured slices stays on the lane kernel at every size; against it, exact special values
-of the initial conditions."""
+of the initial conditions, the dipole series (Zimmermann's and PR/mu's), trajectories that end at a failed
+sample or at the step limit."""
 import numpy as np
 import pytest
 
@@ -112,3 +113,80 @@ def test_orbiting_items_beside_a_deep_queue(eng, which):
     for key in ("len", "status", "nrhs", "e_drift", "rows"):
         assert np.array_equal(a[key], b[key]), key
     assert np.array_equal(alone[0].cpu().numpy(), beside[0].cpu().numpy())
+
+
+def check_same(a, b):
+    for key in ("len", "status", "nrhs", "e_drift", "rows"):
+        assert np.array_equal(a[key], b[key]), key
+
+
+@pytest.mark.parametrize("which,prec", [("hear", H.PREC_FP64), ("hear", H.PREC_MIXED), ("co2ar", H.PREC_FP64),
+                                        ("co2ar", H.PREC_MIXED)])
+def test_zimmermann_series(eng, lane_eng, which, prec):
+    """Both halves of bound pairs, three dipole components a sample."""
+    make, T, pesmin, rmin = SYSTEMS[which]
+    n, L = 70, 96
+    smp = H.Sampler(H.IC_REJECTION, H.PAIR_BOUND, 60.0, rmin, 40.0, pesmin, 0.0)
+    ic = H.sample_ics(make(), smp, 3, n)[0]
+    p = H.cf_params(L, rtol=1e-10 if prec == H.PREC_MIXED else 1e-12, halves=H.HALVES_BOTH, zimmermann=True, precision=prec)
+    got = []
+    for e in (eng, lane_eng):
+        cf, _ = e.cf_run(make(), p, [e.to_device_soa(ic)])
+        got.append((cf[0].cpu().numpy(), e.items(0, 2 * n, L, rows=True, zimmermann=True)))
+    check_same(got[0][1], got[1][1])
+    assert np.array_equal(got[0][0], got[1][0]) and np.any(got[0][0] != 0.0)
+
+
+@pytest.mark.parametrize("which", ["hear", "co2ar"])
+@pytest.mark.parametrize("prec", [H.PREC_FP64, H.PREC_MIXED])
+def test_prmu_series(eng, lane_eng, which, prec):
+    make, T, pesmin, rmin = SYSTEMS[which]
+    L, nfreq, R0 = 512, 200, 12.0
+    smp = H.Sampler(H.IC_R0_INJECT, H.PAIR_FREE, T, rmin, 40.0, pesmin, R0)
+    ic = H.sample_ics(make(), smp, 37, 65)[0]
+    p = H.PrmuParams(1e-10, 1e-10, 200.0, R0, L, nfreq, prec, 0, 0)
+    a, b = [e.prmu(make(), p, e.to_device_soa(ic)) for e in (eng, lane_eng)]
+    assert np.array_equal(a[0].cpu().numpy(), b[0].cpu().numpy()) and a[2] == b[2] > 0
+    assert np.array_equal(np.asarray(a[1]), np.asarray(b[1]))
+
+
+@pytest.mark.parametrize("prec", [H.PREC_FP64, H.PREC_MIXED])
+def test_failed_samples_and_step_limits(eng, lane_eng, prec):
+    """He-Ar pairs that come from 300 bohr and are sampled near their turning point next: the CF jumps by more than
+    1e10 (status 3).  A limit of 5 steps between samples (status 4)."""
+    n, L = 64, 8
+    s = H.he_ar()
+    v = 5.0e-4 * (1.0 + 0.004 * (np.arange(n) - n / 2))
+    ic = np.zeros((n, 6))
+    ic[:, 0], ic[:, 2], ic[:, 4], ic[:, 5] = 0.3, 1.1, 300.0, -s.mu * v
+    ic[:, 1], ic[:, 3] = 0.4, 0.3
+    jump = H.cf_params(L, rtol=1e-10, dt=146.0 / 5.0e-4, Rcut=400.0, precision=prec)
+    smp = H.Sampler(H.IC_R0_INJECT, H.PAIR_FREE, 300.0, 4.0, 40.0, H.PESMIN_HEAR, 15.0)
+    steps = H.cf_params(64, rtol=1e-12, dt=2000.0, Rcut=20.0, max_steps=5, precision=prec)
+    for p, y, status in ((jump, ic, 3), (steps, H.sample_ics(s, smp, 5, n)[0], 4)):
+        got = []
+        for e in (eng, lane_eng):
+            cf, _ = e.cf_run(s, p, [e.to_device_soa(y)])
+            got.append((cf[0].cpu().numpy(), e.items(0, n, p.L, rows=True)))
+        print(f"endings: status {np.bincount(got[0][1]['status'])}", flush=True)
+        assert np.any(got[0][1]["status"] == status)
+        check_same(got[0][1], got[1][1])
+        assert np.array_equal(got[0][0], got[1][0])
+
+
+@pytest.mark.parametrize("which", ["hear", "co2ar", "ch4co2"])
+@pytest.mark.parametrize("prec", [H.PREC_FP64, H.PREC_MIXED])
+@pytest.mark.parametrize("n", [1, 17, 700])
+def test_rows_equal_the_lane_kernel_alone(eng, lane_eng, which, prec, n):
+    """The same call on an engine that stays on the lane kernel: every compared item ran on it."""
+    make, T, pesmin, rmin = SYSTEMS[which]
+    L = 600
+    smp = H.Sampler(H.IC_R0_INJECT, H.PAIR_FREE, T, rmin, 40.0, pesmin, 15.0)
+    ic = H.sample_ics(make(), smp, 6, n)[0]
+    p = H.cf_params(L, rtol=1e-10 if prec == H.PREC_MIXED else 1e-12, Rcut=20.0, halves=H.HALVES_BOTH, precision=prec)
+    got = []
+    for e in (eng, lane_eng):
+        cf, _ = e.cf_run(make(), p, [e.to_device_soa(ic)])
+        got.append((cf[0].cpu().numpy(), e.items(0, 2 * n, L, rows=True)))
+    check_same(got[0][1], got[1][1])
+    assert np.array_equal(got[0][0], got[1][0])
