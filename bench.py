@@ -57,12 +57,14 @@ def rel(a, b):
     return float(np.linalg.norm(a - b) / np.linalg.norm(b))
 
 
-def traffic_from_counters(fetch_dir, write_dir, out_path, kernel="pool_cf_kernel<1, float, 256, 1>"):
-    """Bytes per launch of the mixed CO2-Ar pool kernel from two rocprofv3 counter runs of this
-    script with --calibrate-copy (one with --pmc FETCH_SIZE, one with --pmc WRITE_SIZE; CSV
-    output).  Each counter is scaled by what it reads for the 1 GiB device-to-device copy that
-    --calibrate-copy runs first (the largest __amd_rocclr_copyBuffer dispatch), then averaged
-    over the kernel's dispatches.  Writes the JSON that the roofline's `traffic` reads."""
+def traffic_from_counters(fetch_dir, write_dir, out_path,
+                          kernels=("pool_cf_kernel<1, float, 256, 1>", "row_cf_kernel<1, float, 2>")):
+    """Bytes per step of the mixed CO2-Ar pool's slices, which run on the lane or on the row kernel, from two
+    rocprofv3 counter runs of this script with --calibrate-copy (one with --pmc FETCH_SIZE, one with
+    --pmc WRITE_SIZE; CSV output).  Per step, since the length and the number of the slices follow the
+    queue: the roofline divides by the launches of its own run.  Each counter is scaled by what it reads for the 1 GiB device-to-device copy that
+    --calibrate-copy runs first (the largest __amd_rocclr_copyBuffer dispatch), then summed
+    over the kernels' dispatches.  Writes the JSON that the roofline's `traffic` reads."""
     import csv
     import glob
 
@@ -77,24 +79,24 @@ def traffic_from_counters(fetch_dir, write_dir, out_path, kernel="pool_cf_kernel
         return vals
 
     args = "--steps 20 --warmup 5 --no-serve --no-n2ar --no-ch4co2 --no-oracle --no-hbm --deep 0 --calibrate-copy"
-    res = {"kernel": kernel,
+    res = {"kernel": " and ".join(kernels),
            "workload": "CO2-Ar, 65536 trajectories per step, T=200 K, L=4096, batched mixed engine rtol=1e-10; "
-                       "every dispatch of the kernel in the run (5 warm-up and 20 timed steps)",
+                       "every dispatch of the kernels in the run (5 warm-up and 20 timed steps)",
            "commands": [f"rocprofv3 --pmc FETCH_SIZE --output-format csv -d {fetch_dir} -o fetch -- python3 bench.py {args}",
                         f"rocprofv3 --pmc WRITE_SIZE --output-format csv -d {write_dir} -o write -- python3 bench.py {args}",
                         f"python3 bench.py --traffic-from {fetch_dir} {write_dir}"],
-           "counters": {}}
+           "steps": 25, "counters": {}}
     for name, d in (("fetch", fetch_dir), ("write", write_dir)):
         counter = "FETCH_SIZE" if name == "fetch" else "WRITE_SIZE"
         v = per_dispatch(d, counter)
         copy = max((x for (k, _), x in v.items() if "copyBuffer" in k), default=0.0)
         scale = (1 << 30) / 1024.0 / copy if copy > 0 else None
-        ks = [x for (k, _), x in v.items() if kernel in k]
-        res["counters"][name] = {"counter": counter, "copy_kib": copy, "scale": scale, "dispatches": len(ks),
-                                 "kib_per_dispatch": float(np.mean(ks)) if ks else None}
+        per = {kernel: [x for (k, _), x in v.items() if kernel in k] for kernel in kernels}
+        res["counters"][name] = {"counter": counter, "copy_kib": copy, "scale": scale, "kib": sum(map(sum, per.values())),
+                                 "per_kernel": {k: {"dispatches": len(x), "kib": sum(x)} for k, x in per.items()}}
     f, w = res["counters"]["fetch"], res["counters"]["write"]
-    if f["kib_per_dispatch"] is not None and w["kib_per_dispatch"] is not None and f["scale"] and w["scale"]:
-        res["hbm_bytes_per_launch"] = 1024.0 * (f["kib_per_dispatch"] * f["scale"] + w["kib_per_dispatch"] * w["scale"])
+    if f["kib"] and w["kib"] and f["scale"] and w["scale"]:
+        res["hbm_bytes_per_step"] = 1024.0 * (f["kib"] * f["scale"] + w["kib"] * w["scale"]) / res["steps"]
     json.dump(res, open(out_path, "w"), indent=1)
     return res
 
@@ -528,13 +530,15 @@ def main():
     peak = (f32 + f64) / t_at_peak / 1e12
     traffic, traffic_src = None, None
     tpath = os.path.join(HERE, "profiles", "pool_cf_kernel_co2ar_mixed_traffic.json")
-    if os.path.exists(tpath):
-        traffic = json.load(open(tpath)).get("hbm_bytes_per_launch")
+    per_step = json.load(open(tpath)).get("hbm_bytes_per_step") if os.path.exists(tpath) else None
+    if per_step and (n, L) == (65536, 4096):
+        traffic = per_step * K / nlaunch
         traffic_src = ("profiles/pool_cf_kernel_co2ar_mixed_traffic.json (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE "
-                       "of this workload, scaled by a 1 GiB copy; bench.py --traffic-from)")
+                       "of this workload per step, scaled by a 1 GiB copy; bench.py --traffic-from), over the launches")
     roofline = {"bound": "valu", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
                 "frac": achieved / peak, "traffic": traffic, "traffic_source": traffic_src,
-                "kernel": "pool_cf_kernel<CO2-Ar, float, 256 lanes, 1 wavefront/SIMD> (the mixed-precision pool)",
+                "kernel": "the mixed-precision pool's slices: pool_cf_kernel<CO2-Ar, float, 256 lanes, 1 wavefront/SIMD>, "
+                          "for the last few thousand items row_cf_kernel<CO2-Ar, float>",
                 "pipe": "vector ALU, FP32 and FP64 (no matrix work)",
                 "achieved_fp32_tflops": f32 / secs / 1e12, "peak_fp32_tflops": MI355X_FP32_VECTOR_TFLOPS,
                 "achieved_fp64_tflops": f64 / secs / 1e12, "peak_fp64_tflops": MI355X_FP64_VECTOR_TFLOPS,
