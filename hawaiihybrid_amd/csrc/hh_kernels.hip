@@ -1183,7 +1183,7 @@ __global__ void __launch_bounds__(256) cf_reduce_final_kernel(int L, int nchunks
 // wr[t * ntemp + st] (Boltzmann reweight times the temperature's partition-function ratio);
 // blockIdx.z is a group of NT temperatures, so the rows are read once a group and, kReduceUnroll items
 // in flight, bound by their latency (20000 trajectories of both halves, L = 1024, eight temperatures:
-// a temperature per workgroup, an item at a time, 420 us; this 262).
+// a temperature per workgroup, an item at a time, 420 to 530 us; this 239).
 // Partial sums psum[(st * nchunks + c) * L + k].
 template <int HALVES, int NT>
 __global__ void __launch_bounds__(256) cf_reduce_weighted_partial_kernel(JobDesc jb, long long chunk, int ntemp,
@@ -1400,10 +1400,10 @@ LaneSlots slots_view(int sys, void* base, long long S)
 hipError_t run_reduce_weighted(const JobDesc& jb, int ntemp, const double* wr, const double* nstar, double* psum,
                                double* pcomp, long long chunk, int nchunks, double* cf_out, hipStream_t st)
 {
-    // groups of eight temperatures, of four where there are no more
-    const int nt = ntemp > 4 ? 8 : 4;
-    auto k = jb.halves == 2 ? (nt == 8 ? cf_reduce_weighted_partial_kernel<2, 8> : cf_reduce_weighted_partial_kernel<2, 4>)
-                            : (nt == 8 ? cf_reduce_weighted_partial_kernel<1, 8> : cf_reduce_weighted_partial_kernel<1, 4>);
+    // Groups of four temperatures: 164, 187, 239 and 319 us for 1, 4, 8 and 16 (20000 trajectories of both halves,
+    // L = 1024); of eight 218, 242, 266 and 321, of two 134, 181 and 266 (1, 4, 8), of one 115, 219 and 440.
+    constexpr int nt = 4;
+    auto k = jb.halves == 2 ? cf_reduce_weighted_partial_kernel<2, nt> : cf_reduce_weighted_partial_kernel<1, nt>;
     hipLaunchKernelGGL(k, dim3((jb.L + 255) / 256, nchunks, (ntemp + nt - 1) / nt), dim3(256), 0, st, jb, chunk, ntemp,
                        wr, psum, pcomp);
     hipError_t e = hipGetLastError();

@@ -8,8 +8,9 @@
 // registers of every lane, a tableau row is one FMA per non-zero column for all components at
 // once, and the independent parts of a right-hand side run side by side in the row's lanes (the
 // angles' sines and cosines, the reciprocals, the radial slots of CO2-Ar, the site pairs of
-// CH4-CO2), exchanged with DPP row broadcasts.  What is serial (the Legendre recurrence, Hamilton's
-// equations, the sums in their order) runs in every lane of the row.
+// CH4-CO2), exchanged with DPP row broadcasts; for He-Ar and CO2-Ar every lane forms its own component of
+// Hamilton's equations.  What is serial (the FP64 Legendre recurrence, the sums in their order, all of
+// CH4-CO2's equations) runs in every lane of the row.
 //
 // Every expression is the lane kernel's, in its order, so a trajectory's row is the same bits
 // whichever kernel integrates it, and the two share the slot format: a slice of a pool can run on
