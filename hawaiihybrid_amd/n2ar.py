@@ -118,7 +118,7 @@ class PipNN:
 
     precision MLP_BF16X3 (the default) splits every operand into a BF16 head and tail and takes
     three matrix-core products: within 0.25 cm^-1 of the FP64 networks, the mode for dynamics.
-    MLP_BF16 takes one product: 1.6x the throughput, median error 2e-3 cm^-1 but outliers of
+    MLP_BF16 takes one product: 1.5x the throughput, median error 2e-3 cm^-1 but outliers of
     ~100 cm^-1 on the repulsive wall and ~10% of the largest dipole, so it is a throughput mode,
     not a parity-grade surface."""
 
